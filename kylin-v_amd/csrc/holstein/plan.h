@@ -199,6 +199,67 @@ inline ProductPlan plan_product(const Layout& A, const Layout& B, int nc, char o
     return P;
 }
 
+// A product plan's K ranges cut into nch chunks per group: chunk c's groups write the partial
+// result of the c-th part of their K range at c * out.total, to be summed in chunk order.
+struct SplitK {
+    int nch = 1;
+    std::vector<GemmGroup> groups;
+    std::vector<GemmSeg> segs;
+    std::vector<GemmTile> tiles;  // config 0
+};
+
+// K chunks of a plan.  An output of few tiles leaves most of the 256 CUs idle while each
+// workgroup walks its whole K range alone, 1.1 us per 8-deep stage (an environment update's
+// last product at D = 128, 16 levels: 6 tiles, K = 2048, 286 us whole, 17 + 4 us cut in 32).  Chunks
+// double while the workgroups stay under kSplitWgs and the deepest group keeps kSplitDepth per chunk.
+constexpr int kSplitWgs = 512, kSplitDepth = 64, kSplitMax = 32;
+inline int split_chunks(const ProductPlan& P) {
+    int64_t kmax = 0;
+    for (const auto& g : P.groups) {
+        int64_t k = 0;
+        for (int s = 0; s < g.seg_count; ++s) k += P.segs[g.seg_begin + s].k;
+        kmax = std::max(kmax, k);
+    }
+    int n = 1;
+    while (2 * n <= kSplitMax && (int64_t)P.tiles.size() * 2 * n <= kSplitWgs && kmax / (2 * n) >= kSplitDepth) n *= 2;
+    return n;
+}
+
+inline SplitK split_k(const ProductPlan& P, int nch) {
+    SplitK S;
+    S.nch = nch;
+    for (int c = 0; c < nch; ++c)
+        for (const auto& g : P.groups) {
+            int64_t K = 0;
+            for (int s = 0; s < g.seg_count; ++s) K += P.segs[g.seg_begin + s].k;
+            // chunk boundaries at multiples of 8, so that no stage of the kernel is cut short
+            // where the segments allow it
+            const int64_t per = ((K + nch - 1) / nch + 7) / 8 * 8;
+            const int64_t lo = std::min(K, c * per), hi = std::min(K, lo + per);
+            GemmGroup h = g;
+            h.c_off = g.c_off + (int64_t)c * P.out.total;
+            h.seg_begin = (int)S.segs.size();
+            int64_t at = 0;
+            for (int s = 0; s < g.seg_count; ++s) {
+                const GemmSeg& sg = P.segs[g.seg_begin + s];
+                const int64_t a = std::max(lo, at), b = std::min(hi, at + sg.k);
+                if (a < b) {
+                    const int64_t k0 = a - at;
+                    GemmSeg t = sg;
+                    t.a_off += P.opA == 0 ? k0 : k0 * sg.lda;
+                    t.b_off += P.opB == 0 ? k0 * sg.ldb : k0;
+                    t.k = (int)(b - a);
+                    S.segs.push_back(t);
+                }
+                at += sg.k;
+            }
+            h.seg_count = (int)S.segs.size() - h.seg_begin;
+            S.groups.push_back(h);
+        }
+    S.tiles = cut_tiles(S.groups, 0);
+    return S;
+}
+
 struct WFoldPlan {
     Layout out;
     std::vector<WTask> tasks;

@@ -104,11 +104,21 @@ struct DevProduct {
     const GemmTile* tp[kNumGemmConfigs] = {nullptr};
     int ntiles[kNumGemmConfigs] = {0};
     bool cut[kNumGemmConfigs] = {false};
+    int nch = 1;   // K chunks (split_chunks): above 1 the lists are split_k's
+    DevBuf part;   // and the chunks' partial results go here, one after the other
     void build(Device& dev, ProductPlan plan) {
         p = std::move(plan);
-        lists = upload_packed(dev, p.groups, p.segs, p.tiles);
+        nch = split_chunks(p);
+        if (nch > 1) {
+            const SplitK sk = split_k(p, nch);
+            part = DevBuf(dev.pool.get(), (size_t)nch * p.out.total * sizeof(double2));
+            lists = upload_packed(dev, sk.groups, sk.segs, sk.tiles);
+            ntiles[0] = (int)sk.tiles.size();
+        } else {
+            lists = upload_packed(dev, p.groups, p.segs, p.tiles);
+            ntiles[0] = (int)p.tiles.size();
+        }
         tp[0] = lists.at<GemmTile>(2);
-        ntiles[0] = (int)p.tiles.size();
         cut[0] = true;
     }
     void ensure_tiles(Device& dev, int cfg) {
@@ -122,14 +132,15 @@ struct DevProduct {
     template <class T2>
     void launch(Device& dev, int cfg, const T2* A, const T2* B, T2* C, double ar, double ai) {
         ensure_tiles(dev, cfg);
-        launch_gemm<T2>(dev.stream, p.opA, p.opB, A, B, C, tp[cfg], ntiles[cfg], lists.at<GemmGroup>(0),
-                        lists.at<GemmSeg>(1), ar, ai, cfg);
+        launch_gemm<T2>(dev.stream, p.opA, p.opB, A, B, nch > 1 ? part.as<T2>() : C, tp[cfg], ntiles[cfg],
+                        lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg);
+        if (nch > 1) launch_sum_parts<T2>(dev.stream, part.as<T2>(), nch, p.out.total, C);
     }
     // Tile config for this plan: cached per shape class; on a first encounter every config
     // built for the op pair runs twice on the real operands and the fastest is kept.
     template <class T2>
     int choose(Device& dev, const T2* A, const T2* B, T2* C, double ar, double ai) {
-        if (!dev.autotune || p.flop < 1e8) return 0;
+        if (!dev.autotune || p.flop < 1e8 || nch > 1) return 0;
         const uint64_t key = gemm_shape_key(p, sizeof(T2) == sizeof(double2) ? 0 : 1);
         auto it = dev.gemm_tuned.find(key);
         if (it != dev.gemm_tuned.end()) return it->second;
@@ -165,11 +176,13 @@ struct DevProduct {
     void launch_split(Device& dev, int cfg, const float2* A, const float2* B, float2* C, double ar,
                       double ai) {
         ensure_tiles(dev, cfg);
-        launch_gemm_bf16x3(dev.stream, p.opA, p.opB, A, B, C, tp[cfg], ntiles[cfg], lists.at<GemmGroup>(0),
-                           lists.at<GemmSeg>(1), ar, ai, cfg);
+        launch_gemm_bf16x3(dev.stream, p.opA, p.opB, A, B, nch > 1 ? part.as<float2>() : C, tp[cfg], ntiles[cfg],
+                           lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg);
+        if (nch > 1) launch_sum_parts<float2>(dev.stream, part.as<float2>(), nch, p.out.total, C);
     }
     // Split-BF16 tile (64x64 or 128x128), timed once per shape class like choose().
     int choose_split(Device& dev, const float2* A, const float2* B, float2* C, double ar, double ai) {
+        if (nch > 1) return 0;
         if (const char* t = std::getenv("KV_SPLIT_TILE")) return std::atoi(t) == 128 ? 4 : 0;
         if (!dev.autotune || p.flop < 1e8) return 0;
         const uint64_t key = gemm_shape_key(p, 2);

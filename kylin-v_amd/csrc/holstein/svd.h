@@ -40,6 +40,7 @@
 #include <string>
 #include <vector>
 
+#include "plan.h"
 #include "svd_rule.h"
 #include "tensor.h"
 
@@ -152,9 +153,12 @@ struct SvdOptions {
 
 // C (m x n, ld ldc) = op(A) op(B) for one dense complex problem on the grouped GEMM.
 // upper_only: only the 64 x 64 tiles on or above the diagonal (Hermitian products whose
-// consumer reads one triangle); the rest of C is left as it was.
+// consumer reads one triangle); the rest of C is left as it was, or zero.
 inline void gemm_dense(Device& D, char opA, char opB, const double2* A, int lda, const double2* B,
                        int ldb, double2* C, int ldc, int m, int n, int k, bool upper_only = false) {
+    ProductPlan P;
+    P.opA = op_code(opA);
+    P.opB = op_code(opB);
     GemmGroup g{};
     g.m = m;
     g.n = n;
@@ -165,15 +169,32 @@ inline void gemm_dense(Device& D, char opA, char opB, const double2* A, int lda,
     sg.k = k;
     sg.lda = lda;
     sg.ldb = ldb;
-    std::vector<GemmGroup> gs{g};
-    std::vector<GemmSeg> ss{sg};
-    std::vector<GemmTile> ts;
-    for (int a = 0; a < (m + GEMM_BM - 1) / GEMM_BM; ++a)
-        for (int b = 0; b < (n + GEMM_BN - 1) / GEMM_BN; ++b)
-            if (!upper_only || a * GEMM_BM < (b + 1) * GEMM_BN) ts.push_back(GemmTile{0, a, b, 0});
-    PackedUpload pk = upload_packed(D, gs, ss, ts);
-    launch_gemm<double2>(D.stream, op_code(opA), op_code(opB), A, B, C, pk.at<GemmTile>(2),
-                         (int)ts.size(), pk.at<GemmGroup>(0), pk.at<GemmSeg>(1), 1.0, 0.0);
+    P.groups.push_back(g);
+    P.segs.push_back(sg);
+    auto cut = [&](const std::vector<GemmGroup>& gs) {
+        std::vector<GemmTile> ts;
+        for (const GemmTile& t : cut_tiles(gs, 0))
+            if (!upper_only || t.tm * GEMM_BM < (t.tn + 1) * GEMM_BN) ts.push_back(t);
+        return ts;
+    };
+    P.tiles = cut(P.groups);
+    P.out.total = (int64_t)m * n;
+    // few tiles and a deep K: partial products summed in chunk order, as in DevProduct
+    const int nch = ldc == n ? split_chunks(P) : 1;
+    if (nch > 1) {
+        const SplitK sk = split_k(P, nch);
+        const std::vector<GemmTile> ts = cut(sk.groups);
+        PackedUpload pk = upload_packed(D, sk.groups, sk.segs, ts);
+        DevBuf part(D.pool.get(), (size_t)nch * P.out.total * sizeof(double2));
+        if (upper_only) launch_zero(D.stream, part.get(), part.bytes());  // the tiles left out
+        launch_gemm<double2>(D.stream, P.opA, P.opB, A, B, part.as<double2>(), pk.at<GemmTile>(2), (int)ts.size(),
+                             pk.at<GemmGroup>(0), pk.at<GemmSeg>(1), 1.0, 0.0);
+        launch_sum_parts<double2>(D.stream, part.as<double2>(), nch, P.out.total, C);
+        return;
+    }
+    PackedUpload pk = upload_packed(D, P.groups, P.segs, P.tiles);
+    launch_gemm<double2>(D.stream, P.opA, P.opB, A, B, C, pk.at<GemmTile>(2), (int)P.tiles.size(),
+                         pk.at<GemmGroup>(0), pk.at<GemmSeg>(1), 1.0, 0.0);
 }
 
 struct SectorSvd {
@@ -680,7 +701,7 @@ inline void gram_eigvecs(Device& D, Solver& sol, SectorSvd& X, int lo, hipStream
         launch_zero(st, Sp.get(), Sp.bytes());  // blocks with fewer chunks leave parts unset
         launch_gemm<double2>(st, 0, 2, V.as<double2>(), V.as<double2>(), Sp.as<double2>(), tiles,
                              s_tiles, pk.at<GemmGroup>(0), pk.at<GemmSeg>(1), 1.0, 0.0);
-        launch_sum_parts(st, Sp.as<double2>(), nch_max, (int64_t)nblk * sbw, S.as<double2>());
+        launch_sum_parts<double2>(st, Sp.as<double2>(), nch_max, (int64_t)nblk * sbw, S.as<double2>());
         launch_hh_tfactor(st, S.as<double2>(), X.tau.as<double2>(), T.as<double2>(), nblk, bw, nref);
         auto* v = reinterpret_cast<rocblas_double_complex*>(V.get());
         auto* p = reinterpret_cast<rocblas_double_complex*>(P.get());
@@ -703,7 +724,7 @@ inline void gram_eigvecs(Device& D, Solver& sol, SectorSvd& X, int lo, hipStream
             launch_gemm<double2>(st, 0, 2, Z.as<double2>(), V.as<double2>(), Yp.as<double2>(),
                                  tiles + y_off[b], y_cnt[b], pk.at<GemmGroup>(0), pk.at<GemmSeg>(1), 1.0,
                                  0.0);
-            launch_sum_parts(st, Yp.as<double2>(), nch[b], (int64_t)bw * k, Y.as<double2>());
+            launch_sum_parts<double2>(st, Yp.as<double2>(), nch[b], (int64_t)bw * k, Y.as<double2>());
             ok(rocblas_zgemm(h, rocblas_operation_none, rocblas_operation_none, mb, k, bw, &mone,
                              p + (size_t)b * sv + r0, n, y, bw, &one, z + r0, n));
         }
@@ -1012,7 +1033,7 @@ inline void gemm_jobs(Device& D, char opA, char opB, const std::vector<GemmJob>&
                          pk.at<GemmGroup>(0), pk.at<GemmSeg>(1), 1.0, 0.0, cfg);
     if (nch > 1)
         for (size_t q = 0; q < jobs.size(); ++q)
-            launch_sum_parts(D.stream, part.as<double2>() + poff[q], nch, (int64_t)jobs[q].m * jobs[q].n,
+            launch_sum_parts<double2>(D.stream, part.as<double2>() + poff[q], nch, (int64_t)jobs[q].m * jobs[q].n,
                              jobs[q].C);
     D.spans.close(t0, D.stream, &D.blk.gemm_ms);
     D.blk.gemm_flop += flop;

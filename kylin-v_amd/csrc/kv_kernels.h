@@ -85,7 +85,8 @@ void launch_hh_explicit(hipStream_t st, const double2* A, double2* V, int n, int
 void launch_hh_tfactor(hipStream_t st, const double2* S, const double2* tau, double2* T, int nblocks,
                        int bw, int nref);
 // out[e] = sum_{p < np} part[p n + e]: partial products of a split-K GEMM summed.
-void launch_sum_parts(hipStream_t st, const double2* part, int np, int64_t n, double2* out);
+template <class T2>
+void launch_sum_parts(hipStream_t st, const T2* part, int np, int64_t n, T2* out);
 // Z[j n + i] = C[(c0 + j) ldc + i]  (i < n, j < k): real columns to complex.
 void launch_real_cols(hipStream_t st, const double* C, int ldc, int c0, int k, int n, double2* Z);
 

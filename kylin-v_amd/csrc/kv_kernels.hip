@@ -1362,24 +1362,34 @@ void launch_hh_tfactor(hipStream_t st, const double2* S, const double2* tau, dou
 }
 
 // out[e] = sum_{p < np} part[p * n + e]  (split-K partial products summed).
-__global__ __launch_bounds__(256) void sum_parts_kernel(const double2* __restrict__ part, int np,
-                                                        int64_t n, double2* __restrict__ out) {
+// Bound by the partials' read (np x n elements from L2 / HBM); eight loads in flight per lane.
+template <class T2>
+__global__ __launch_bounds__(256) void sum_parts_kernel(const T2* __restrict__ part, int np,
+                                                        int64_t n, T2* __restrict__ out) {
+    using T = typename ScalarOf<T2>::T;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-        double re = 0, im = 0;
+        T re = 0, im = 0;
+#pragma unroll 8
         for (int p = 0; p < np; ++p) {
-            const double2 v = part[(int64_t)p * n + e];
+            const T2 v = part[(int64_t)p * n + e];
             re += v.x;
             im += v.y;
         }
-        out[e] = make_double2(re, im);
+        T2 o;
+        o.x = re;
+        o.y = im;
+        out[e] = o;
     }
 }
 
-void launch_sum_parts(hipStream_t st, const double2* part, int np, int64_t n, double2* out) {
+template <class T2>
+void launch_sum_parts(hipStream_t st, const T2* part, int np, int64_t n, T2* out) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(sum_parts_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, part, np, n, out);
+    hipLaunchKernelGGL(sum_parts_kernel<T2>, dim3(ew_blocks(n)), dim3(256), 0, st, part, np, n, out);
     KV_HIP(hipGetLastError());
 }
+template void launch_sum_parts<double2>(hipStream_t, const double2*, int, int64_t, double2*);
+template void launch_sum_parts<float2>(hipStream_t, const float2*, int, int64_t, float2*);
 
 // Z[j n + i] = C[(c0 + j) ldc + i] for i < n, j < k (real columns to complex).
 __global__ __launch_bounds__(256) void real_cols_kernel(const double* __restrict__ C, int ldc, int c0,
