@@ -45,72 +45,65 @@ inline KrylovExit local_krylov(const std::shared_ptr<Device>& dev, int nsite, co
     const int64_t n = xl.total;
     const int nv_max = std::max(max_iter, 2);
     Device& D = *dev;
-    std::unique_ptr<Tensor> xin = relayout(dev, *x, xl);
+    std::unique_ptr<Tensor> spread;
+    const Tensor* xin = x.get();
+    if (!same_layout(x->lay, xl)) {
+        spread = relayout(dev, *x, xl);
+        xin = spread.get();
+    }
     DevBuf V(D.pool.get(), (size_t)nv_max * (size_t)n * sizeof(double2));
     DevBuf hv(D.pool.get(), (size_t)n * sizeof(double2));
-    // device scalars: [0..1] beta, [2..3] alpha, [4] |h|^2, [5] |x|^2 ; reduction scratch
-    DevBuf sc(D.pool.get(), 8 * sizeof(double));
-    DevBuf scratch(D.pool.get(), 2 * 1024 * sizeof(double));
-    double* s = sc.as<double>();
+    DevBuf part(D.pool.get(), kLanczosPart * sizeof(double));
     double2* Vb = V.as<double2>();
-    launch_nrm2sq(D.stream, xin->d(), n, s + 5, scratch.as<double>());
-    launch_scale_invsqrt_dev(D.stream, Vb, xin->d(), s + 5, n);
+    double2* h = hv.as<double2>();
+    LanczosHost* rec = D.lanczos_host;
+    const uint64_t tag = ++D.lanczos_calls << 8;
+    launch_lanczos_begin(D.stream, xin->d(), Vb, n, part.as<double>(), D.lanczos_dev);
 
-    std::vector<std::complex<double>> alp, bet_up;
-    int k = 0;
-    double err = 1.0;
-    KrylovExit ex;
-    bool conv = false;
-    double host[6];
-    while (k < max_iter - 1 && err > tol) {
-        double2* vk = Vb + (int64_t)k * n;
+    // The recurrence and its stopping rule run on the device; the host queues iteration k + 1
+    // before it reads the scalars of iteration k, and the launches of an iteration past the
+    // last one return at once.
+    auto queue = [&](int k) {
         // Mixed precision: the first matvec runs in FP64.  Its rounding error enters the
         // result at first order in dt/2 |H v|; the errors of later Krylov vectors are
         // damped by further powers of the Lanczos coefficients, so FP32 suffices there.
-        H.apply(vk, hv.as<double2>(), dt * 0.5, log, k == 0);
-        if (stats) {
-            stats->heff_flop += H.flop();
-            stats->matvecs += 1;
+        double2* vk = Vb + (int64_t)k * n;
+        H.apply(vk, h, dt * 0.5, log, k == 0, &D.lanczos_dev->stop[k]);
+        launch_lanczos_step(D.stream, h, vk - n, vk, vk + n, n, part.as<double>(), D.lanczos_dev, k, tol, rec + k,
+                            tag | (uint64_t)k);
+    };
+    std::vector<std::complex<double>> alp, bet_up;
+    double err = 1.0;
+    KrylovExit ex;
+    const int last = max_iter - 2;  // the last iteration the cap allows
+    if (last >= 0 && err > tol) {
+        queue(0);
+        for (int k = 0;; ++k) {
+            const size_t logged = log ? log->pending.size() : 0;
+            if (k < last) queue(k + 1);
+            D.wait_record(rec[k], tag | (uint64_t)k);
+            if (stats) {
+                stats->heff_flop += H.flop();
+                stats->matvecs += 1;
+            }
+            if (k > 0) bet_up.emplace_back(rec[k].beta_re, rec[k].beta_im);
+            alp.emplace_back(rec[k].alpha_re, rec[k].alpha_im);
+            err = rec[k].err;
+            const bool stopped = !(err > tol);
+            if (stopped && log) log->drop(logged);
+            if (stopped || k == last) break;
         }
-        // beta = <h|v_{k-1}>, h -= beta v_{k-1}, alpha = <h|v_k>, h -= alpha v_k, |h|^2: the
-        // reference's order, each subtraction fused with the reduction after it
-        double2* h = hv.as<double2>();
-        double2* sb = reinterpret_cast<double2*>(s);
-        if (k > 0) {
-            double2* vkm = Vb + (int64_t)(k - 1) * n;
-            launch_dotc(D.stream, h, vkm, n, sb, scratch.as<double>());
-            launch_axpy_dotc(D.stream, h, vkm, sb, vk, n, sb + 1, scratch.as<double>());
-        } else {
-            launch_dotc(D.stream, h, vk, n, sb + 1, scratch.as<double>());
-        }
-        launch_axpy_nrm2sq(D.stream, h, vk, sb + 1, n, s + 4, scratch.as<double>());
-        KV_HIP(hipMemcpyAsync(host, s, 5 * sizeof(double), hipMemcpyDeviceToHost, D.stream));
-        D.sync();
-        if (log) log->resolve(kstats ? *kstats : D.stats);
-        if (k > 0) bet_up.emplace_back(host[0], host[1]);
-        alp.emplace_back(host[2], host[3]);
-        const double nm = std::sqrt(host[4]);
-        err *= nm;
-        if (err < tol) {
-            conv = true;
-            break;
-        }
-        launch_scale_invsqrt_dev(D.stream, Vb + (int64_t)(k + 1) * n, hv.as<double2>(), s + 4, n);
-        ++k;
     }
-    ex.converged = conv;
+    ex.converged = err < tol;
     ex.iterations = (int)alp.size();
     ex.error = err;
     std::vector<std::complex<double>> c = krylov_coefficients(alp, bet_up, reverse);
-    DevBuf cd(D.pool.get(), c.size() * sizeof(double2));
-    KV_HIP(hipMemcpyAsync(cd.get(), c.data(), c.size() * sizeof(double2), hipMemcpyHostToDevice,
-                          D.stream));
     auto out = Tensor::create(dev, xl, false);
-    launch_lincomb(D.stream, out->d(), Vb, cd.as<double2>(), (int)c.size(), n);
-    launch_nrm2sq(D.stream, out->d(), n, s + 5, scratch.as<double>());
-    KV_HIP(hipMemcpyAsync(host + 5, s + 5, sizeof(double), hipMemcpyDeviceToHost, D.stream));
+    launch_lanczos_end(D.stream, out->d(), Vb, reinterpret_cast<const double2*>(c.data()), (int)c.size(), n,
+                       part.as<double>(), rec + kLanczosMax, tag | 0xff);
     D.sync();
-    ex.loss_norm = 1.0 - std::sqrt(host[5]);
+    if (log) log->resolve(kstats ? *kstats : D.stats);
+    ex.loss_norm = 1.0 - std::sqrt(rec[kLanczosMax].nsq);
     x = std::move(out);
     return ex;
 }

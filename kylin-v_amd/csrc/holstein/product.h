@@ -63,6 +63,14 @@ struct EventLog {
         }
         pending.clear();
     }
+    // forgets the records from the n-th on (launches that found their iteration stopped)
+    void drop(size_t n) {
+        while (pending.size() > n) {
+            spare.push_back(pending.back().a);
+            spare.push_back(pending.back().b);
+            pending.pop_back();
+        }
+    }
     ~EventLog() {
         for (auto& r : pending) {
             (void)hipEventDestroy(r.a);
@@ -130,11 +138,12 @@ struct DevProduct {
         cut[cfg] = true;
     }
     template <class T2>
-    void launch(Device& dev, int cfg, const T2* A, const T2* B, T2* C, double ar, double ai) {
+    void launch(Device& dev, int cfg, const T2* A, const T2* B, T2* C, double ar, double ai,
+                const int* stop = nullptr) {
         ensure_tiles(dev, cfg);
         launch_gemm<T2>(dev.stream, p.opA, p.opB, A, B, nch > 1 ? part.as<T2>() : C, tp[cfg], ntiles[cfg],
-                        lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg);
-        if (nch > 1) launch_sum_parts<T2>(dev.stream, part.as<T2>(), nch, p.out.total, C);
+                        lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg, stop);
+        if (nch > 1) launch_sum_parts<T2>(dev.stream, part.as<T2>(), nch, p.out.total, C, stop);
     }
     // Tile config for this plan: cached per shape class; on a first encounter every config
     // built for the op pair runs twice on the real operands and the fastest is kept.
@@ -174,11 +183,11 @@ struct DevProduct {
         return best;
     }
     void launch_split(Device& dev, int cfg, const float2* A, const float2* B, float2* C, double ar,
-                      double ai) {
+                      double ai, const int* stop = nullptr) {
         ensure_tiles(dev, cfg);
         launch_gemm_bf16x3(dev.stream, p.opA, p.opB, A, B, nch > 1 ? part.as<float2>() : C, tp[cfg], ntiles[cfg],
-                           lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg);
-        if (nch > 1) launch_sum_parts<float2>(dev.stream, part.as<float2>(), nch, p.out.total, C);
+                           lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg, stop);
+        if (nch > 1) launch_sum_parts<float2>(dev.stream, part.as<float2>(), nch, p.out.total, C, stop);
     }
     // Split-BF16 tile (64x64 or 128x128), timed once per shape class like choose().
     int choose_split(Device& dev, const float2* A, const float2* B, float2* C, double ar, double ai) {
@@ -207,7 +216,7 @@ struct DevProduct {
     }
     template <class T2>
     void run(Device& dev, const T2* A, const T2* B, T2* C, double alpha_re = 1.0,
-             double alpha_im = 0.0, EventLog* log = nullptr, bool split = false) {
+             double alpha_im = 0.0, EventLog* log = nullptr, bool split = false, const int* stop = nullptr) {
         int cfg = 0;
         if constexpr (std::is_same<T2, float2>::value) {
             cfg = split ? choose_split(dev, A, B, C, alpha_re, alpha_im)
@@ -223,12 +232,12 @@ struct DevProduct {
         }
         if constexpr (std::is_same<T2, float2>::value) {
             if (split)
-                launch_split(dev, cfg, A, B, C, alpha_re, alpha_im);
+                launch_split(dev, cfg, A, B, C, alpha_re, alpha_im, stop);
             else
-                launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im);
+                launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im, stop);
         } else {
             KV_REQUIRE(!split, ERR_INTERNAL, "split-BF16 GEMM takes FP32 operands");
-            launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im);
+            launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im, stop);
         }
         if (log) {
             KV_HIP(hipEventRecord(b, dev.stream));
@@ -246,7 +255,7 @@ struct DevWFold {
         lists = upload_packed(dev, p.tasks, p.terms);
     }
     template <class T2>
-    void run(Device& dev, const T2* in, T2* out, EventLog* log = nullptr) const {
+    void run(Device& dev, const T2* in, T2* out, EventLog* log = nullptr, const int* stop = nullptr) const {
         hipEvent_t a = nullptr, b = nullptr;
         if (log) {
             a = log->get();
@@ -254,7 +263,7 @@ struct DevWFold {
             KV_HIP(hipEventRecord(a, dev.stream));
         }
         launch_wfold<T2>(dev.stream, in, out, lists.at<WTask>(0), (int)p.tasks.size(),
-                         lists.at<WTerm>(1), p.maxPQ);
+                         lists.at<WTerm>(1), p.maxPQ, stop);
         if (log) {
             KV_HIP(hipEventRecord(b, dev.stream));
             log->pending.push_back({a, b, p.flop, 1, 0.0});
@@ -376,39 +385,39 @@ struct Heff {
 
     template <class T2>
     void chain(const T2* Ld, const T2* Rd, const T2* x, T2* y, double alpha, EventLog* log,
-               bool split = false) {
-        s1.run<T2>(*dev, Ld, x, t1.as<T2>(), 1.0, 0.0, log, split);
+               bool split = false, const int* stop = nullptr) {
+        s1.run<T2>(*dev, Ld, x, t1.as<T2>(), 1.0, 0.0, log, split, stop);
         const T2* last = t1.as<T2>();
         // FP64 keeps the two folds one after the other (the reference's order of sums);
         // the FP32 operands take the one-pass composite, which saves a pass over the
         // intermediate at the cost of a different rounding order
         const bool one_pass = S.nsite == 2 && !std::is_same<T2, double2>::value;
         if (one_pass) {
-            s23.run<T2>(*dev, last, t3.as<T2>(), log);
+            s23.run<T2>(*dev, last, t3.as<T2>(), log, stop);
             last = t3.as<T2>();
         } else {
             if (S.nsite >= 1) {
-                s2.run<T2>(*dev, last, t2.as<T2>(), log);
+                s2.run<T2>(*dev, last, t2.as<T2>(), log, stop);
                 last = t2.as<T2>();
             }
             if (S.nsite == 2) {
-                s3.run<T2>(*dev, last, t3.as<T2>(), log);
+                s3.run<T2>(*dev, last, t3.as<T2>(), log, stop);
                 last = t3.as<T2>();
             }
         }
-        s4.run<T2>(*dev, last, Rd, y, alpha, 0.0, log, split);
+        s4.run<T2>(*dev, last, Rd, y, alpha, 0.0, log, split, stop);
     }
     // y = alpha * H_eff x, x and y FP64 slabs in layout() order; force64 runs the
-    // contractions in FP64 whatever the plan's precision
+    // contractions in FP64 whatever the plan's precision; stop: see kv_kernels.h
     void apply(const double2* x, double2* y, double alpha, EventLog* log = nullptr,
-               bool force64 = false) {
+               bool force64 = false, const int* stop = nullptr) {
         if (prec == PREC_F64 || force64) {
-            chain<double2>(L->d(), R->d(), x, y, alpha, log);
+            chain<double2>(L->d(), R->d(), x, y, alpha, log, false, stop);
         } else {
-            launch_f64_to_f32(dev->stream, x, x32.as<float2>(), S.xl.total);
+            launch_f64_to_f32(dev->stream, x, x32.as<float2>(), S.xl.total, stop);
             chain<float2>(L32.as<float2>(), R32.as<float2>(), x32.as<float2>(), y32.as<float2>(),
-                          1.0, log, prec == PREC_BF16X3);
-            launch_f32_to_f64(dev->stream, y32.as<float2>(), y, alpha, S.xl.total);
+                          1.0, log, prec == PREC_BF16X3, stop);
+            launch_f32_to_f64(dev->stream, y32.as<float2>(), y, alpha, S.xl.total, stop);
         }
     }
 };

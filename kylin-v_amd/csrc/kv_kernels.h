@@ -9,23 +9,28 @@
 
 namespace kv {
 
+// `stop` on the launches of an H_eff matvec: a device word; the kernel does nothing when it is
+// set (the Lanczos iteration it belongs to comes after the one that converged).
+
 // cfg selects the tile shape (kGemmConfigs in kv_types.h); tiles must have been cut for it
 template <class T2>
 void launch_gemm(hipStream_t st, int opA, int opB, const T2* A, const T2* B, T2* C,
                  const GemmTile* tiles, int ntiles, const GemmGroup* groups,
-                 const GemmSeg* segs, double alpha_re, double alpha_im, int cfg = 0);
+                 const GemmSeg* segs, double alpha_re, double alpha_im, int cfg = 0,
+                 const int* stop = nullptr);
 // Tile configs built per op pair and precision (every config is free of register spills).
 bool gemm_config_supports(int cfg, int opA, int opB, bool fp64);
 // Split-BF16 variant on the tile list of config 0 (64x64) or 4 (128x128): FP32 complex
 // operands and output.
 void launch_gemm_bf16x3(hipStream_t st, int opA, int opB, const float2* A, const float2* B,
                         float2* C, const GemmTile* tiles, int ntiles, const GemmGroup* groups,
-                        const GemmSeg* segs, double alpha_re, double alpha_im, int cfg);
+                        const GemmSeg* segs, double alpha_re, double alpha_im, int cfg,
+                        const int* stop = nullptr);
 
 // MPO fold; maxPQ = the largest task's P x Q (sets the workgroups per task).
 template <class T2>
 void launch_wfold(hipStream_t st, const T2* in, T2* out, const WTask* tasks, int ntasks,
-                  const WTerm* terms, int64_t maxPQ);
+                  const WTerm* terms, int64_t maxPQ, const int* stop = nullptr);
 
 template <class T2>
 void launch_perm(hipStream_t st, const T2* in, T2* out, const PermTask* tasks, int ntasks,
@@ -47,29 +52,39 @@ void launch_dotc(hipStream_t st, const double2* a, const double2* b, int64_t n,
                  double2* out, double* scratch);
 // out[0] = sum |a|^2
 void launch_nrm2sq(hipStream_t st, const double2* a, int64_t n, double* out, double* scratch);
-// y -= c[0] * x   (c on the device)
-void launch_axpy_neg_dev(hipStream_t st, double2* y, const double2* x, const double2* c,
-                         int64_t n);
-// y -= c[0] x (c on the device), then out = sum conj(y) z (complex) or sum |y|^2: the
-// subtraction and the reduction that follows it in one pass over y, with the arithmetic of
-// launch_axpy_neg_dev followed by launch_dotc / launch_nrm2sq.
-void launch_axpy_dotc(hipStream_t st, double2* y, const double2* x, const double2* c, const double2* z, int64_t n,
-                      double2* out, double* scratch);
-void launch_axpy_nrm2sq(hipStream_t st, double2* y, const double2* x, const double2* c, int64_t n, double* out,
-                        double* scratch);
-// dst = src / sqrt(nsq[0])  (nsq on the device)
-void launch_scale_invsqrt_dev(hipStream_t st, double2* dst, const double2* src,
-                              const double* nsq, int64_t n);
 // dst = src * s
 void launch_scale(hipStream_t st, double2* dst, const double2* src, double s, int64_t n);
 void launch_zaxpby(hipStream_t st, double2* out, const double2* x, const double2* y, double2 a,
                    double2 b, int64_t n);
-// out = sum_i c[i] * V[i*n + e],  c on the device
-void launch_lincomb(hipStream_t st, double2* out, const double2* V, const double2* c, int nv,
-                    int64_t n);
-void launch_f64_to_f32(hipStream_t st, const double2* src, float2* dst, int64_t n);
+// ---- Lanczos recurrence ----------------------------------------------------------------
+constexpr int kLanczosMax = 64;         // iterations of one call
+constexpr int kLanczosSmall = 12288;    // elements up to which one workgroup runs an iteration
+constexpr int kLanczosPart = 6 * 1024;  // doubles of reduction scratch
+// State of one call on the device: stop[k] set if iteration k is not to run.
+struct LanczosDev {
+    double2 beta, alpha;
+    double err[kLanczosMax + 1];
+    int stop[kLanczosMax + 1];
+};
+// One iteration's scalars in pinned host memory; complete once seen holds the launch's tag.
+struct LanczosHost {
+    double beta_re, beta_im, alpha_re, alpha_im, nsq, err;
+    unsigned long long seen;
+    double pad;
+};
+// v0 = x / |x|; resets the state.
+void launch_lanczos_begin(hipStream_t st, const double2* x, double2* v0, int64_t n, double* part, LanczosDev* dev);
+// h = H v_k -> beta (k > 0), alpha, |h|, v_{k+1} and the stop word of iteration k + 1: set when the
+// product of the residual norms is no longer above tol.  Does nothing when iteration k is stopped.
+void launch_lanczos_step(hipStream_t st, double2* h, const double2* vkm, const double2* vk, double2* vn, int64_t n,
+                         double* part, LanczosDev* dev, int k, double tol, LanczosHost* rec, uint64_t tag);
+// out = sum_i c_i V_i (c on the host, nv <= kLanczosMax); |out|^2 to rec->nsq.
+void launch_lanczos_end(hipStream_t st, double2* out, const double2* V, const double2* c, int nv, int64_t n,
+                        double* part, LanczosHost* rec, uint64_t tag);
+void launch_f64_to_f32(hipStream_t st, const double2* src, float2* dst, int64_t n, const int* stop = nullptr);
 // dst = s * src
-void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n);
+void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n,
+                       const int* stop = nullptr);
 
 // A[i ld + i] = (v, 0) for i in [from, to) (the diagonal of a square matrix).
 void launch_set_diag(hipStream_t st, double2* A, int64_t ld, int from, int to, double v);
@@ -86,7 +101,7 @@ void launch_hh_tfactor(hipStream_t st, const double2* S, const double2* tau, dou
                        int bw, int nref);
 // out[e] = sum_{p < np} part[p n + e]: partial products of a split-K GEMM summed.
 template <class T2>
-void launch_sum_parts(hipStream_t st, const T2* part, int np, int64_t n, T2* out);
+void launch_sum_parts(hipStream_t st, const T2* part, int np, int64_t n, T2* out, const int* stop = nullptr);
 // Z[j n + i] = C[(c0 + j) ldc + i]  (i < n, j < k): real columns to complex.
 void launch_real_cols(hipStream_t st, const double* C, int ldc, int c0, int k, int n, double2* Z);
 

@@ -60,7 +60,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM * BN <= 
     const typename Cx<T>::T2* __restrict__ A, const typename Cx<T>::T2* __restrict__ B,
     typename Cx<T>::T2* __restrict__ C, const GemmTile* __restrict__ tiles,
     const GemmGroup* __restrict__ groups, const GemmSeg* __restrict__ segs, T alpha_re,
-    T alpha_im) {
+    T alpha_im, const int* __restrict__ stop) {
+    if (stop && *stop) return;
     using T2 = typename Cx<T>::T2;
     using acc_t = typename Cx<T>::acc;
     constexpr int SI = BM / 32, SJ = BN / 32;  // 16x16 sub-tiles per wave
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM * BN <= 
 template <class T2>
 void launch_gemm(hipStream_t st, int opA, int opB, const T2* A, const T2* B, T2* C,
                  const GemmTile* tiles, int ntiles, const GemmGroup* groups,
-                 const GemmSeg* segs, double alpha_re, double alpha_im, int cfg) {
+                 const GemmSeg* segs, double alpha_re, double alpha_im, int cfg, const int* stop) {
     using T = typename ScalarOf<T2>::T;
     if (ntiles <= 0) return;
     const dim3 grid(ntiles), block(256);
@@ -374,7 +375,7 @@ void launch_gemm(hipStream_t st, int opA, int opB, const T2* A, const T2* B, T2*
 #define KV_GEMM_CASE(C_, OA, OB, BM_, BN_, BK_)                                                  \
     if (cfg == C_ && opA == OA && opB == OB) {                                                 \
         hipLaunchKernelGGL((zgemm_grouped_kernel<T, OA, OB, BM_, BN_, BK_>), grid, block, 0, st, \
-                           A, B, C, tiles, groups, segs, ar, ai);                              \
+                           A, B, C, tiles, groups, segs, ar, ai, stop);                        \
         KV_HIP(hipGetLastError());                                                             \
         return;                                                                                \
     }
@@ -420,10 +421,10 @@ bool gemm_config_supports(int cfg, int opA, int opB, bool fp64) {
 
 template void launch_gemm<double2>(hipStream_t, int, int, const double2*, const double2*,
                                    double2*, const GemmTile*, int, const GemmGroup*,
-                                   const GemmSeg*, double, double, int);
+                                   const GemmSeg*, double, double, int, const int*);
 template void launch_gemm<float2>(hipStream_t, int, int, const float2*, const float2*,
                                   float2*, const GemmTile*, int, const GemmGroup*,
-                                  const GemmSeg*, double, double, int);
+                                  const GemmSeg*, double, double, int, const int*);
 
 // ------------------------------------------------------------------------------------
 // grouped complex GEMM, split-BF16 (FP32 operands and accumulation)
@@ -459,7 +460,8 @@ template <int OPA, int OPB, int BM, int BN, int SI, int SJ>
 __global__ __launch_bounds__(64 * (BM / (16 * SI)) * (BN / (16 * SJ))) void zgemm_bf16x3_kernel(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C,
     const GemmTile* __restrict__ tiles, const GemmGroup* __restrict__ groups,
-    const GemmSeg* __restrict__ segs, float alpha_re, float alpha_im) {
+    const GemmSeg* __restrict__ segs, float alpha_re, float alpha_im, const int* __restrict__ stop) {
+    if (stop && *stop) return;
     constexpr int BK = 32, LDK = BK + 8;  // row pitch stays a multiple of 16 bytes
     constexpr int WN = BN / (16 * SJ), NT = 64 * (BM / (16 * SI)) * WN;
     __shared__ __attribute__((aligned(16))) __bf16 As[4][BM][LDK];
@@ -662,17 +664,17 @@ __global__ __launch_bounds__(64 * (BM / (16 * SI)) * (BN / (16 * SJ))) void zgem
 // the FP32 kernel's configs 0 and 4.
 void launch_gemm_bf16x3(hipStream_t st, int opA, int opB, const float2* A, const float2* B,
                         float2* C, const GemmTile* tiles, int ntiles, const GemmGroup* groups,
-                        const GemmSeg* segs, double alpha_re, double alpha_im, int cfg) {
+                        const GemmSeg* segs, double alpha_re, double alpha_im, int cfg, const int* stop) {
     if (ntiles <= 0) return;
     const float ar = (float)alpha_re, ai = (float)alpha_im;
 #define KV_BF_CASE(OA, OB)                                                                     \
     if (opA == OA && opB == OB) {                                                              \
         if (cfg == 4)                                                                          \
             hipLaunchKernelGGL((zgemm_bf16x3_kernel<OA, OB, 128, 128, 4, 2>), dim3(ntiles),     \
-                               dim3(512), 0, st, A, B, C, tiles, groups, segs, ar, ai);        \
+                               dim3(512), 0, st, A, B, C, tiles, groups, segs, ar, ai, stop);  \
         else                                                                                   \
             hipLaunchKernelGGL((zgemm_bf16x3_kernel<OA, OB, 64, 64, 2, 2>), dim3(ntiles),       \
-                               dim3(256), 0, st, A, B, C, tiles, groups, segs, ar, ai);        \
+                               dim3(256), 0, st, A, B, C, tiles, groups, segs, ar, ai, stop);  \
         KV_HIP(hipGetLastError());                                                             \
         return;                                                                                \
     }
@@ -701,7 +703,9 @@ template <class T2>
 __global__ __launch_bounds__(256) void wfold_kernel(const T2* __restrict__ in,
                                                     T2* __restrict__ out,
                                                     const WTask* __restrict__ tasks,
-                                                    const WTerm* __restrict__ terms) {
+                                                    const WTerm* __restrict__ terms,
+                                                    const int* __restrict__ stop) {
+    if (stop && *stop) return;
     using T = typename ScalarOf<T2>::T;
     const WTask tk = tasks[blockIdx.x];
     const WTerm* __restrict__ tt = terms + tk.term_begin;
@@ -764,19 +768,19 @@ __global__ __launch_bounds__(256) void wfold_kernel(const T2* __restrict__ in,
 
 template <class T2>
 void launch_wfold(hipStream_t st, const T2* in, T2* out, const WTask* tasks, int ntasks,
-                  const WTerm* terms, int64_t maxPQ) {
+                  const WTerm* terms, int64_t maxPQ, const int* stop) {
     if (ntasks <= 0) return;
     int64_t gy = (maxPQ + 255) / 256;
     if (gy > 64) gy = 64;
     if (gy < 1) gy = 1;
     hipLaunchKernelGGL((wfold_kernel<T2>), dim3(ntasks, (unsigned)gy), dim3(256), 0, st, in, out, tasks,
-                       terms);
+                       terms, stop);
     KV_HIP(hipGetLastError());
 }
 template void launch_wfold<double2>(hipStream_t, const double2*, double2*, const WTask*, int,
-                                    const WTerm*, int64_t);
+                                    const WTerm*, int64_t, const int*);
 template void launch_wfold<float2>(hipStream_t, const float2*, float2*, const WTask*, int,
-                                   const WTerm*, int64_t);
+                                   const WTerm*, int64_t, const int*);
 
 // ------------------------------------------------------------------------------------
 // block permutation
@@ -1007,111 +1011,396 @@ static unsigned ew_blocks(int64_t n) {
     return (unsigned)b;
 }
 
-__global__ __launch_bounds__(256) void axpy_neg_dev_kernel(double2* __restrict__ y,
-                                                           const double2* __restrict__ x,
-                                                           const double2* __restrict__ c,
-                                                           int64_t n) {
-    const double2 cc = c[0];
-    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-        const double2 v = x[e];
-        double2 o = y[e];
-        o.x -= cc.x * v.x - cc.y * v.y;
-        o.y -= cc.x * v.y + cc.y * v.x;
-        y[e] = o;
+// ---- Lanczos recurrence -------------------------------------------------------------
+// One iteration after h = H v_k: beta = <h|v_{k-1}>, h -= beta v_{k-1}, alpha = <h|v_k>,
+// h -= alpha v_k, |h|^2, v_{k+1} = h / |h|, in the reference's order and with one reduction
+// tree throughout: 256-element chunks dealt round-robin to up to RED_BLOCKS workgroups, a
+// pairwise tree over a workgroup's 256 lanes, then the same tree over the workgroups.
+// Long vectors (bound by HBM, 11 passes per iteration) take one launch per phase, each
+// forming the total of the phase before from its partials (at most 16 KB from L2) instead of
+// waiting for a one-workgroup kernel; short ones (kLanczosSmall: bound by launches, 2.2 us and
+// a gap each) run the whole recurrence in one workgroup with h in registers.  The launches
+// of an iteration read its stop word first, so the host may queue the next iteration before
+// it has seen the scalars of this one.
+// One site at D = 16, 4 levels (nine iterations of 11 launches, a copy and a wait each): 796 us a
+// call before, 368 now; the middle bond at D = 256, 16 levels with its SVD 32.0 -> 29.3 ms.
+
+// The total over a wave of values already summed to one per lane, in the tree's order.
+__device__ inline double tree64(double v) {
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v += __shfl_down(v, s);
+    return v;
+}
+
+// Total of nb partials (NC interleaved components), formed by every wave of a 256-thread
+// workgroup; sh holds 256 values per component.
+template <int NC>
+__device__ inline double2 partials_total(const double* __restrict__ part, int nb, double (*sh)[256]) {
+    double a = 0, b = 0;
+    for (int i = threadIdx.x; i < nb; i += 256) {
+        a += part[NC * i];
+        if (NC == 2) b += part[NC * i + 1];
+    }
+    __syncthreads();
+    sh[0][threadIdx.x] = a;
+    if (NC == 2) sh[1][threadIdx.x] = b;
+    __syncthreads();
+    const int t = threadIdx.x & 63;
+    double2 r = make_double2(0, 0);
+    r.x = __shfl(tree64((sh[0][t] + sh[0][t + 128]) + (sh[0][t + 64] + sh[0][t + 192])), 0);
+    if (NC == 2) r.y = __shfl(tree64((sh[1][t] + sh[1][t + 128]) + (sh[1][t + 64] + sh[1][t + 192])), 0);
+    return r;
+}
+
+// A workgroup's partial from its 256 lanes' sums.
+template <int NC>
+__device__ inline void partial_store(double a, double b, double* __restrict__ part, double (*sh)[256]) {
+    __syncthreads();
+    sh[0][threadIdx.x] = a;
+    if (NC == 2) sh[1][threadIdx.x] = b;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int t = threadIdx.x;
+    const double x = tree64((sh[0][t] + sh[0][t + 128]) + (sh[0][t + 64] + sh[0][t + 192]));
+    double y = 0;
+    if (NC == 2) y = tree64((sh[1][t] + sh[1][t + 128]) + (sh[1][t + 64] + sh[1][t + 192]));
+    if (t == 0) {
+        part[NC * blockIdx.x] = x;
+        if (NC == 2) part[NC * blockIdx.x + 1] = y;
     }
 }
 
-void launch_axpy_neg_dev(hipStream_t st, double2* y, const double2* x, const double2* c,
-                         int64_t n) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(axpy_neg_dev_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, y, x, c, n);
-    KV_HIP(hipGetLastError());
+// What the host reads of iteration k; `seen` is written last.
+__device__ inline void lanczos_publish(LanczosHost* rec, double2 beta, double2 alpha, double nsq, double err,
+                                       unsigned long long tag) {
+    rec->beta_re = beta.x;
+    rec->beta_im = beta.y;
+    rec->alpha_re = alpha.x;
+    rec->alpha_im = alpha.y;
+    rec->nsq = nsq;
+    rec->err = err;
+    __threadfence_system();
+    __hip_atomic_store(&rec->seen, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Lanczos passes fused with the subtraction that precedes them: y -= c[0] x, written back,
-// then per-workgroup partial sums of conj(y) z (DOT) or of |y|^2 for reduce2_final_kernel.
-// Element formulas, the element-to-block assignment and the reduction tree are those of
-// axpy_neg_dev_kernel followed by dotc_partial_kernel / nrm2sq_partial_kernel.
-template <bool DOT>
-__global__ __launch_bounds__(256) void axpy_reduce_partial_kernel(double2* __restrict__ y,
-                                                                  const double2* __restrict__ x,
-                                                                  const double2* __restrict__ c,
-                                                                  const double2* __restrict__ z, int64_t n,
-                                                                  double* __restrict__ part) {
-    __shared__ double sr[256], si[256];
-    const double2 cc = c[0];
-    double re = 0, im = 0;
+// partial sums of |x|^2; clears the call's stop words and sets err[0] = 1.
+__global__ __launch_bounds__(256) void lanczos_begin_kernel(const double2* __restrict__ x, int64_t n,
+                                                            double* __restrict__ part, LanczosDev* __restrict__ st) {
+    __shared__ double sh[1][256];
+    if (blockIdx.x == 0 && threadIdx.x <= kLanczosMax) {
+        st->stop[threadIdx.x] = 0;
+        if (threadIdx.x == 0) st->err[0] = 1.0;
+    }
+    double re = 0;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
         const double2 v = x[e];
-        double2 o = y[e];
-        o.x -= cc.x * v.x - cc.y * v.y;
-        o.y -= cc.x * v.y + cc.y * v.x;
-        y[e] = o;
-        if constexpr (DOT) {
+        re += v.x * v.x + v.y * v.y;
+    }
+    partial_store<1>(re, 0, part, sh);
+}
+
+// v_0 = x / |x| from the partials of lanczos_begin_kernel.
+__global__ __launch_bounds__(256) void lanczos_first_kernel(const double2* __restrict__ x, double2* __restrict__ v0,
+                                                            int64_t n, const double* __restrict__ part, int nb) {
+    __shared__ double sh[1][256];
+    const double f = 1.0 / sqrt(partials_total<1>(part, nb, sh).x);
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+        double2 v = x[e];
+        v.x *= f;
+        v.y *= f;
+        v0[e] = v;
+    }
+}
+
+// Phases of one iteration.  DOT: partials of <h|z> alone (the first phase).  SUBDOT: c = the
+// total of the phase before, kept in *c_out; h -= c x; partials of <h|z>.  SUBNRM: the same with
+// |h|^2.
+enum { LZ_DOT, LZ_SUBDOT, LZ_SUBNRM };
+template <int PHASE>
+__global__ __launch_bounds__(256) void lanczos_phase_kernel(double2* __restrict__ h, const double2* __restrict__ x,
+                                                            const double2* __restrict__ z, int64_t n,
+                                                            const double* __restrict__ in, int nb,
+                                                            double* __restrict__ out, double2* __restrict__ c_out,
+                                                            const int* __restrict__ stop) {
+    if (*stop) return;
+    __shared__ double sh[2][256];
+    double2 c = make_double2(0, 0);
+    if constexpr (PHASE != LZ_DOT) {
+        c = partials_total<2>(in, nb, sh);
+        if (blockIdx.x == 0 && threadIdx.x == 0) *c_out = c;
+    }
+    double re = 0, im = 0;
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+        double2 o = h[e];
+        if constexpr (PHASE != LZ_DOT) {
+            const double2 v = x[e];
+            o.x -= c.x * v.x - c.y * v.y;
+            o.y -= c.x * v.y + c.y * v.x;
+            h[e] = o;
+        }
+        if constexpr (PHASE == LZ_SUBNRM) {
+            re += o.x * o.x + o.y * o.y;
+        } else {
             const double2 w = z[e];
             re += o.x * w.x + o.y * w.y;  // conj(o) * w
             im += o.x * w.y - o.y * w.x;
-        } else {
-            re += o.x * o.x + o.y * o.y;
         }
     }
-    sr[threadIdx.x] = re;
-    if constexpr (DOT) si[threadIdx.x] = im;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            sr[threadIdx.x] += sr[threadIdx.x + s];
-            if constexpr (DOT) si[threadIdx.x] += si[threadIdx.x + s];
-        }
-        __syncthreads();
+    partial_store<PHASE == LZ_SUBNRM ? 1 : 2>(re, im, out, sh);
+}
+
+// |h|^2 from its partials, err_{k+1} = err_k |h| and the stop word of iteration k + 1; unless
+// stopped, v_{k+1} = h / |h|.
+__global__ __launch_bounds__(256) void lanczos_next_kernel(const double2* __restrict__ h, double2* __restrict__ vn,
+                                                           int64_t n, const double* __restrict__ part, int nb,
+                                                           LanczosDev* __restrict__ st, int k, double tol,
+                                                           LanczosHost* rec, unsigned long long tag) {
+    if (st->stop[k]) return;
+    __shared__ double sh[1][256];
+    const double nsq = partials_total<1>(part, nb, sh).x;
+    const double err = st->err[k] * sqrt(nsq);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->err[k + 1] = err;
+        st->stop[k + 1] = !(err > tol);
+        lanczos_publish(rec, st->beta, st->alpha, nsq, err, tag);
     }
-    if (threadIdx.x == 0) {
-        if constexpr (DOT) {
-            part[2 * blockIdx.x] = sr[0];
-            part[2 * blockIdx.x + 1] = si[0];
-        } else {
-            part[blockIdx.x] = sr[0];
-        }
-    }
-}
-
-void launch_axpy_dotc(hipStream_t st, double2* y, const double2* x, const double2* c, const double2* z, int64_t n,
-                      double2* out, double* scratch) {
-    const int nb = red_blocks(n);
-    hipLaunchKernelGGL(axpy_reduce_partial_kernel<true>, dim3(nb), dim3(256), 0, st, y, x, c, z, n, scratch);
-    KV_HIP(hipGetLastError());
-    hipLaunchKernelGGL(reduce2_final_kernel, dim3(1), dim3(256), 0, st, scratch, nb, reinterpret_cast<double*>(out),
-                       2);
-    KV_HIP(hipGetLastError());
-}
-
-void launch_axpy_nrm2sq(hipStream_t st, double2* y, const double2* x, const double2* c, int64_t n, double* out,
-                        double* scratch) {
-    const int nb = red_blocks(n);
-    hipLaunchKernelGGL(axpy_reduce_partial_kernel<false>, dim3(nb), dim3(256), 0, st, y, x, c, nullptr, n, scratch);
-    KV_HIP(hipGetLastError());
-    hipLaunchKernelGGL(reduce2_final_kernel, dim3(1), dim3(256), 0, st, scratch, nb, out, 1);
-    KV_HIP(hipGetLastError());
-}
-
-__global__ __launch_bounds__(256) void scale_invsqrt_dev_kernel(double2* __restrict__ dst,
-                                                                const double2* __restrict__ src,
-                                                                const double* __restrict__ nsq,
-                                                                int64_t n) {
-    const double f = 1.0 / sqrt(nsq[0]);
+    if (!(err > tol)) return;
+    const double f = 1.0 / sqrt(nsq);
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-        double2 v = src[e];
+        double2 v = h[e];
         v.x *= f;
         v.y *= f;
-        dst[e] = v;
+        vn[e] = v;
     }
 }
 
-void launch_scale_invsqrt_dev(hipStream_t st, double2* dst, const double2* src,
-                              const double* nsq, int64_t n) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(scale_invsqrt_dev_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, dst, src,
-                       nsq, n);
+// One wave's partial of a 256-element chunk: lane t holds elements t, t + 64, t + 128, t + 192.
+__device__ inline double chunk_sum(const double (&p)[4]) { return tree64((p[0] + p[2]) + (p[1] + p[3])); }
+// Total of nb <= 64 chunk partials, in every lane.
+__device__ inline double chunks_total(const double* sh, int nb) {
+    const int t = threadIdx.x & 63;
+    return __shfl(tree64(t < nb ? sh[t] : 0.0), 0);
+}
+
+// v_0 = x / |x| and the call's state, in one workgroup (n <= kLanczosSmall).
+__global__ __launch_bounds__(1024) void lanczos_first_small_kernel(const double2* __restrict__ x,
+                                                                   double2* __restrict__ v0, int n,
+                                                                   LanczosDev* __restrict__ st) {
+    __shared__ double sh[64];
+    const int wave = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int nb = (n + 255) / 256;
+    if (threadIdx.x <= kLanczosMax) {
+        st->stop[threadIdx.x] = 0;
+        if (threadIdx.x == 0) st->err[0] = 1.0;
+    }
+    for (int b = wave; b < nb; b += 16) {
+        double p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int e = b * 256 + j * 64 + t;
+            const double2 v = e < n ? x[e] : make_double2(0, 0);
+            p[j] = v.x * v.x + v.y * v.y;
+        }
+        const double s = chunk_sum(p);
+        if (t == 0) sh[b] = s;
+    }
+    __syncthreads();
+    const double f = 1.0 / sqrt(chunks_total(sh, nb));
+    for (int e = threadIdx.x; e < n; e += 1024) {
+        double2 v = x[e];
+        v.x *= f;
+        v.y *= f;
+        v0[e] = v;
+    }
+}
+
+// The whole recurrence of one iteration in one workgroup (n <= kLanczosSmall = 16 waves x NC
+// chunks x 256): h stays in registers from its first read to v_{k+1}.
+template <int NC>
+__global__ __launch_bounds__(1024) void lanczos_small_kernel(const double2* __restrict__ h,
+                                                             const double2* __restrict__ vkm,
+                                                             const double2* __restrict__ vk,
+                                                             double2* __restrict__ vn, int n,
+                                                             LanczosDev* __restrict__ st, int k, double tol,
+                                                             LanczosHost* rec, unsigned long long tag) {
+    if (st->stop[k]) return;
+    __shared__ double sr[64], si[64];
+    const int wave = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int nb = (n + 255) / 256;
+    // v_{k-1}, then v_k: kept beside h where the registers hold both (128 per lane), else read
+    // twice (from L2)
+    constexpr bool KEEP = NC <= 2;
+    double2 r[NC][4], v[KEEP ? NC : 1][4];
+    auto at = [&](const double2* p, int c, int j) -> double2 {
+        const int e = (wave + 16 * c) * 256 + j * 64 + t;
+        return e < n ? p[e] : make_double2(0, 0);
+    };
+    const double2* src = k > 0 ? vkm : vk;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            r[c][j] = at(h, c, j);
+            if (KEEP) v[c][j] = at(src, c, j);
+        }
+    auto dot = [&]() -> double2 {  // <r|v>
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            double p[4], q[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const double2 w = KEEP ? v[KEEP ? c : 0][j] : at(src, c, j);
+                p[j] = r[c][j].x * w.x + r[c][j].y * w.y;
+                q[j] = r[c][j].x * w.y - r[c][j].y * w.x;
+            }
+            const double a = chunk_sum(p), b = chunk_sum(q);
+            if (t == 0) {
+                sr[wave + 16 * c] = a;
+                si[wave + 16 * c] = b;
+            }
+        }
+        __syncthreads();
+        const double2 d = make_double2(chunks_total(sr, nb), chunks_total(si, nb));
+        __syncthreads();
+        return d;
+    };
+    auto sub = [&](double2 d) {  // r -= d v
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const double2 w = KEEP ? v[KEEP ? c : 0][j] : at(src, c, j);
+                r[c][j].x -= d.x * w.x - d.y * w.y;
+                r[c][j].y -= d.x * w.y + d.y * w.x;
+            }
+    };
+    double2 beta = make_double2(0, 0);
+    if (k > 0) {
+        beta = dot();
+        sub(beta);
+        src = vk;
+        if (KEEP) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[KEEP ? c : 0][j] = at(src, c, j);
+        }
+    }
+    const double2 alpha = dot();
+    sub(alpha);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        double p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = r[c][j].x * r[c][j].x + r[c][j].y * r[c][j].y;
+        const double a = chunk_sum(p);
+        if (t == 0) sr[wave + 16 * c] = a;
+    }
+    __syncthreads();
+    const double nsq = chunks_total(sr, nb);
+    const double err = st->err[k] * sqrt(nsq);
+    if (threadIdx.x == 0) {
+        st->err[k + 1] = err;
+        st->stop[k + 1] = !(err > tol);
+        lanczos_publish(rec, beta, alpha, nsq, err, tag);
+    }
+    if (!(err > tol)) return;
+    const double f = 1.0 / sqrt(nsq);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int e = (wave + 16 * c) * 256 + j * 64 + t;
+            if (e < n) vn[e] = make_double2(f * r[c][j].x, f * r[c][j].y);
+        }
+}
+
+// out = sum_i c_i V_i and the partials of |out|^2; the coefficients travel as an argument.
+struct LincombArgs {
+    double2 c[kLanczosMax];
+};
+__global__ __launch_bounds__(256) void lincomb_kernel(double2* __restrict__ out, const double2* __restrict__ V,
+                                                      LincombArgs a, int nv, int64_t n, double* __restrict__ part) {
+    __shared__ double sh[1][256];
+    double sq = 0;
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+        double re = 0, im = 0;
+        for (int i = 0; i < nv; ++i) {
+            const double2 v = V[(int64_t)i * n + e];
+            const double2 ci = a.c[i];
+            re += ci.x * v.x - ci.y * v.y;
+            im += ci.x * v.y + ci.y * v.x;
+        }
+        out[e] = make_double2(re, im);
+        sq += re * re + im * im;
+    }
+    partial_store<1>(sq, 0, part, sh);
+}
+
+// The total of nb partials to the host.
+__global__ __launch_bounds__(256) void lanczos_end_kernel(const double* __restrict__ part, int nb, LanczosHost* rec,
+                                                          unsigned long long tag) {
+    __shared__ double sh[1][256];
+    const double s = partials_total<1>(part, nb, sh).x;
+    if (threadIdx.x == 0) lanczos_publish(rec, make_double2(0, 0), make_double2(0, 0), s, 0, tag);
+}
+
+void launch_lanczos_begin(hipStream_t st, const double2* x, double2* v0, int64_t n, double* part, LanczosDev* dev) {
+    if (n <= kLanczosSmall) {
+        hipLaunchKernelGGL(lanczos_first_small_kernel, dim3(1), dim3(1024), 0, st, x, v0, (int)n, dev);
+        KV_HIP(hipGetLastError());
+        return;
+    }
+    const int nb = red_blocks(n);
+    hipLaunchKernelGGL(lanczos_begin_kernel, dim3(nb), dim3(256), 0, st, x, n, part, dev);
+    KV_HIP(hipGetLastError());
+    hipLaunchKernelGGL(lanczos_first_kernel, dim3(nb), dim3(256), 0, st, x, v0, n, part, nb);
+    KV_HIP(hipGetLastError());
+}
+
+void launch_lanczos_step(hipStream_t st, double2* h, const double2* vkm, const double2* vk, double2* vn, int64_t n,
+                         double* part, LanczosDev* dev, int k, double tol, LanczosHost* rec, uint64_t tag) {
+    if (n <= kLanczosSmall) {
+        static_assert(kLanczosSmall == 3 * 16 * 256, "the chunks of the largest variant");
+        const auto f = n <= kLanczosSmall / 3       ? lanczos_small_kernel<1>
+                       : n <= 2 * kLanczosSmall / 3 ? lanczos_small_kernel<2>
+                                                    : lanczos_small_kernel<3>;
+        hipLaunchKernelGGL(f, dim3(1), dim3(1024), 0, st, h, vkm, vk, vn, (int)n, dev, k, tol, rec,
+                           (unsigned long long)tag);
+        KV_HIP(hipGetLastError());
+        return;
+    }
+    const int nb = red_blocks(n);
+    const dim3 grid(nb), block(256);
+    double *pa = part, *pb = part + 2 * RED_BLOCKS, *pc = part + 4 * RED_BLOCKS;
+    const int* stop = &dev->stop[k];
+    if (k > 0) {
+        hipLaunchKernelGGL(lanczos_phase_kernel<LZ_DOT>, grid, block, 0, st, h, nullptr, vkm, n, nullptr, 0, pa,
+                           nullptr, stop);
+        KV_HIP(hipGetLastError());
+        hipLaunchKernelGGL(lanczos_phase_kernel<LZ_SUBDOT>, grid, block, 0, st, h, vkm, vk, n, pa, nb, pb, &dev->beta,
+                           stop);
+    } else {
+        hipLaunchKernelGGL(lanczos_phase_kernel<LZ_DOT>, grid, block, 0, st, h, nullptr, vk, n, nullptr, 0, pb,
+                           nullptr, stop);
+    }
+    KV_HIP(hipGetLastError());
+    hipLaunchKernelGGL(lanczos_phase_kernel<LZ_SUBNRM>, grid, block, 0, st, h, vk, nullptr, n, pb, nb, pc, &dev->alpha,
+                       stop);
+    KV_HIP(hipGetLastError());
+    hipLaunchKernelGGL(lanczos_next_kernel, grid, block, 0, st, h, vn, n, pc, nb, dev, k, tol, rec,
+                       (unsigned long long)tag);
+    KV_HIP(hipGetLastError());
+}
+
+void launch_lanczos_end(hipStream_t st, double2* out, const double2* V, const double2* c, int nv, int64_t n,
+                        double* part, LanczosHost* rec, uint64_t tag) {
+    const int nb = red_blocks(n);
+    LincombArgs a{};
+    for (int i = 0; i < nv; ++i) a.c[i] = c[i];
+    hipLaunchKernelGGL(lincomb_kernel, dim3(nb), dim3(256), 0, st, out, V, a, nv, n, part);
+    KV_HIP(hipGetLastError());
+    hipLaunchKernelGGL(lanczos_end_kernel, dim3(1), dim3(256), 0, st, part, nb, rec, (unsigned long long)tag);
     KV_HIP(hipGetLastError());
 }
 
@@ -1160,55 +1449,35 @@ void launch_zaxpby(hipStream_t st, double2* out, const double2* x, const double2
     KV_HIP(hipGetLastError());
 }
 
-__global__ __launch_bounds__(256) void lincomb_kernel(double2* __restrict__ out,
-                                                      const double2* __restrict__ V,
-                                                      const double2* __restrict__ c, int nv,
-                                                      int64_t n) {
-    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-        double re = 0, im = 0;
-        for (int i = 0; i < nv; ++i) {
-            const double2 v = V[(int64_t)i * n + e];
-            const double2 ci = c[i];
-            re += ci.x * v.x - ci.y * v.y;
-            im += ci.x * v.y + ci.y * v.x;
-        }
-        out[e] = make_double2(re, im);
-    }
-}
-
-void launch_lincomb(hipStream_t st, double2* out, const double2* V, const double2* c, int nv,
-                    int64_t n) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(lincomb_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, out, V, c, nv, n);
-    KV_HIP(hipGetLastError());
-}
-
 __global__ __launch_bounds__(256) void f64_to_f32_kernel(const double2* __restrict__ s,
-                                                         float2* __restrict__ d, int64_t n) {
+                                                         float2* __restrict__ d, int64_t n,
+                                                         const int* __restrict__ stop) {
+    if (stop && *stop) return;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
         const double2 v = s[e];
         d[e] = make_float2((float)v.x, (float)v.y);
     }
 }
 
-void launch_f64_to_f32(hipStream_t st, const double2* src, float2* dst, int64_t n) {
+void launch_f64_to_f32(hipStream_t st, const double2* src, float2* dst, int64_t n, const int* stop) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(f64_to_f32_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, src, dst, n);
+    hipLaunchKernelGGL(f64_to_f32_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, src, dst, n, stop);
     KV_HIP(hipGetLastError());
 }
 
 __global__ __launch_bounds__(256) void f32_to_f64_kernel(const float2* __restrict__ s,
                                                          double2* __restrict__ d, double f,
-                                                         int64_t n) {
+                                                         int64_t n, const int* __restrict__ stop) {
+    if (stop && *stop) return;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
         const float2 v = s[e];
         d[e] = make_double2(f * (double)v.x, f * (double)v.y);
     }
 }
 
-void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n) {
+void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n, const int* stop) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(f32_to_f64_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, src, dst, s, n);
+    hipLaunchKernelGGL(f32_to_f64_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, src, dst, s, n, stop);
     KV_HIP(hipGetLastError());
 }
 
@@ -1365,7 +1634,9 @@ void launch_hh_tfactor(hipStream_t st, const double2* S, const double2* tau, dou
 // Bound by the partials' read (np x n elements from L2 / HBM); eight loads in flight per lane.
 template <class T2>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const T2* __restrict__ part, int np,
-                                                        int64_t n, T2* __restrict__ out) {
+                                                        int64_t n, T2* __restrict__ out,
+                                                        const int* __restrict__ stop) {
+    if (stop && *stop) return;
     using T = typename ScalarOf<T2>::T;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
         T re = 0, im = 0;
@@ -1383,13 +1654,13 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const T2* __restrict__ p
 }
 
 template <class T2>
-void launch_sum_parts(hipStream_t st, const T2* part, int np, int64_t n, T2* out) {
+void launch_sum_parts(hipStream_t st, const T2* part, int np, int64_t n, T2* out, const int* stop) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(sum_parts_kernel<T2>, dim3(ew_blocks(n)), dim3(256), 0, st, part, np, n, out);
+    hipLaunchKernelGGL(sum_parts_kernel<T2>, dim3(ew_blocks(n)), dim3(256), 0, st, part, np, n, out, stop);
     KV_HIP(hipGetLastError());
 }
-template void launch_sum_parts<double2>(hipStream_t, const double2*, int, int64_t, double2*);
-template void launch_sum_parts<float2>(hipStream_t, const float2*, int, int64_t, float2*);
+template void launch_sum_parts<double2>(hipStream_t, const double2*, int, int64_t, double2*, const int*);
+template void launch_sum_parts<float2>(hipStream_t, const float2*, int, int64_t, float2*, const int*);
 
 // Z[j n + i] = C[(c0 + j) ldc + i] for i < n, j < k (real columns to complex).
 __global__ __launch_bounds__(256) void real_cols_kernel(const double* __restrict__ C, int ldc, int c0,

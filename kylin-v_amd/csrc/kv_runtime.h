@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "kv_error.h"
+#include "kv_kernels.h"
 
 namespace kv {
 
@@ -239,12 +240,21 @@ struct Device {
     // GEMM tile autotuner: (precision, opA, opB, shape class) -> tile config
     bool autotune = true;
     std::map<uint64_t, int> gemm_tuned;
+    // Lanczos state: the device's, and one record per iteration (the last one the result's norm)
+    // in pinned host memory; a call's records carry tags of their own.
+    LanczosDev* lanczos_dev = nullptr;
+    LanczosHost* lanczos_host = nullptr;
+    uint64_t lanczos_calls = 0;
     explicit Device(int dev) : id(dev) {
         KV_HIP(hipSetDevice(dev));
         KV_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         pool.reset(new Pool(dev));
         if (const char* a = std::getenv("KV_AUTOTUNE")) autotune = a[0] != '0';
         KV_HIP(hipHostMalloc(&ring_, kRingBytes, hipHostMallocDefault));
+        KV_HIP(hipHostMalloc((void**)&lanczos_host, (kLanczosMax + 1) * sizeof(LanczosHost),
+                             hipHostMallocMapped | hipHostMallocCoherent));
+        std::memset((void*)lanczos_host, 0, (kLanczosMax + 1) * sizeof(LanczosHost));
+        KV_HIP(hipMalloc((void**)&lanczos_dev, sizeof(LanczosDev)));
     }
     ~Device() {
         if (stream) {
@@ -253,6 +263,8 @@ struct Device {
             (void)hipStreamDestroy(stream);
         }
         if (ring_) (void)hipHostFree(ring_);
+        if (lanczos_host) (void)hipHostFree(lanczos_host);
+        if (lanczos_dev) (void)hipFree(lanczos_dev);
     }
     Device(const Device&) = delete;
     Device& operator=(const Device&) = delete;
@@ -261,6 +273,25 @@ struct Device {
         KV_HIP(hipStreamSynchronize(stream));
         ring_off_ = 0;
         spans.resolve();
+    }
+    // Waits until the record that launch `tag` publishes has arrived.  The stream is asked now and
+    // then, so that a failed launch ends the wait with its error.
+    void wait_record(const LanczosHost& r, uint64_t tag) {
+        for (unsigned spin = 1;; ++spin) {
+            if (__atomic_load_n(&r.seen, __ATOMIC_ACQUIRE) == tag) return;
+            if (spin % 4096) {
+                __builtin_ia32_pause();
+                continue;
+            }
+            const hipError_t e = hipStreamQuery(stream);
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();
+                continue;
+            }
+            KV_HIP(e);
+            if (__atomic_load_n(&r.seen, __ATOMIC_ACQUIRE) == tag) return;
+            throw Error(ERR_INTERNAL, "Lanczos scalars did not arrive");
+        }
     }
     // Host-to-device copy of a small host array (work descriptors) that returns without
     // waiting: the bytes go through a pinned staging ring, whose slots are reused only after
