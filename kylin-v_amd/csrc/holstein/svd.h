@@ -4,8 +4,9 @@
 //
 // Per charge sector three FP64 routes (sectors whose smaller side is below iso_min, and
 // zero-keeping truncations that cannot take a Gram route, use the first):
-//  * exact: rocSOLVER one-sided Jacobi (zgesvdj), or zgesvd when cutoff < 0 keeps zero
-//    singular values (their vectors must still be an orthonormal completion);
+//  * exact: the engine's one-workgroup Jacobi SVD where jacobi_takes the sector (all of a
+//    bond in one launch), else rocSOLVER's (zgesvdj, or zgesvd when cutoff < 0 keeps zero
+//    singular values, whose vectors must still be an orthonormal completion);
 //  * smaller-side Gram (when the isometry is the larger side): G on the smaller side by
 //    the MFMA GEMM, Hermitian eigen-decomposition (batched zhetrd, dstedc per sector,
 //    eigenvectors back-transformed only for the kept values), the isometry as M V / s by
@@ -206,7 +207,7 @@ struct SectorSvd {
     bool colside = true;  // Gram of M^H M (else M M^H)
     bool s_absorbed = false;  // the non-isometric factor already carries S
     double gscale = 1.0;      // G was divided by this (|M|_F^2) before the eigensolver
-    DevBuf M, G, S, U, Vh;  // U: nr x ldU, Vh: k x nc
+    DevBuf M, G, U, Vh;  // U: nr x ldU, Vh: k x nc
     int ldU = 0;
     std::vector<double> s;  // descending
     // Gram eigenvectors: rows [ev_lo, k) of the ascending eigenvector matrix, row j - ev_lo of
@@ -237,7 +238,7 @@ inline void exact_sector(Device& D, Solver& sol, SectorSvd& X, bool keep_zero) {
     DevBuf A(D.pool.get(), (size_t)(X.nr * X.nc) * sizeof(double2));
     KV_HIP(hipMemcpyAsync(A.get(), X.M.get(), (size_t)(X.nr * X.nc) * sizeof(double2),
                           hipMemcpyDeviceToDevice, D.stream));
-    X.S = DevBuf(D.pool.get(), (size_t)k * sizeof(double));
+    DevBuf S(D.pool.get(), (size_t)k * sizeof(double));
     X.Vh = DevBuf(D.pool.get(), (size_t)(X.nc * k) * sizeof(double2));  // rocSOLVER U
     X.U = DevBuf(D.pool.get(), (size_t)(k * X.nr) * sizeof(double2));   // rocSOLVER V^H
     DevBuf E(D.pool.get(), (size_t)std::max(k, 1) * sizeof(double));
@@ -250,21 +251,87 @@ inline void exact_sector(Device& D, Solver& sol, SectorSvd& X, bool keep_zero) {
         DevBuf res(D.pool.get(), sizeof(double)), nsw(D.pool.get(), sizeof(rocblas_int));
         st = rocsolver_zgesvdj(sol.h, rocblas_svect_singular, rocblas_svect_singular,
                                (rocblas_int)X.nc, (rocblas_int)X.nr, a, (rocblas_int)X.nc, 0.0,
-                               res.as<double>(), 100, nsw.as<rocblas_int>(), X.S.as<double>(), u,
+                               res.as<double>(), 100, nsw.as<rocblas_int>(), S.as<double>(), u,
                                (rocblas_int)X.nc, v, (rocblas_int)k, info.as<rocblas_int>());
     } else {
         st = rocsolver_zgesvd(sol.h, rocblas_svect_singular, rocblas_svect_singular,
                               (rocblas_int)X.nc, (rocblas_int)X.nr, a, (rocblas_int)X.nc,
-                              X.S.as<double>(), u, (rocblas_int)X.nc, v, (rocblas_int)k,
+                              S.as<double>(), u, (rocblas_int)X.nc, v, (rocblas_int)k,
                               E.as<double>(), rocblas_outofplace, info.as<rocblas_int>());
     }
     KV_REQUIRE(st == rocblas_status_success, ERR_SOLVER, "rocSOLVER SVD failed");
     rocblas_int hinfo = 0;
     X.s.resize(k);
     KV_HIP(hipMemcpyAsync(&hinfo, info.get(), sizeof(rocblas_int), hipMemcpyDeviceToHost, D.stream));
-    KV_HIP(hipMemcpyAsync(X.s.data(), X.S.get(), k * sizeof(double), hipMemcpyDeviceToHost, D.stream));
+    KV_HIP(hipMemcpyAsync(X.s.data(), S.get(), k * sizeof(double), hipMemcpyDeviceToHost, D.stream));
     D.sync();
     KV_REQUIRE(hinfo == 0, ERR_SOLVER, "Problems in SVD (did not converge)");
+}
+
+// Sectors the one-workgroup SVD takes.  Above kJacobiElems its reflectors would walk the long side
+// through one CU for longer than zgeqrf's launches take.  Under a truncating cutoff it starts at a
+// larger side of kJacobiLong: chains whose sectors are all smaller than that (the
+// projected-purification layout) truncate at values below what zgesvdj resolves, so what they
+// keep, and with it their results at the 1e-10 level, follows zgesvdj's rounding (an 8-site step:
+// energy 4e-10 where it is 0, and 2e-12 with this kernel, in 59 instead of 114 ms), and runs of
+// such chains go on as they began.
+constexpr int64_t kJacobiElems = (int64_t)1 << 18, kJacobiLong = 128;
+inline bool jacobi_takes(int64_t nr, int64_t nc, double cutoff) {
+    return std::min(nr, nc) <= kJacobiMax && nr * nc <= kJacobiElems &&
+           (cutoff < 0.0 || std::max(nr, nc) >= kJacobiLong);
+}
+
+// The exact route for sectors that jacobi_takes: all of them in one launch and one wait.  With
+// keep_zero a sector whose smallest values vanish next to its largest goes to zgesvd, whose
+// vectors for them are an orthonormal completion.
+inline void jacobi_sectors(Device& D, Solver& sol, const std::vector<SectorSvd*>& xs, bool keep_zero) {
+    if (xs.empty()) return;
+    std::vector<SvdJob> jobs;
+    std::vector<size_t> soff;
+    size_t work = 0, ns = 0;
+    int nmax = 0, mmax = 0;
+    for (auto* x : xs) {
+        work += (size_t)(x->nr * x->nc) * (x->nr >= x->nc ? 2 : 1);
+        soff.push_back(ns);
+        ns += (size_t)std::min(x->nr, x->nc);
+    }
+    DevBuf W(D.pool.get(), work * sizeof(double2)), S(D.pool.get(), ns * sizeof(double));
+    size_t at = 0;
+    for (size_t i = 0; i < xs.size(); ++i) {
+        SectorSvd& X = *xs[i];
+        const int k = (int)std::min(X.nr, X.nc);
+        X.k = X.ldU = k;
+        X.gram = false;
+        X.U = DevBuf(D.pool.get(), (size_t)(X.nr * k) * sizeof(double2));
+        X.Vh = DevBuf(D.pool.get(), (size_t)(X.nc * k) * sizeof(double2));
+        SvdJob j{};
+        j.M = X.M.as<double2>();
+        j.U = X.U.as<double2>();
+        j.Vh = X.Vh.as<double2>();
+        j.A = W.as<double2>() + at;
+        at += (size_t)(X.nr * X.nc);
+        if (X.nr >= X.nc) {
+            j.T = W.as<double2>() + at;
+            at += (size_t)(X.nr * X.nc);
+        }
+        j.S = S.as<double>() + soff[i];
+        j.nr = (int)X.nr;
+        j.nc = (int)X.nc;
+        jobs.push_back(j);
+        nmax = std::max(nmax, k);
+        mmax = std::max(mmax, (int)std::max(X.nr, X.nc));
+    }
+    DevBuf dj = upload_vec(D, jobs);
+    launch_jacobi_svd(D.stream, dj.as<SvdJob>(), (int)jobs.size(), nmax, mmax);
+    std::vector<double> h(ns);
+    KV_HIP(hipMemcpyAsync(h.data(), S.get(), ns * sizeof(double), hipMemcpyDeviceToHost, D.stream));
+    D.sync();
+    for (size_t i = 0; i < xs.size(); ++i) {
+        SectorSvd& X = *xs[i];
+        X.s.assign(h.begin() + soff[i], h.begin() + soff[i] + X.k);
+        for (double v : X.s) KV_REQUIRE(std::isfinite(v) && v >= 0.0, ERR_SOLVER, "Problems in SVD (did not converge)");
+        if (keep_zero && X.s.back() <= 1e-60 * X.s.front()) exact_sector(D, sol, X, true);
+    }
 }
 
 // Gram matrix of a sector (G = M^H M when cols <= rows, else M M^H; the isometric route
@@ -767,7 +834,6 @@ inline void gram_vectors(Device& D, Solver& sol, SectorSvd& X, int nk) {
     std::vector<double> inv(nk);
     for (int j = 0; j < nk; ++j) inv[j] = X.s[j] > 0 ? 1.0 / X.s[j] : 0.0;
     DevBuf dinv = upload_vec(D, inv);
-    X.S = upload_vec(D, std::vector<double>(X.s.begin(), X.s.begin() + nk));
     // B2 = diag(1/s) B
     DevBuf B2(D.pool.get(), (size_t)nk * n * sizeof(double2));
     {
@@ -875,7 +941,6 @@ inline void iso_vectors(Device& D, Solver& sol, SectorSvd& X, int nk) {
                                nullptr);
     }
     X.s_absorbed = true;
-    X.S = upload_vec(D, std::vector<double>(X.s.begin(), X.s.begin() + nk));
     X.ldU = nk;
     X.U = DevBuf(D.pool.get(), (size_t)(X.nr * nk) * sizeof(double2));
     X.Vh = DevBuf(D.pool.get(), (size_t)(nk * X.nc) * sizeof(double2));
@@ -1318,7 +1383,6 @@ inline void block_ritz(Device& D, Solver& sol, std::vector<BlockJob*>& J, bool i
 inline void block_vectors(Device& D, SectorSvd& X, int nk) {
     const int kc = X.kc;
     X.s_absorbed = true;
-    X.S = upload_vec(D, std::vector<double>(X.s.begin(), X.s.begin() + nk));
     X.ldU = kc;
     X.Vh = DevBuf(D.pool.get(), (size_t)kc * X.nc * sizeof(double2));
     if (!X.colside) {  // U = Z (nr x kc); S V^H = W^H (kc x nc)
@@ -1338,6 +1402,7 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
     const int np = (int)S.pairs.size();
     std::vector<SectorSvd> X(np);
     SvdResult res;
+    std::vector<SectorSvd*> small;
     // full routes: the isometric-side Gram matrix when the isometry is the smaller side, the
     // smaller side's Gram matrix (guarded below) otherwise, the exact SVD for small sectors
     auto full_route = [&](int p) {
@@ -1348,8 +1413,14 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
             gram_prepare(D, X[p], true, !left2right);
         else if (big && cutoff >= 0.0)
             gram_prepare(D, X[p]);
+        else if (jacobi_takes(X[p].nr, X[p].nc, cutoff))
+            small.push_back(&X[p]);
         else
             exact_sector(D, sol, X[p], cutoff < 0.0);
+    };
+    auto small_sectors = [&] {  // those full_route has left to the batched exact route
+        jacobi_sectors(D, sol, small, cutoff < 0.0);
+        small.clear();
     };
     // the isometric Gram route on the longer side, Householder-reduced to the shorter one
     // when it is at least twice as long
@@ -1365,7 +1436,11 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
     const int bw = std::max(maxdim, std::min(maxdim + kBlockOversample, kBlockEigSmall));
     const bool block_ok = opt.block && !opt.force_exact && cutoff >= 0.0 && maxdim > 0 && bw <= kCholMax;
     std::vector<int> cand;
-    // phase 1: gather every sector matrix and compute its singular values
+    // phase 1: gather every sector matrix (one launch; offsets are measured from the lowest of
+    // their addresses) and compute its singular values
+    std::vector<Copy2D> gather;
+    int gather_rows = 1;
+    double2* M0 = nullptr;
     for (int p = 0; p < np; ++p) {
         const SvdSector& rs = S.rows[S.pairs[p].first];
         const SvdSector& cs = S.cols[S.pairs[p].second];
@@ -1373,9 +1448,12 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
         X[p].nc = cs.len;
         KV_REQUIRE(rs.len < (1 << 30) && cs.len < (1 << 30), ERR_ARG, "sector matrix too large");
         X[p].M = DevBuf(D.pool.get(), (size_t)(rs.len * cs.len) * sizeof(double2));
-        launch_zero(D.stream, X[p].M.get(), X[p].M.bytes());
-        std::vector<Copy2D> cps;
-        int maxrows = 1;
+        if (!M0 || X[p].M.as<double2>() < M0) M0 = X[p].M.as<double2>();
+    }
+    for (int p = 0; p < np; ++p) {
+        const SvdSector& rs = S.rows[S.pairs[p].first];
+        const SvdSector& cs = S.cols[S.pairs[p].second];
+        int64_t filled = 0;
         for (const auto& rsub : rs.subs)
             for (const auto& csub : cs.subs) {
                 Idx q{};
@@ -1385,25 +1463,31 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
                 if (bi < 0) continue;
                 Copy2D c{};
                 c.src_off = A.lay.blocks[bi].off;
-                c.dst_off = rsub.pos * cs.len + csub.pos;
+                c.dst_off = (X[p].M.as<double2>() - M0) + rsub.pos * cs.len + csub.pos;
                 c.rows = (int)rsub.size;
                 c.cols = (int)csub.size;
                 c.src_ld = (int)csub.size;
                 c.dst_ld = (int)cs.len;
-                maxrows = std::max(maxrows, c.rows);
-                cps.push_back(c);
+                gather_rows = std::max(gather_rows, c.rows);
+                filled += rsub.size * csub.size;
+                gather.push_back(c);
             }
-        if (!cps.empty()) {
-            DevBuf dc = upload_vec(D, cps);
-            launch_copy2d<double2>(D.stream, A.d(), X[p].M.as<double2>(), dc.as<Copy2D>(),
-                                   (int)cps.size(), maxrows, nullptr);
-        }
+        if (filled < rs.len * cs.len) launch_zero(D.stream, X[p].M.get(), X[p].M.bytes());
+    }
+    if (!gather.empty()) {
+        DevBuf dc = upload_vec(D, gather);
+        launch_copy2d<double2>(D.stream, A.d(), M0, dc.as<Copy2D>(), (int)gather.size(), gather_rows, nullptr);
+    }
+    for (int p = 0; p < np; ++p) {
+        const SvdSector& rs = S.rows[S.pairs[p].first];
+        const SvdSector& cs = S.cols[S.pairs[p].second];
         // sectors at least block_min (3) times as wide as the block take the block subspace route
         if (block_ok && (double)std::min(rs.len, cs.len) >= opt.block_min * bw)
             cand.push_back(p);
         else
             full_route(p);
     }
+    small_sectors();
     // the block route, all its sectors together: start block, one power step, Rayleigh-Ritz
     std::vector<BlockJob> jobs(cand.size());
     std::vector<int> job_of(np, -1);
@@ -1437,6 +1521,7 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
                 res.block_fallbacks += 1;
                 D.blk.fallbacks += 1;
             }
+        small_sectors();
     }
     // Gram eigenproblems: one call for all sectors (zheevd needs one side per call)
     {
@@ -1524,6 +1609,7 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
                     X[p].Z.reset();
                     X[p].W.reset();
                     full_route(p);
+                    small_sectors();
                     if (X[p].gram) gram_solve(D, sol, {&X[p]}, opt.eig_mode, opt.roc_trd);
                     if (X[p].iso) X[p].s.resize((size_t)std::min(X[p].nr, X[p].nc));
                     res.block_fallbacks += 1;
@@ -1605,27 +1691,37 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
     res.left = Tensor::create(dev, Ll, false);
     res.right = Tensor::create(dev, Rl, false);
     res.svals.resize(np);
+    // one launch for each factor; offsets are measured from the lowest of the sectors' buffers
+    std::vector<Copy2D> lc, rc;
+    std::vector<double> scale;
+    int maxr_l = 1, maxr_r = 1;
+    const double2 *U0 = nullptr, *V0 = nullptr;
+    for (int p = 0; p < np; ++p) {
+        if (kept[p] <= 0) continue;
+        if (!U0 || X[p].U.as<double2>() < U0) U0 = X[p].U.as<double2>();
+        if (!V0 || X[p].Vh.as<double2>() < V0) V0 = X[p].Vh.as<double2>();
+    }
     for (int p = 0; p < np; ++p) {
         if (kept[p] <= 0) continue;
         const SvdSector& rs = S.rows[S.pairs[p].first];
         const SvdSector& cs = S.cols[S.pairs[p].second];
         const int nk = kept[p];
         const int64_t nc = cs.len;
-        std::vector<Copy2D> lc, rc;
-        int maxr_l = 1, maxr_r = 1;
+        const int64_t u0 = X[p].U.as<double2>() - U0, v0 = X[p].Vh.as<double2>() - V0;
         for (const auto& rsub : rs.subs) {
             Idx q{};
             for (int l = 0; l < S.r1; ++l) q[l] = rsub.qn[l];
             q[S.r1] = -left_dir * rs.q;
             const int bi = Ll.find(q);
             Copy2D c{};
-            c.src_off = rsub.pos * (int64_t)X[p].ldU;  // U_M rows [pos, pos+size)
+            c.src_off = u0 + rsub.pos * (int64_t)X[p].ldU;  // U_M rows [pos, pos+size)
             c.dst_off = Ll.blocks[bi].off;
             c.rows = (int)rsub.size;
             c.cols = nk;
             c.src_ld = X[p].ldU;
             c.dst_ld = nk;
             c.scale_mode = (left2right || X[p].s_absorbed) ? 0 : 2;  // U S when S goes left
+            c.scale_off = (int)scale.size();
             maxr_l = std::max(maxr_l, c.rows);
             lc.push_back(c);
         }
@@ -1635,23 +1731,23 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
             for (int l = 0; l < S.r2; ++l) q[1 + l] = csub.qn[l];
             const int bi = Rl.find(q);
             Copy2D c{};
-            c.src_off = csub.pos;  // V_M^H rows [0, nk), cols [pos, pos+size), ld nc
+            c.src_off = v0 + csub.pos;  // V_M^H rows [0, nk), cols [pos, pos+size), ld nc
             c.dst_off = Rl.blocks[bi].off;
             c.rows = nk;
             c.cols = (int)csub.size;
             c.src_ld = (int)nc;
             c.dst_ld = (int)csub.size;
             c.scale_mode = (left2right && !X[p].s_absorbed) ? 1 : 0;  // S V^H when S goes right
+            c.scale_off = (int)scale.size();
             maxr_r = std::max(maxr_r, c.rows);
             rc.push_back(c);
         }
-        PackedUpload pk = upload_packed(D, lc, rc);
-        launch_copy2d<double2>(D.stream, X[p].U.as<double2>(), res.left->d(), pk.at<Copy2D>(0),
-                               (int)lc.size(), maxr_l, X[p].S.as<double>());
-        launch_copy2d<double2>(D.stream, X[p].Vh.as<double2>(), res.right->d(), pk.at<Copy2D>(1),
-                               (int)rc.size(), maxr_r, X[p].S.as<double>());
         res.svals[p].assign(X[p].s.begin(), X[p].s.begin() + nk);
+        scale.insert(scale.end(), res.svals[p].begin(), res.svals[p].end());
     }
+    PackedUpload pk = upload_packed(D, lc, rc, scale);
+    launch_copy2d<double2>(D.stream, U0, res.left->d(), pk.at<Copy2D>(0), (int)lc.size(), maxr_l, pk.at<double>(2));
+    launch_copy2d<double2>(D.stream, V0, res.right->d(), pk.at<Copy2D>(1), (int)rc.size(), maxr_r, pk.at<double>(2));
     return res;
 }
 

@@ -86,6 +86,21 @@ void launch_f64_to_f32(hipStream_t st, const double2* src, float2* dst, int64_t 
 void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n,
                        const int* stop = nullptr);
 
+// ---- SVD of small sectors ----------------------------------------------------------------
+constexpr int kJacobiMax = 64;  // largest smaller side
+// M (nr x nc, row-major) = U S Vh: U nr x k, Vh k x nc (row-major), S descending, k = min(nr, nc).
+// A and T: workspaces of nr x nc (T only where nr >= nc).  S is NaN where M holds a NaN or an
+// infinity and -1 where the rotations did not converge.  Vectors of zero singular values are
+// zero on the shorter side, except those of a zero matrix.
+struct SvdJob {
+    const double2* M;
+    double2 *U, *Vh, *A, *T;
+    double* S;
+    int nr, nc;
+};
+// nmax / mmax: the largest smaller / larger side of the jobs.
+void launch_jacobi_svd(hipStream_t st, const SvdJob* jobs, int njobs, int nmax, int mmax);
+
 // A[i ld + i] = (v, 0) for i in [from, to) (the diagonal of a square matrix).
 void launch_set_diag(hipStream_t st, double2* A, int64_t ld, int from, int to, double v);
 // dst (n x n, ld n) = the lower (j <= i) or upper (j >= i) triangle of src (ld lds), the rest zero.

@@ -87,3 +87,64 @@ def test_local_krylov_at_the_sizes_where_its_kernels_change(dl, p, dr, max_iter)
         # both sides: at most 15 Krylov vectors of rounding errors against a unit vector
         assert np.linalg.norm(g - w) < 1e-12
         assert ex["iters"] == info.iters and ex["converged"] == info.converged
+
+
+# the Jacobi route's row-count variants (64, 256, 512, more), square, wide and tall, one row or
+# column, odd widths, the widest it takes and the largest matrix; sectors share one launch
+SVD = [[(1, 1)], [(1, 9), (9, 1), (2, 3)], [(33, 32), (5, 64), (63, 64)], [(63, 63), (64, 17), (256, 31)],
+       [(1, 128), (200, 63), (256, 2)], [(257, 12), (40, 512)], [(513, 33), (3, 1500)], [(4161, 63)], [(63, 4161)]]
+SPECTRA = {"flat": lambda k: np.linspace(1.0, 0.5, k), "graded": lambda k: 10.0 ** -np.linspace(0, 14, k),
+           "repeated": lambda k: np.where(np.arange(k) < (k + 1) // 2, 1.0, 1e-3),
+           "deficient": lambda k: np.where(np.arange(k) < (k + 1) // 2, 1.0 / (1 + np.arange(k)), 0.0)}
+
+
+@pytest.mark.parametrize("shapes", SVD)
+@pytest.mark.parametrize("spectrum", [*SPECTRA, "copies"])
+@pytest.mark.parametrize("l2r", [True, False])
+def test_small_sectors_svd(shapes, spectrum, l2r):
+    kv = GE.load_package()
+    rng = np.random.default_rng([len(shapes), *shapes[0]])
+    print(f"case svd {shapes} {spectrum} l2r {l2r}", flush=True)
+
+    def unitary(m, k):
+        return np.linalg.qr(cplx(rng, m, k))[0]
+
+    blocks = {}
+    for q, (m, n) in enumerate(shapes):
+        k = min(m, n)
+        if spectrum == "copies":  # equal rows and columns, many of them zero
+            a = cplx(rng, m, n)
+            a[k // 2:], a[:, k // 3 + 1:] = 0, a[:, :1]
+            blocks[(q, q)] = a
+            continue
+        blocks[(q, q)] = (unitary(m, k) * SPECTRA[spectrum](k)) @ unitary(n, k).conj().T
+    t = kv.Tensor.from_blocks((1, -1), blocks)
+    # with a truncating cutoff the route starts at a longer side of 128
+    cutoffs = [-1.0] if min(map(max, shapes)) < 128 else [1e-13 if spectrum in ("deficient", "copies") else 0.0, -1.0]
+    for cutoff in cutoffs:
+        left, right = kv.svd_impl(t, 1, cutoff, 10 ** 6, l2r)
+        L, R = left.to_blocks()[1], right.to_blocks()[1]
+        for q, (m, n) in enumerate(shapes):
+            M = blocks[(q, q)]
+            if (q, q) not in L:  # nothing of the sector is above the cutoff
+                assert np.linalg.norm(M, 2) <= 1e-13
+                continue
+            u, v = L[(q, q)], R[(q, q)]
+            iso = u.conj().T @ u if l2r else v @ v.conj().T
+            k = min(m, n)
+            assert cutoff >= 0 or iso.shape == (k, k)
+            # k rotations or reflections over a side of max(m, n), a few roundings each
+            tol = 40 * EPS * np.sqrt(k * max(m, n))
+            assert np.abs(iso - np.eye(len(iso))).max() < tol
+            assert np.linalg.norm(u @ v - M) <= tol * np.linalg.norm(M) + (cutoff if cutoff > 0 else 0) * k
+            s = np.sort(np.linalg.norm(v, axis=1) if l2r else np.linalg.norm(u, axis=0))[::-1]
+            want = np.linalg.svd(M, compute_uv=False)[:len(s)]
+            assert np.abs(s - want).max() <= tol * want[0]
+
+
+def test_svd_of_a_non_finite_sector_is_refused():
+    kv = GE.load_package()
+    m = np.ones((128, 3), complex)
+    m[2, 1] = np.nan
+    with pytest.raises(kv.KVError):
+        kv.svd_impl(kv.Tensor.from_blocks((1, -1), {(0, 0): m}), 1, 1e-10, 10, True)
