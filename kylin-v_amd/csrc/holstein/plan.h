@@ -348,6 +348,36 @@ inline WFoldPlan plan_wfold(const Layout& X, int p, const Layout& W, const doubl
         out.finalize();
     }
     std::vector<char> covered(out.blocks.size(), 0);
+    // nonzero entries of each W block by (s', wR) row, in the order (wL, s)
+    struct Nz {
+        int wl, s;
+        double re, im;
+    };
+    struct Rows {
+        std::vector<int> begin;
+        std::vector<Nz> nz;
+    };
+    std::vector<Rows> wrows(W.blocks.size());
+    auto rows_of = [&](int j) -> const Rows& {
+        Rows& R = wrows[j];
+        if (!R.begin.empty()) return R;
+        const BlockDesc& wb = W.blocks[j];
+        const int WR = wb.shape[3];
+        const int64_t per = (int64_t)wb.shape[1] * wb.shape[2] * WR;
+        R.begin.assign((size_t)wb.shape[0] * WR + 1, 0);
+        const double* d = Wd + 2 * wb.off;
+        for (int64_t e = 0; e < wb.size; ++e)
+            if (d[2 * e] != 0.0 || d[2 * e + 1] != 0.0) R.begin[(e / per) * WR + e % WR + 1] += 1;
+        for (size_t r = 1; r < R.begin.size(); ++r) R.begin[r] += R.begin[r - 1];
+        R.nz.resize(R.begin.back());
+        std::vector<int> at(R.begin.begin(), R.begin.end() - 1);
+        for (int64_t e = 0; e < wb.size; ++e)
+            if (d[2 * e] != 0.0 || d[2 * e + 1] != 0.0) {
+                const int64_t in = e % per / WR;
+                R.nz[at[(e / per) * WR + e % WR]++] = Nz{(int)(in / wb.shape[2]), (int)(in % wb.shape[2]), d[2 * e], d[2 * e + 1]};
+            }
+        return R;
+    };
     for (auto& kvp : groups) {
         Idx q{};
         for (int r = 0; r < out.rank; ++r) q[r] = kvp.first[r];
@@ -373,23 +403,20 @@ inline WFoldPlan plan_wfold(const Layout& X, int p, const Layout& W, const doubl
                 t.term_begin = (int)F.terms.size();
                 for (auto& pr : kvp.second.pairs) {
                     const BlockDesc& xb = X.blocks[pr.first];
-                    const BlockDesc& wb = W.blocks[pr.second];
                     const int WL = xb.shape[p], S = xb.shape[p + 1];
-                    for (int wl = 0; wl < WL; ++wl)
-                        for (int s = 0; s < S; ++s) {
-                            const int64_t e =
-                                wb.off + (((int64_t)sp * WL + wl) * S + s) * WR + wr;
-                            const double re = Wd[2 * e], im = Wd[2 * e + 1];
-                            if (re == 0.0 && im == 0.0) continue;
-                            WTerm w{};
-                            w.in_base = xb.off + ((int64_t)wl * S + s) * Qd;
-                            w.in_pstride = (int64_t)WL * S * Qd;
-                            w.re = re;
-                            w.im = im;
-                            F.terms.push_back(w);
-                            F.term_src.push_back({pr.first, wl, s});
-                            F.flop += 8.0 * (double)Pd * (double)Qd;
-                        }
+                    const Rows& R = rows_of(pr.second);
+                    const int row = sp * WR + wr;
+                    for (int e = R.begin[row]; e < R.begin[row + 1]; ++e) {
+                        const Nz& z = R.nz[e];
+                        WTerm w{};
+                        w.in_base = xb.off + ((int64_t)z.wl * S + z.s) * Qd;
+                        w.in_pstride = (int64_t)WL * S * Qd;
+                        w.re = z.re;
+                        w.im = z.im;
+                        F.terms.push_back(w);
+                        F.term_src.push_back({pr.first, z.wl, z.s});
+                        F.flop += 8.0 * (double)Pd * (double)Qd;
+                    }
                 }
                 t.term_count = (int)F.terms.size() - t.term_begin;
                 F.tasks.push_back(t);
@@ -422,64 +449,93 @@ inline WFoldPlan plan_wfold(const Layout& X, int p, const Layout& W, const doubl
 //                                  sum_{wL, s1} W1[s1', wL, s1, w1] X[pre, wL, s1, s2, post],
 // one task per (F2 task, s1') over P = pre, Q = post, with a term per pair of nonzero W
 // entries (weight W2 W1, X's slice of F1's term shifted to s2).  Z's layout is F2's.
-inline WFoldPlan compose_wfold(const WFoldPlan& F1, const WFoldPlan& F2, const Layout& Y) {
+// Only the two folds' own lists are built here: at 64 levels the composite has 49k tasks of
+// 231k terms, which took 15 to 20 ms to list on the host and 10 MB to upload; a kernel expands
+// them (wcompose_expand) in 9 us.
+struct ComposePlan {
+    std::vector<WComposeTask> tasks;   // one per F2 task
+    std::vector<WComposeTerm> terms;   // one per F2 term
+    int ntasks = 0;                    // composite tasks and term slots
+    int64_t nterms = 0;
+    int64_t maxPQ = 0;
+    double flop = 0;
+};
+
+inline ComposePlan plan_compose(const WFoldPlan& F1, const WFoldPlan& F2, const Layout& Y) {
     KV_REQUIRE(F1.term_src.size() == F1.terms.size() && F2.term_src.size() == F2.terms.size() &&
                    F1.task_src.size() == F1.tasks.size() && F2.task_src.size() == F2.tasks.size(),
-               ERR_INTERNAL, "compose_wfold: plans without provenance");
-    WFoldPlan C;
-    C.out = F2.out;
-    // F1's task writing Y block yb at (s1', w1)
-    std::map<std::array<int, 3>, int> f1_task;
-    for (size_t t = 0; t < F1.tasks.size(); ++t)
-        if (F1.task_src[t][0] >= 0) f1_task[F1.task_src[t]] = (int)t;
+               ERR_INTERNAL, "plan_compose: plans without provenance");
+    ComposePlan C;
+    // F1's first task writing Y block yb (its tasks follow in the order s1', w1)
+    std::vector<int> first(Y.blocks.size(), -1);
+    for (size_t t = F1.tasks.size(); t-- > 0;)
+        if (F1.task_src[t][0] >= 0) first[F1.task_src[t][0]] = (int)t;
+    C.terms.reserve(F2.terms.size());
     for (size_t t2 = 0; t2 < F2.tasks.size(); ++t2) {
         const WTask& T2 = F2.tasks[t2];
+        WComposeTask c{};
+        c.out_base = T2.out_base;
+        c.Q = T2.Q;
+        c.task0 = C.ntasks;
+        c.slot = C.nterms;
+        c.term_begin = (int)C.terms.size();
         if (F2.task_src[t2][0] < 0) {  // an output block no term reaches: zeros
-            C.tasks.push_back(T2);
-            C.tasks.back().term_begin = (int)C.terms.size();
-            C.task_src.push_back({-1, -1, -1});
-            C.maxP = std::max(C.maxP, T2.P);
-            C.maxPQ = std::max<int64_t>(C.maxPQ, (int64_t)T2.P * T2.Q);
-            continue;
-        }
-        const BlockDesc& Ob = C.out.blocks[F2.task_src[t2][0]];
-        const int S1 = Ob.shape[1];  // s1' (F2's pre is (pre, s1'))
-        KV_REQUIRE(S1 > 0 && T2.P % S1 == 0, ERR_INTERNAL, "compose_wfold: pre does not end in s1'");
-        for (int s1 = 0; s1 < S1; ++s1) {
-            WTask t{};
-            t.out_base = T2.out_base + (int64_t)s1 * T2.out_pstride;
-            t.out_pstride = (int64_t)S1 * T2.out_pstride;
-            t.P = T2.P / S1;
-            t.Q = T2.Q;
-            t.term_begin = (int)C.terms.size();
+            c.out_pstride = T2.out_pstride;
+            c.P = T2.P;
+            c.S1 = 1;
+        } else {
+            const int S1 = F2.out.blocks[F2.task_src[t2][0]].shape[1];  // F2's pre is (pre, s1')
+            KV_REQUIRE(S1 > 0 && T2.P % S1 == 0, ERR_INTERNAL, "plan_compose: pre does not end in s1'");
+            c.out_pstride = (int64_t)S1 * T2.out_pstride;
+            c.s1_stride = T2.out_pstride;
+            c.P = T2.P / S1;
+            c.S1 = S1;
             for (int k2 = T2.term_begin; k2 < T2.term_begin + T2.term_count; ++k2) {
-                const WTerm& w2 = F2.terms[k2];
                 const auto& src = F2.term_src[k2];  // (Y block, w1, s2)
-                auto it = f1_task.find({src[0], s1, src[1]});
-                if (it == f1_task.end()) continue;  // that slice of Y is zero
-                const WTask& T1 = F1.tasks[it->second];
-                KV_REQUIRE(T1.P == t.P, ERR_INTERNAL, "compose_wfold: pre extents differ");
-                for (int k1 = T1.term_begin; k1 < T1.term_begin + T1.term_count; ++k1) {
-                    const WTerm& w1 = F1.terms[k1];
-                    WTerm w{};
-                    w.in_base = w1.in_base + (int64_t)src[2] * t.Q;
-                    w.in_pstride = w1.in_pstride;
-                    w.re = w2.re * w1.re - w2.im * w1.im;
-                    w.im = w2.re * w1.im + w2.im * w1.re;
-                    C.terms.push_back(w);
-                    C.term_src.push_back({-1, -1, -1});
-                    C.flop += 8.0 * (double)t.P * (double)t.Q;
-                }
+                WComposeTerm w{};
+                w.shift = (int64_t)src[2] * T2.Q;
+                w.re = F2.terms[k2].re;
+                w.im = F2.terms[k2].im;
+                w.f1_task = first[src[0]] < 0 ? -1 : first[src[0]] + src[1];
+                w.f1_stride = Y.blocks[src[0]].shape[2];
+                KV_REQUIRE(w.f1_task < 0 || F1.tasks[w.f1_task].P == c.P, ERR_INTERNAL,
+                           "plan_compose: pre extents differ");
+                C.terms.push_back(w);
             }
-            t.term_count = (int)C.terms.size() - t.term_begin;
-            C.tasks.push_back(t);
-            C.task_src.push_back({-1, -1, -1});
-            C.maxP = std::max(C.maxP, t.P);
-            C.maxPQ = std::max<int64_t>(C.maxPQ, (int64_t)t.P * t.Q);
+            c.term_count = (int)C.terms.size() - c.term_begin;
+            for (int s1 = 0; s1 < S1; ++s1) {
+                int nt = 0;
+                for (int k = c.term_begin; k < c.term_begin + c.term_count; ++k)
+                    if (C.terms[k].f1_task >= 0)
+                        nt += F1.tasks[C.terms[k].f1_task + s1 * C.terms[k].f1_stride].term_count;
+                c.maxt = std::max(c.maxt, nt);
+                C.flop += 8.0 * nt * (double)c.P * (double)c.Q;
+            }
         }
+        C.ntasks += c.S1;
+        C.nterms += (int64_t)c.S1 * c.maxt;
+        KV_REQUIRE(C.nterms < (1ll << 31), ERR_ARG, "MPO fold: too many terms");
+        C.maxPQ = std::max<int64_t>(C.maxPQ, (int64_t)c.P * c.Q);
+        C.tasks.push_back(c);
     }
-    (void)Y;
     return C;
+}
+
+// The composite's lists, expanded on the host.
+inline WFoldPlan compose_wfold(const WFoldPlan& F1, const WFoldPlan& F2, const Layout& Y) {
+    const ComposePlan C = plan_compose(F1, F2, Y);
+    WFoldPlan W;
+    W.out = F2.out;
+    W.tasks.resize(C.ntasks);
+    W.terms.resize(C.nterms);
+    W.maxPQ = C.maxPQ;
+    W.flop = C.flop;
+    for (const auto& c : C.tasks) {
+        W.maxP = std::max(W.maxP, c.P);
+        for (int s1 = 0; s1 < c.S1; ++s1)
+            wcompose_expand(c, s1, C.terms.data(), F1.tasks.data(), F1.terms.data(), W.tasks.data(), W.terms.data());
+    }
+    return W;
 }
 
 struct PermPlan {
@@ -559,13 +615,13 @@ struct HeffStructure {
     Layout xl;
     ProductPlan s1, s4;
     WFoldPlan s2, s3;
-    WFoldPlan s23;  // two sites: both folds as one pass (compose_wfold)
+    WFoldPlan s23;  // two sites, where asked for: both folds as one pass, expanded on the host
     double flop = 0;
 };
 
 inline HeffStructure plan_heff(int nsite, const Layout& L, const Layout* W1, const double* W1d,
                                const Layout* W2, const double* W2d, const Layout& R,
-                               const Layout& x) {
+                               const Layout& x, bool composite = true) {
     KV_REQUIRE(nsite >= 0 && nsite <= 2, ERR_ARG, "nsite must be 0, 1 or 2");
     KV_REQUIRE(x.rank == nsite + 2, ERR_ARG, "x rank does not match nsite");
     HeffStructure H;
@@ -591,7 +647,7 @@ inline HeffStructure plan_heff(int nsite, const Layout& L, const Layout* W1, con
     const Layout* t = nsite == 2 ? &H.s3.out : (nsite == 1 ? &H.s2.out : &H.s1.out);
     H.s4 = plan_product(*t, R, 2, 'N', 'T', &cur);
     H.xl = cur;
-    if (nsite == 2) H.s23 = compose_wfold(H.s2, H.s3, H.s2.out);
+    if (nsite == 2 && composite) H.s23 = compose_wfold(H.s2, H.s3, H.s2.out);
     H.flop = H.s1.flop + H.s2.flop + H.s3.flop + H.s4.flop;
     return H;
 }

@@ -271,6 +271,39 @@ struct DevWFold {
     }
 };
 
+// The two folds of a two-site H_eff as one pass, its tasks expanded on the device.
+struct DevCompose {
+    int ntasks = 0;
+    int64_t maxPQ = 0;
+    double flop = 0;
+    DevBuf tasks, terms;
+    void build(Device& dev, const DevWFold& f1, const DevWFold& f2) {
+        const ComposePlan C = plan_compose(f1.p, f2.p, f1.p.out);
+        ntasks = C.ntasks;
+        maxPQ = C.maxPQ;
+        flop = C.flop;
+        tasks = DevBuf(dev.pool.get(), (size_t)C.ntasks * sizeof(WTask));
+        terms = DevBuf(dev.pool.get(), (size_t)C.nterms * sizeof(WTerm));
+        const PackedUpload pk = upload_packed(dev, C.tasks, C.terms);
+        launch_wcompose(dev.stream, pk.at<WComposeTask>(0), (int)C.tasks.size(), pk.at<WComposeTerm>(1),
+                        f1.lists.at<WTask>(0), f1.lists.at<WTerm>(1), tasks.as<WTask>(), terms.as<WTerm>());
+    }
+    template <class T2>
+    void run(Device& dev, const T2* in, T2* out, EventLog* log, const int* stop) const {
+        hipEvent_t a = nullptr, b = nullptr;
+        if (log) {
+            a = log->get();
+            b = log->get();
+            KV_HIP(hipEventRecord(a, dev.stream));
+        }
+        launch_wfold<T2>(dev.stream, in, out, tasks.as<WTask>(), ntasks, terms.as<WTerm>(), maxPQ, stop);
+        if (log) {
+            KV_HIP(hipEventRecord(b, dev.stream));
+            log->pending.push_back({a, b, flop, 1, 0.0});
+        }
+    }
+};
+
 // product<N1,N2,nc>(m1, m2, T1, T2) on the device, FP64 (holstein/product.h:61-201).
 inline std::unique_ptr<Tensor> product(const std::shared_ptr<Device>& dev, const Tensor& A,
                                        const Tensor& B, int nc, char opA, char opB) {
@@ -346,7 +379,8 @@ struct Heff {
     Prec prec = PREC_F64;
     DevProduct s1, s4;
     // the MPO folds; two sites in FP32 / split-BF16 also both folds as one pass (s23)
-    DevWFold s2, s3, s23;
+    DevWFold s2, s3;
+    DevCompose s23;
     const Tensor* L = nullptr;
     const Tensor* R = nullptr;
     DevBuf L32, R32, x32, y32, t1, t2, t3;
@@ -360,11 +394,11 @@ struct Heff {
         const double* w1d = W1 ? W1->host_data().data() : nullptr;
         const double* w2d = W2 ? W2->host_data().data() : nullptr;
         S = plan_heff(nsite, Lt.lay, W1 ? &W1->lay : nullptr, w1d, W2 ? &W2->lay : nullptr, w2d,
-                      Rt.lay, x);
+                      Rt.lay, x, false);
         s1.build(*dev, S.s1);
         if (nsite >= 1) s2.build(*dev, S.s2);
         if (nsite == 2) s3.build(*dev, S.s3);
-        if (nsite == 2 && p != PREC_F64) s23.build(*dev, S.s23);
+        if (nsite == 2 && p != PREC_F64) s23.build(*dev, s2, s3);
         s4.build(*dev, S.s4);
         // intermediates sized for FP64 so either precision can run through them
         const size_t es = sizeof(double2);

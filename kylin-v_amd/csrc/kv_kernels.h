@@ -32,6 +32,10 @@ template <class T2>
 void launch_wfold(hipStream_t st, const T2* in, T2* out, const WTask* tasks, int ntasks,
                   const WTerm* terms, int64_t maxPQ, const int* stop = nullptr);
 
+// Expands the composite of two folds (wcompose_expand for every task and s1').
+void launch_wcompose(hipStream_t st, const WComposeTask* tasks2, int n2, const WComposeTerm* terms2,
+                     const WTask* tasks1, const WTerm* terms1, WTask* tasks, WTerm* terms);
+
 template <class T2>
 void launch_perm(hipStream_t st, const T2* in, T2* out, const PermTask* tasks, int ntasks,
                  int64_t maxsize);

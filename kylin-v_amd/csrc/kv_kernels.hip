@@ -782,6 +782,22 @@ template void launch_wfold<double2>(hipStream_t, const double2*, double2*, const
 template void launch_wfold<float2>(hipStream_t, const float2*, float2*, const WTask*, int,
                                    const WTerm*, int64_t, const int*);
 
+__global__ __launch_bounds__(64) void wcompose_kernel(const WComposeTask* __restrict__ tasks2,
+                                                      const WComposeTerm* __restrict__ terms2,
+                                                      const WTask* __restrict__ tasks1,
+                                                      const WTerm* __restrict__ terms1, WTask* __restrict__ tasks,
+                                                      WTerm* __restrict__ terms) {
+    const WComposeTask c = tasks2[blockIdx.x];
+    for (int s1 = threadIdx.x; s1 < c.S1; s1 += 64) wcompose_expand(c, s1, terms2, tasks1, terms1, tasks, terms);
+}
+
+void launch_wcompose(hipStream_t st, const WComposeTask* tasks2, int n2, const WComposeTerm* terms2,
+                     const WTask* tasks1, const WTerm* terms1, WTask* tasks, WTerm* terms) {
+    if (n2 <= 0) return;
+    hipLaunchKernelGGL(wcompose_kernel, dim3(n2), dim3(64), 0, st, tasks2, terms2, tasks1, terms1, tasks, terms);
+    KV_HIP(hipGetLastError());
+}
+
 // ------------------------------------------------------------------------------------
 // block permutation
 // ------------------------------------------------------------------------------------

@@ -47,6 +47,54 @@ struct WTask {
     int P, Q, term_begin, term_count;
 };
 
+// ---- two MPO folds as one: tasks expanded from the two folds' own lists ------------------
+// A task of the second fold stands for S1 composite tasks (one per s1' of the first), whose
+// terms are its own terms times those of the first fold's task that wrote the slice they read.
+struct WComposeTask {
+    int64_t out_base, out_pstride, s1_stride;  // of s1' = 0; out_base grows by s1_stride per s1'
+    int64_t slot;                              // composite terms of s1' start at slot + s1' * maxt
+    int P, Q, S1, task0;                       // composite tasks task0 .. task0 + S1 - 1
+    int term_begin, term_count, maxt, pad;     // terms of the second fold
+};
+struct WComposeTerm {
+    int64_t shift;  // added to the first fold's in_base
+    double re, im;
+    int f1_task, f1_stride;  // the first fold's task of s1' = 0 (-1: that slice is zero), per s1'
+};
+
+#ifdef __HIPCC__
+#define KV_HD __host__ __device__
+#else
+#define KV_HD
+#endif
+// Composite task s1 of c into tasks[c.task0 + s1] and its terms.
+KV_HD inline void wcompose_expand(const WComposeTask& c, int s1, const WComposeTerm* terms2, const WTask* tasks1,
+                                  const WTerm* terms1, WTask* tasks, WTerm* terms) {
+    WTask t;
+    t.out_base = c.out_base + (int64_t)s1 * c.s1_stride;
+    t.out_pstride = c.out_pstride;
+    t.P = c.P;
+    t.Q = c.Q;
+    int64_t at = c.slot + (int64_t)s1 * c.maxt;
+    t.term_begin = (int)at;
+    for (int k2 = c.term_begin; k2 < c.term_begin + c.term_count; ++k2) {
+        const WComposeTerm w2 = terms2[k2];
+        if (w2.f1_task < 0) continue;
+        const WTask t1 = tasks1[w2.f1_task + s1 * w2.f1_stride];
+        for (int k1 = t1.term_begin; k1 < t1.term_begin + t1.term_count; ++k1) {
+            const WTerm w1 = terms1[k1];
+            WTerm w;
+            w.in_base = w1.in_base + w2.shift;
+            w.in_pstride = w1.in_pstride;
+            w.re = w2.re * w1.re - w2.im * w1.im;
+            w.im = w2.re * w1.im + w2.im * w1.re;
+            terms[at++] = w;
+        }
+    }
+    t.term_count = (int)(at - t.term_begin);
+    tasks[c.task0 + s1] = t;
+}
+
 // ---- block permutation (tensor transpose) ----------------------------------------------
 constexpr int PERM_MAXR = 6;
 struct PermTask {
