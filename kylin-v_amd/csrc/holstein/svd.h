@@ -103,14 +103,11 @@ struct SvdResult {
     std::string detail;  // per sector: rows x cols, route, s_max, last kept value
 };
 
-// Side from which the split eigensolver replaces zheevd by default.  Below it the
-// back-transformation of all vectors inside zheevd is cheap, and the split route's extra
-// launches and host synchronisations cost more than they save: with the split route at
-// every side, 8 concurrent chains of the batching workload ran 7% slower.  From 512 up the
-// split route wins: rocSOLVER's column-by-column reduction dominates zheevd there (the
-// 32-site chain's edge bonds, 512-wide Gram matrices, and the batching chains' largest
-// sectors).
-constexpr int kSplitEigMin = 512;
+// Side from which the split eigensolver replaces zheevd by default.  With the reflectors
+// applied in one launch it is the faster one from 128 up, alone and with eight contexts at once
+// (a bond of two n x 2n sectors, ms, against zheevd: n = 80 1.82 / 1.85, 128 2.82 / 3.39,
+// 256 6.3 / 8.0, 500 11.9 / 14.7; eight at once, n = 128 10.1 / 10.8, 256 13.9 / 18.4).
+constexpr int kSplitEigMin = 128;
 // The side from which the split route is taken (KV_SPLIT_MIN overrides kSplitEigMin).
 inline int split_eig_min() {
     static const int v = [] {
@@ -688,6 +685,7 @@ inline void gram_solve(Device& D, Solver& sol, std::vector<SectorSvd*> xs, int m
 // eigenvectors Zt[:, lo:k] carried back through the reflectors, Z <- Q Z with
 // Q = H_0 H_1 ... H_{n-2}, applied block by block from the last one:
 // Z <- Z - V_b (T_b (V_b^H Z)) = Z - P_b Y_b,  Y_b = V_b^H Z,  P_b = V_b T_b.
+// Sides up to kHhApplyMax: one launch that applies the reflectors one by one (launch_hh_apply).
 // Column-major throughout (the rocBLAS layout); V_b and P_b are zero above row b*bw + 1.
 // S_b = V_b^H V_b and Y_b have few outputs (bw x bw, bw x k) over up to n rows, so both run
 // split over row chunks on the grouped GEMM (one group per block and chunk, partial
@@ -703,6 +701,12 @@ inline void gram_eigvecs(Device& D, Solver& sol, SectorSvd& X, int lo, hipStream
     KV_REQUIRE(X.Zt.get() != nullptr, ERR_INTERNAL, "Gram eigenvectors requested before the eigensolver");
     const int k = n - lo;
     DevBuf Z(D.pool.get(), (size_t)n * k * sizeof(double2));
+    if (n <= kHhApplyMax) {
+        launch_hh_apply(st, X.G.as<double2>(), X.tau.as<double2>(), X.Zt.as<double>(), n, lo, k, Z.as<double2>());
+        X.Ev = std::move(Z);
+        X.ev_lo = lo;
+        return;
+    }
     launch_real_cols(st, X.Zt.as<double>(), n, lo, k, n, Z.as<double2>());
     const int nref = n - 1;
     if (nref > 0 && k > 0) {

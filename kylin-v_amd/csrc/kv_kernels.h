@@ -112,6 +112,11 @@ void launch_tri_copy(hipStream_t st, const double2* src, int64_t lds, double2* d
 
 // Back-transformation of a lower-triangle Householder tridiagonalisation (LAPACK layout:
 // reflector i stored below the subdiagonal of column i, tau_i separately).
+// Sides up to kHhApplyMax in one launch: Z = Q C(:, c0 : c0 + k), C real (ld n), Z complex (ld n).
+constexpr int kHhApplyMax = 512;
+void launch_hh_apply(hipStream_t st, const double2* A, const double2* tau, const double* C, int n, int c0, int k,
+                     double2* Z);
+// Larger sides in blocks of reflectors.
 // V (column-major n x ncols): the reflector vectors written out with their unit entries.
 void launch_hh_explicit(hipStream_t st, const double2* A, double2* V, int n, int ncols);
 // T (bw x bw per block, column-major, upper; bw <= 128): triangular factor of reflectors

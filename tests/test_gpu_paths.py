@@ -148,3 +148,35 @@ def test_svd_of_a_non_finite_sector_is_refused():
     m[2, 1] = np.nan
     with pytest.raises(kv.KVError):
         kv.svd_impl(kv.Tensor.from_blocks((1, -1), {(0, 0): m}), 1, 1e-10, 10, True)
+
+
+# sides of the eigenvectors' back-transformation: its variants' limits (64, 128, 256, 512) and
+# one more, kept counts that its columns per wave do not divide, sectors of different sides
+GRAM = [([64], 63), ([65, 65], 130), ([127], 31), ([128, 129], 100), ([256], 255), ([257, 70], 33), ([511], 7), ([513], 200)]
+
+
+@pytest.mark.parametrize("sides,keep", GRAM)
+@pytest.mark.parametrize("l2r", [True, False])
+def test_gram_sectors_svd(sides, keep, l2r, monkeypatch):
+    monkeypatch.setenv("KV_SVD", "full")  # not the block subspace route
+    kv = GE.load_package()
+    rng = np.random.default_rng(sides)
+    print(f"case gram svd {sides} keep {keep} l2r {l2r}", flush=True)
+    blocks = {}
+    for q, n in enumerate(sides):
+        u, v = np.linalg.qr(cplx(rng, n, n))[0], np.linalg.qr(cplx(rng, n + 5, n))[0]
+        m = (u * 10.0 ** (-2.0 * (np.arange(n) + 0.1 * q) / n)) @ v.conj().T
+        blocks[(q, q)] = m if l2r else m.conj().T
+    left, right = kv.svd_impl(kv.Tensor.from_blocks((1, -1), blocks), 1, 1e-10, keep, l2r)
+    L, R = left.to_blocks()[1], right.to_blocks()[1]
+    assert sum(b.shape[1] for b in L.values()) == min(keep, sum(sides))
+    for q, n in enumerate(sides):
+        u, v = L[(q, q)], R[(q, q)]
+        k = u.shape[1]
+        U, s, V = np.linalg.svd(blocks[(q, q)], full_matrices=False)
+        iso = u.conj().T @ u if l2r else v @ v.conj().T
+        # n reflectors and as many merges of orthonormal bases, a few roundings each; the kept
+        # subspace turns by the Gram matrix's rounding over the gap of its values at the cut
+        assert np.abs(iso - np.eye(k)).max() < 16 * n * EPS
+        gap = s[k - 1] ** 2 - (s[k] ** 2 if k < n else 0.0)
+        assert np.linalg.norm(u @ v - (U[:, :k] * s[:k]) @ V[:k]) < 64 * n * EPS / gap
