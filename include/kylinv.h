@@ -107,7 +107,7 @@ int kv_product(kv_ctx* ctx, const kv_tensor* m1, const kv_tensor* m2, int nc,
                char op1, char op2, int precision, kv_tensor** out);
 
 /* Profiling form of kv_heff_apply: builds H_eff once, applies it once untimed (tile
- * autotuning), then `reps` times timed by HIP events on the context stream.
+ * autotuning), then `reps` times timed on the device.
  * out[8] = {seconds per apply, algorithmic flop per apply, GEMM kernel seconds per apply,
  * GEMM flop per apply, GEMM launches per apply, MPO-fold seconds per apply, MPO-fold flop
  * per apply, MPO-fold launches per apply}.  No reference counterpart (the reference's
@@ -235,7 +235,7 @@ int kv_tdvp_get_site(kv_tdvp* s, int i, kv_tensor** out);
 int kv_tdvp_bond_dims(kv_tdvp* s, int* dims);
 /* Per-module timing in seconds, names of the reference's Timer modules
  * (holstein/tdvp.h:85-214): "Evl-2","Evl-1","Evl-0","SVD","Update","Sweep", plus
- * GPU time (HIP events on the context stream) and algorithmic flops of the H_eff matvec
+ * GPU time (the device clock at the start of successive launches) and algorithmic flops of the H_eff matvec
  * kernels and of the environment-update kernels.  Writes up to n values in this order:
  *   0 Evl-2  1 Evl-1  2 Evl-0  3 SVD  4 Update  5 Sweep  (wall seconds)
  *   6 heff_gpu_s  7 heff_flop  8 env_gpu_s  9 env_flop  10 matvecs

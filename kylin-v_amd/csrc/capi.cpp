@@ -384,11 +384,14 @@ int kv_heff_profile(kv_ctx* ctx, int nsite, const kv_tensor* L, const kv_tensor*
         auto y = kv::Tensor::create(ctx->dev, H.layout(), false);
         H.apply(xin->d(), y->d(), 1.0);  // first call: GEMM tile autotuning, not timed
         ctx->dev->sync();
-        kv::EventLog log;
+        kv::MarkLog log(*ctx->dev);
         kv::KernelStats st;
         kv::EventTimer ev;
         ev.start(ctx->dev->stream);
-        for (int r = 0; r < reps; ++r) H.apply(xin->d(), y->d(), 1.0, &log);
+        for (int r = 0; r < reps; ++r) {
+            H.apply(xin->d(), y->d(), 1.0, &log);
+            if (kv::Mark* done = log.end()) kv::launch_mark(ctx->dev->stream, done);
+        }
         ev.stop(ctx->dev->stream);
         const double wall_ms = ev.ms();
         ctx->dev->sync();
@@ -471,6 +474,7 @@ int kv_tdvp_create(kv_ctx* ctx, int nsites, kv_tensor* const* mps, kv_tensor* co
         h->ctx = ctx;
         try {
             h->s.reset(new kv::TDVP(ctx->dev, std::move(a), std::move(w), c));
+            ctx->dev->sync();
         } catch (...) {
             delete h;
             throw;
@@ -487,12 +491,18 @@ int kv_tdvp_destroy(kv_tdvp* s) {
 
 int kv_tdvp_two_site(kv_tdvp* s) {
     if (!s || !s->s) return KV_ERR_ARG;
-    return guard(s->ctx, [&] { s->s->two_site(); });
+    return guard(s->ctx, [&] {
+        s->s->two_site();
+        s->ctx->dev->sync();
+    });
 }
 
 int kv_tdvp_one_site(kv_tdvp* s) {
     if (!s || !s->s) return KV_ERR_ARG;
-    return guard(s->ctx, [&] { s->s->one_site(); });
+    return guard(s->ctx, [&] {
+        s->s->one_site();
+        s->ctx->dev->sync();
+    });
 }
 
 int kv_tdvp_get_site(kv_tdvp* s, int i, kv_tensor** out) {
@@ -512,6 +522,7 @@ int kv_tdvp_sa_one_site(kv_tdvp* s, const double* betas, int nbetas, uint64_t se
         std::vector<double> b(betas, betas + nbetas);
         for (double x : b) KV_REQUIRE(std::isfinite(x) && x > 0.0, kv::ERR_ARG, "SA-1TDVP: bad inverse width");
         s->s->one_site(&b, seed);
+        s->ctx->dev->sync();
     });
 }
 
@@ -545,6 +556,7 @@ int kv_tdvp_global_krylov(kv_tdvp* s, int* iterations) {
     if (!s || !s->s) return KV_ERR_ARG;
     return guard(s->ctx, [&] {
         kv::GlobalKrylovExit ex = s->s->global_krylov();
+        s->ctx->dev->sync();
         if (iterations) *iterations = ex.iterations;
     });
 }

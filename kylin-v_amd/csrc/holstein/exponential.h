@@ -37,7 +37,7 @@ struct LanczosStats {
 inline KrylovExit local_krylov(const std::shared_ptr<Device>& dev, int nsite, const Tensor& L,
                                Tensor* W1, Tensor* W2, const Tensor& R,
                                std::unique_ptr<Tensor>& x, double dt, double tol, int max_iter,
-                               bool reverse, Prec prec, EventLog* log = nullptr,
+                               bool reverse, Prec prec, MarkLog* log = nullptr,
                                LanczosStats* stats = nullptr, KernelStats* kstats = nullptr) {
     Heff H;
     H.build(dev, nsite, L, W1, W2, R, x->lay, prec);
@@ -70,7 +70,7 @@ inline KrylovExit local_krylov(const std::shared_ptr<Device>& dev, int nsite, co
         double2* vk = Vb + (int64_t)k * n;
         H.apply(vk, h, dt * 0.5, log, k == 0, &D.lanczos_dev->stop[k]);
         launch_lanczos_step(D.stream, h, vk - n, vk, vk + n, n, part.as<double>(), D.lanczos_dev, k, tol, rec + k,
-                            tag | (uint64_t)k);
+                            tag | (uint64_t)k, log ? log->end() : nullptr);
     };
     std::vector<std::complex<double>> alp, bet_up;
     double err = 1.0;
@@ -79,7 +79,7 @@ inline KrylovExit local_krylov(const std::shared_ptr<Device>& dev, int nsite, co
     if (last >= 0 && err > tol) {
         queue(0);
         for (int k = 0;; ++k) {
-            const size_t logged = log ? log->pending.size() : 0;
+            const size_t logged = log ? log->size() : 0;
             if (k < last) queue(k + 1);
             D.wait_record(rec[k], tag | (uint64_t)k);
             if (stats) {

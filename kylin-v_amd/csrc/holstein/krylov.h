@@ -180,9 +180,13 @@ inline void canonicalize(const std::shared_ptr<Device>& dev, Solver& sol, State&
 inline std::unique_ptr<Tensor> env_mps_mpo(const std::shared_ptr<Device>& dev, const Tensor& L,
                                            const Tensor& A, Tensor& W) {
     DevProduct s1;
-    s1.build(*dev, plan_product(L.lay, A.lay, 1, 'N', 'N'));
+    StagedLists lists;
+    s1.stage(*dev, plan_product(L.lay, A.lay, 1, 'N', 'N'), lists);
     DevWFold s2;
-    s2.build(*dev, plan_wfold(s1.p.out, 1, W.lay, W.host_data().data()));
+    s2.stage(plan_wfold(s1.p.out, 1, W.lay, W.host_data().data()), lists);
+    lists.commit(*dev);
+    s1.bind(lists);
+    s2.bind(lists);
     DevBuf t1(dev->pool.get(), (size_t)s1.p.out.total * sizeof(double2));
     auto out = Tensor::create(dev, s2.p.out, false);
     s1.run<double2>(*dev, L.d(), A.d(), t1.as<double2>());
@@ -304,10 +308,16 @@ inline std::unique_ptr<Tensor> heff2(const std::shared_ptr<Device>& dev, const T
                                      Tensor* W2, const Tensor& R, const Tensor& x) {
     DevProduct s1, s4;
     DevWFold s2, s3;
-    s1.build(*dev, plan_product(L.lay, x.lay, 1, 'N', 'N'));
-    s2.build(*dev, plan_wfold(s1.p.out, 1, W1->lay, W1->host_data().data()));
-    s3.build(*dev, plan_wfold(s2.p.out, 2, W2->lay, W2->host_data().data()));
-    s4.build(*dev, plan_product(s3.p.out, R.lay, 2, 'N', 'T'));
+    StagedLists lists;
+    s1.stage(*dev, plan_product(L.lay, x.lay, 1, 'N', 'N'), lists);
+    s2.stage(plan_wfold(s1.p.out, 1, W1->lay, W1->host_data().data()), lists);
+    s3.stage(plan_wfold(s2.p.out, 2, W2->lay, W2->host_data().data()), lists);
+    s4.stage(*dev, plan_product(s3.p.out, R.lay, 2, 'N', 'T'), lists);
+    lists.commit(*dev);
+    s1.bind(lists);
+    s2.bind(lists);
+    s3.bind(lists);
+    s4.bind(lists);
     DevBuf t1(dev->pool.get(), (size_t)s1.p.out.total * sizeof(double2));
     DevBuf t2(dev->pool.get(), (size_t)s2.p.out.total * sizeof(double2));
     DevBuf t3(dev->pool.get(), (size_t)s3.p.out.total * sizeof(double2));

@@ -16,68 +16,84 @@ namespace kv {
 // PREC_BF16X3: FP32 storage, GEMMs as split-BF16 products with FP32 accumulation
 enum Prec { PREC_F64 = 0, PREC_F32 = 1, PREC_BF16X3 = 2 };
 
-// Event pairs recorded around contraction kernels; resolved after the host has
-// synchronised the stream anyway (no extra syncs on the hot path).
-struct EventLog {
-    struct Rec {
-        hipEvent_t a, b;
-        double flop;
-        int kind;      // 0 gemm (FP64 operands), 1 wfold, 2 gemm (FP32 operands)
-        double bytes;  // algorithmic bytes: operands and result once each
-    };
-    std::vector<Rec> pending;
-    std::vector<hipEvent_t> spare;
-    hipEvent_t get() {
-        if (!spare.empty()) {
-            hipEvent_t e = spare.back();
-            spare.pop_back();
-            return e;
-        }
-        hipEvent_t e;
-        KV_HIP(hipEventCreate(&e));
-        return e;
+// Times of the contraction launches, from the device's wall clock: a launch is marked as it
+// starts and ends where the next mark stands (kv_kernels.h); resolved after the host has
+// synchronised the stream anyway.  Events around each launch were packets of their own between
+// the kernels and several host calls a launch: a third of a step of small tensors.
+class MarkLog {
+  public:
+    explicit MarkLog(Device& dev) : dev_(dev) {
+        int khz = 0;
+        KV_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev.id));
+        ms_per_tick_ = 1.0 / (double)(khz > 0 ? khz : 100000);
     }
+    MarkLog(const MarkLog&) = delete;
+    MarkLog& operator=(const MarkLog&) = delete;
+    ~MarkLog() {
+        dev_.mark_chunks.insert(dev_.mark_chunks.end(), chunks_.begin(), chunks_.end());
+    }
+    // The mark of a launch of this kind: 0 gemm (FP64 operands), 1 wfold, 2 gemm (FP32 operands);
+    // bytes: operands and result once each.
+    Mark* begin(int kind, double flop, double bytes) {
+        Mark* m = slot();
+        pending_.push_back({m, flop, bytes, kind});
+        return m;
+    }
+    // The mark that ends the last launch (nothing, where none has begun since the last end).
+    Mark* end() {
+        if (pending_.empty() || pending_.back().kind < 0) return nullptr;
+        Mark* m = slot();
+        pending_.push_back({m, 0.0, 0.0, -1});
+        return m;
+    }
+    size_t size() const { return pending_.size(); }
+    // forgets the records from the n-th on (launches that found their iteration stopped)
+    void drop(size_t n) { pending_.resize(n); }
     // call only after the stream has been synchronised
     void resolve(KernelStats& st) {
-        for (auto& r : pending) {
-            float ms = 0;
-            KV_HIP(hipEventElapsedTime(&ms, r.a, r.b));
-            if (r.kind == 0 || r.kind == 2) {
-                st.gemm_ms += ms;
-                st.gemm_flop += r.flop;
-                st.gemm_bytes += r.bytes;
-                if (r.kind == 2) {
-                    st.gemm32_ms += ms;
-                    st.gemm32_flop += r.flop;
-                    st.gemm32_bytes += r.bytes;
-                    st.gemm32_launches += 1;
-                }
-                st.gemm_launches += 1;
-            } else {
+        for (size_t i = 0; i + 1 < pending_.size(); ++i) {
+            const Rec& r = pending_[i];
+            if (r.kind < 0) continue;
+            const double ms = ms_per_tick_ * (double)(*pending_[i + 1].at - *r.at);
+            if (r.kind == 1) {
                 st.wfold_ms += ms;
                 st.wfold_flop += r.flop;
                 st.wfold_launches += 1;
+                continue;
             }
-            spare.push_back(r.a);
-            spare.push_back(r.b);
+            st.gemm_ms += ms;
+            st.gemm_flop += r.flop;
+            st.gemm_bytes += r.bytes;
+            st.gemm_launches += 1;
+            if (r.kind == 2) {
+                st.gemm32_ms += ms;
+                st.gemm32_flop += r.flop;
+                st.gemm32_bytes += r.bytes;
+                st.gemm32_launches += 1;
+            }
         }
-        pending.clear();
+        pending_.clear();
+        used_ = 0;
     }
-    // forgets the records from the n-th on (launches that found their iteration stopped)
-    void drop(size_t n) {
-        while (pending.size() > n) {
-            spare.push_back(pending.back().a);
-            spare.push_back(pending.back().b);
-            pending.pop_back();
-        }
+
+  private:
+    struct Rec {
+        Mark* at;
+        double flop, bytes;
+        int kind;  // -1: an end
+    };
+    static constexpr size_t kChunk = Device::kMarkChunk;
+    Mark* slot() {
+        if (used_ == chunks_.size() * kChunk) chunks_.push_back(dev_.mark_chunk());
+        Mark* m = chunks_[used_ / kChunk] + used_ % kChunk;
+        ++used_;
+        return m;
     }
-    ~EventLog() {
-        for (auto& r : pending) {
-            (void)hipEventDestroy(r.a);
-            (void)hipEventDestroy(r.b);
-        }
-        for (auto e : spare) (void)hipEventDestroy(e);
-    }
+    Device& dev_;
+    std::vector<Mark*> chunks_;
+    size_t used_ = 0;
+    std::vector<Rec> pending_;
+    double ms_per_tick_ = 1e-5;
 };
 
 // Shape class of a product plan for the tile autotuner: log2 buckets of the m, n and total
@@ -107,27 +123,37 @@ inline uint64_t gemm_shape_key(const ProductPlan& p, int prec) {
 
 struct DevProduct {
     ProductPlan p;
-    PackedUpload lists;  // groups, segments and config 0's tiles, one upload
-    DevBuf tiles[kNumGemmConfigs];  // other configs' tiles, cut on first use
+    const GemmGroup* groups = nullptr;  // in the lists the plan was staged with
+    const GemmSeg* segs = nullptr;
+    DevBuf tiles[kNumGemmConfigs];  // other configs' tiles than 0, cut on first use
     const GemmTile* tp[kNumGemmConfigs] = {nullptr};
     int ntiles[kNumGemmConfigs] = {0};
     bool cut[kNumGemmConfigs] = {false};
     int nch = 1;   // K chunks (split_chunks): above 1 the lists are split_k's
     DevBuf part;   // and the chunks' partial results go here, one after the other
-    void build(Device& dev, ProductPlan plan) {
+    size_t off[3] = {0, 0, 0};
+    // the plan's groups, segments and config 0's tiles into L; bind() after L's commit
+    void stage(Device& dev, ProductPlan plan, StagedLists& L) {
         p = std::move(plan);
         nch = split_chunks(p);
+        auto put = [&](const auto& lists) {
+            off[0] = L.stage(lists.groups);
+            off[1] = L.stage(lists.segs);
+            off[2] = L.stage(lists.tiles);
+            ntiles[0] = (int)lists.tiles.size();
+        };
         if (nch > 1) {
-            const SplitK sk = split_k(p, nch);
             part = DevBuf(dev.pool.get(), (size_t)nch * p.out.total * sizeof(double2));
-            lists = upload_packed(dev, sk.groups, sk.segs, sk.tiles);
-            ntiles[0] = (int)sk.tiles.size();
+            put(split_k(p, nch));
         } else {
-            lists = upload_packed(dev, p.groups, p.segs, p.tiles);
-            ntiles[0] = (int)p.tiles.size();
+            put(p);
         }
-        tp[0] = lists.at<GemmTile>(2);
         cut[0] = true;
+    }
+    void bind(const StagedLists& L) {
+        groups = L.at<GemmGroup>(off[0]);
+        segs = L.at<GemmSeg>(off[1]);
+        tp[0] = L.at<GemmTile>(off[2]);
     }
     void ensure_tiles(Device& dev, int cfg) {
         if (cut[cfg]) return;
@@ -139,10 +165,10 @@ struct DevProduct {
     }
     template <class T2>
     void launch(Device& dev, int cfg, const T2* A, const T2* B, T2* C, double ar, double ai,
-                const int* stop = nullptr) {
+                const int* stop = nullptr, Mark* mark = nullptr) {
         ensure_tiles(dev, cfg);
         launch_gemm<T2>(dev.stream, p.opA, p.opB, A, B, nch > 1 ? part.as<T2>() : C, tp[cfg], ntiles[cfg],
-                        lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg, stop);
+                        groups, segs, ar, ai, cfg, stop, mark);
         if (nch > 1) launch_sum_parts<T2>(dev.stream, part.as<T2>(), nch, p.out.total, C, stop);
     }
     // Tile config for this plan: cached per shape class; on a first encounter every config
@@ -183,10 +209,10 @@ struct DevProduct {
         return best;
     }
     void launch_split(Device& dev, int cfg, const float2* A, const float2* B, float2* C, double ar,
-                      double ai, const int* stop = nullptr) {
+                      double ai, const int* stop = nullptr, Mark* mark = nullptr) {
         ensure_tiles(dev, cfg);
         launch_gemm_bf16x3(dev.stream, p.opA, p.opB, A, B, nch > 1 ? part.as<float2>() : C, tp[cfg], ntiles[cfg],
-                           lists.at<GemmGroup>(0), lists.at<GemmSeg>(1), ar, ai, cfg, stop);
+                           groups, segs, ar, ai, cfg, stop, mark);
         if (nch > 1) launch_sum_parts<float2>(dev.stream, part.as<float2>(), nch, p.out.total, C, stop);
     }
     // Split-BF16 tile (64x64 or 128x128), timed once per shape class like choose().
@@ -216,7 +242,7 @@ struct DevProduct {
     }
     template <class T2>
     void run(Device& dev, const T2* A, const T2* B, T2* C, double alpha_re = 1.0,
-             double alpha_im = 0.0, EventLog* log = nullptr, bool split = false, const int* stop = nullptr) {
+             double alpha_im = 0.0, MarkLog* log = nullptr, bool split = false, const int* stop = nullptr) {
         int cfg = 0;
         if constexpr (std::is_same<T2, float2>::value) {
             cfg = split ? choose_split(dev, A, B, C, alpha_re, alpha_im)
@@ -224,50 +250,39 @@ struct DevProduct {
         } else {
             cfg = choose<T2>(dev, A, B, C, alpha_re, alpha_im);
         }
-        hipEvent_t a = nullptr, b = nullptr;
-        if (log) {
-            a = log->get();
-            b = log->get();
-            KV_HIP(hipEventRecord(a, dev.stream));
-        }
+        Mark* mark = nullptr;
+        if (log && !p.tiles.empty())
+            mark = log->begin(sizeof(T2) == sizeof(float2) ? 2 : 0, p.flop, p.unique * (double)sizeof(T2));
         if constexpr (std::is_same<T2, float2>::value) {
             if (split)
-                launch_split(dev, cfg, A, B, C, alpha_re, alpha_im, stop);
+                launch_split(dev, cfg, A, B, C, alpha_re, alpha_im, stop, mark);
             else
-                launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im, stop);
+                launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im, stop, mark);
         } else {
             KV_REQUIRE(!split, ERR_INTERNAL, "split-BF16 GEMM takes FP32 operands");
-            launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im, stop);
-        }
-        if (log) {
-            KV_HIP(hipEventRecord(b, dev.stream));
-            log->pending.push_back({a, b, p.flop, sizeof(T2) == sizeof(float2) ? 2 : 0,
-                                    p.unique * (double)sizeof(T2)});
+            launch<T2>(dev, cfg, A, B, C, alpha_re, alpha_im, stop, mark);
         }
     }
 };
 
 struct DevWFold {
     WFoldPlan p;
-    PackedUpload lists;  // tasks and terms, one upload
-    void build(Device& dev, WFoldPlan plan) {
+    const WTask* tasks = nullptr;  // in the lists the plan was staged with
+    const WTerm* terms = nullptr;
+    size_t off[2] = {0, 0};
+    void stage(WFoldPlan plan, StagedLists& L) {
         p = std::move(plan);
-        lists = upload_packed(dev, p.tasks, p.terms);
+        off[0] = L.stage(p.tasks);
+        off[1] = L.stage(p.terms);
+    }
+    void bind(const StagedLists& L) {
+        tasks = L.at<WTask>(off[0]);
+        terms = L.at<WTerm>(off[1]);
     }
     template <class T2>
-    void run(Device& dev, const T2* in, T2* out, EventLog* log = nullptr, const int* stop = nullptr) const {
-        hipEvent_t a = nullptr, b = nullptr;
-        if (log) {
-            a = log->get();
-            b = log->get();
-            KV_HIP(hipEventRecord(a, dev.stream));
-        }
-        launch_wfold<T2>(dev.stream, in, out, lists.at<WTask>(0), (int)p.tasks.size(),
-                         lists.at<WTerm>(1), p.maxPQ, stop);
-        if (log) {
-            KV_HIP(hipEventRecord(b, dev.stream));
-            log->pending.push_back({a, b, p.flop, 1, 0.0});
-        }
+    void run(Device& dev, const T2* in, T2* out, MarkLog* log = nullptr, const int* stop = nullptr) const {
+        Mark* mark = log && !p.tasks.empty() ? log->begin(1, p.flop, 0.0) : nullptr;
+        launch_wfold<T2>(dev.stream, in, out, tasks, (int)p.tasks.size(), terms, p.maxPQ, stop, mark);
     }
 };
 
@@ -277,30 +292,28 @@ struct DevCompose {
     int64_t maxPQ = 0;
     double flop = 0;
     DevBuf tasks, terms;
-    void build(Device& dev, const DevWFold& f1, const DevWFold& f2) {
+    int ntasks2 = 0;
+    size_t off[2] = {0, 0};
+    void stage(Device& dev, const DevWFold& f1, const DevWFold& f2, StagedLists& L) {
         const ComposePlan C = plan_compose(f1.p, f2.p, f1.p.out);
         ntasks = C.ntasks;
+        ntasks2 = (int)C.tasks.size();
         maxPQ = C.maxPQ;
         flop = C.flop;
         tasks = DevBuf(dev.pool.get(), (size_t)C.ntasks * sizeof(WTask));
         terms = DevBuf(dev.pool.get(), (size_t)C.nterms * sizeof(WTerm));
-        const PackedUpload pk = upload_packed(dev, C.tasks, C.terms);
-        launch_wcompose(dev.stream, pk.at<WComposeTask>(0), (int)C.tasks.size(), pk.at<WComposeTerm>(1),
-                        f1.lists.at<WTask>(0), f1.lists.at<WTerm>(1), tasks.as<WTask>(), terms.as<WTerm>());
+        off[0] = L.stage(C.tasks);
+        off[1] = L.stage(C.terms);
+    }
+    // after L's commit and f1's bind
+    void expand(Device& dev, const DevWFold& f1, const StagedLists& L) {
+        launch_wcompose(dev.stream, L.at<WComposeTask>(off[0]), ntasks2, L.at<WComposeTerm>(off[1]), f1.tasks,
+                        f1.terms, tasks.as<WTask>(), terms.as<WTerm>());
     }
     template <class T2>
-    void run(Device& dev, const T2* in, T2* out, EventLog* log, const int* stop) const {
-        hipEvent_t a = nullptr, b = nullptr;
-        if (log) {
-            a = log->get();
-            b = log->get();
-            KV_HIP(hipEventRecord(a, dev.stream));
-        }
-        launch_wfold<T2>(dev.stream, in, out, tasks.as<WTask>(), ntasks, terms.as<WTerm>(), maxPQ, stop);
-        if (log) {
-            KV_HIP(hipEventRecord(b, dev.stream));
-            log->pending.push_back({a, b, flop, 1, 0.0});
-        }
+    void run(Device& dev, const T2* in, T2* out, MarkLog* log, const int* stop) const {
+        Mark* mark = log && ntasks > 0 ? log->begin(1, flop, 0.0) : nullptr;
+        launch_wfold<T2>(dev.stream, in, out, tasks.as<WTask>(), ntasks, terms.as<WTerm>(), maxPQ, stop, mark);
     }
 };
 
@@ -308,7 +321,10 @@ struct DevCompose {
 inline std::unique_ptr<Tensor> product(const std::shared_ptr<Device>& dev, const Tensor& A,
                                        const Tensor& B, int nc, char opA, char opB) {
     DevProduct dp;
-    dp.build(*dev, plan_product(A.lay, B.lay, nc, opA, opB));
+    StagedLists L;
+    dp.stage(*dev, plan_product(A.lay, B.lay, nc, opA, opB), L);
+    L.commit(*dev);
+    dp.bind(L);
     auto C = Tensor::create(dev, dp.p.out, false);
     dp.run<double2>(*dev, A.d(), B.d(), C->d());
     return C;
@@ -377,6 +393,7 @@ struct Heff {
     std::shared_ptr<Device> dev;
     HeffStructure S;
     Prec prec = PREC_F64;
+    StagedLists lists;
     DevProduct s1, s4;
     // the MPO folds; two sites in FP32 / split-BF16 also both folds as one pass (s23)
     DevWFold s2, s3;
@@ -395,11 +412,18 @@ struct Heff {
         const double* w2d = W2 ? W2->host_data().data() : nullptr;
         S = plan_heff(nsite, Lt.lay, W1 ? &W1->lay : nullptr, w1d, W2 ? &W2->lay : nullptr, w2d,
                       Rt.lay, x, false);
-        s1.build(*dev, S.s1);
-        if (nsite >= 1) s2.build(*dev, S.s2);
-        if (nsite == 2) s3.build(*dev, S.s3);
-        if (nsite == 2 && p != PREC_F64) s23.build(*dev, s2, s3);
-        s4.build(*dev, S.s4);
+        const bool one_pass = nsite == 2 && p != PREC_F64;
+        s1.stage(*dev, S.s1, lists);
+        if (nsite >= 1) s2.stage(S.s2, lists);
+        if (nsite == 2) s3.stage(S.s3, lists);
+        if (one_pass) s23.stage(*dev, s2, s3, lists);
+        s4.stage(*dev, S.s4, lists);
+        lists.commit(*dev);  // one upload for the launches of every stage
+        s1.bind(lists);
+        if (nsite >= 1) s2.bind(lists);
+        if (nsite == 2) s3.bind(lists);
+        if (one_pass) s23.expand(*dev, s2, lists);
+        s4.bind(lists);
         // intermediates sized for FP64 so either precision can run through them
         const size_t es = sizeof(double2);
         t1 = DevBuf(dev->pool.get(), (size_t)S.s1.out.total * es);
@@ -418,7 +442,7 @@ struct Heff {
     double flop() const { return S.flop; }
 
     template <class T2>
-    void chain(const T2* Ld, const T2* Rd, const T2* x, T2* y, double alpha, EventLog* log,
+    void chain(const T2* Ld, const T2* Rd, const T2* x, T2* y, double alpha, MarkLog* log,
                bool split = false, const int* stop = nullptr) {
         s1.run<T2>(*dev, Ld, x, t1.as<T2>(), 1.0, 0.0, log, split, stop);
         const T2* last = t1.as<T2>();
@@ -442,8 +466,9 @@ struct Heff {
         s4.run<T2>(*dev, last, Rd, y, alpha, 0.0, log, split, stop);
     }
     // y = alpha * H_eff x, x and y FP64 slabs in layout() order; force64 runs the
-    // contractions in FP64 whatever the plan's precision; stop: see kv_kernels.h
-    void apply(const double2* x, double2* y, double alpha, EventLog* log = nullptr,
+    // contractions in FP64 whatever the plan's precision; stop: see kv_kernels.h.  The caller marks
+    // the end of the last launch (log->end())
+    void apply(const double2* x, double2* y, double alpha, MarkLog* log = nullptr,
                bool force64 = false, const int* stop = nullptr) {
         if (prec == PREC_F64 || force64) {
             chain<double2>(L->d(), R->d(), x, y, alpha, log, false, stop);
@@ -451,17 +476,18 @@ struct Heff {
             launch_f64_to_f32(dev->stream, x, x32.as<float2>(), S.xl.total, stop);
             chain<float2>(L32.as<float2>(), R32.as<float2>(), x32.as<float2>(), y32.as<float2>(),
                           1.0, log, prec == PREC_BF16X3, stop);
-            launch_f32_to_f64(dev->stream, y32.as<float2>(), y, alpha, S.xl.total, stop);
+            launch_f32_to_f64(dev->stream, y32.as<float2>(), y, alpha, S.xl.total, stop, log ? log->end() : nullptr);
         }
     }
 };
 
 // env_sweep (holstein/product.h:488-521): L2R  L' = bra^dag . (L . ket . W);
-// R2L: the same after transposing bra/ket (2,1,0) and W (0,3,2,1).
+// R2L: the same after transposing bra/ket (2,1,0) and W (0,3,2,1).  One upload carries the lists
+// of every launch.  Without `wait` the result is ready in stream order.
 inline std::unique_ptr<Tensor> env_update(const std::shared_ptr<Device>& dev, const Tensor& env,
                                           const Tensor* bra, Tensor& W, const Tensor& ket,
-                                          bool l2r, Prec prec, EventLog* log = nullptr,
-                                          double* flop = nullptr) {
+                                          bool l2r, Prec prec, MarkLog* log = nullptr,
+                                          double* flop = nullptr, bool wait = true) {
     std::unique_ptr<Tensor> kt, bt;
     const Tensor* k = &ket;
     const Tensor* b = bra ? bra : &ket;
@@ -469,12 +495,19 @@ inline std::unique_ptr<Tensor> env_update(const std::shared_ptr<Device>& dev, co
     std::vector<double> wt;
     const Layout* wlay = &W.lay;
     const double* wd = W.host_data().data();
+    StagedLists L;
+    PermPlan pk, pb;
+    size_t pk_off = 0, pb_off = 0;
     if (!l2r) {
         const Idx ax{2, 1, 0, 0, 0, 0};
-        kt = transpose(dev, ket, ax);
+        pk = plan_perm(ket.lay, ax);
+        pk_off = L.stage(pk.tasks);
+        kt = Tensor::create(dev, pk.out, false);
         k = kt.get();
         if (bra) {
-            bt = transpose(dev, *bra, ax);
+            pb = plan_perm(bra->lay, ax);
+            pb_off = L.stage(pb.tasks);
+            bt = Tensor::create(dev, pb.out, false);
             b = bt.get();
         } else {
             b = k;
@@ -487,33 +520,45 @@ inline std::unique_ptr<Tensor> env_update(const std::shared_ptr<Device>& dev, co
     if (flop) *flop += E.flop;
     DevProduct s1, s3;
     DevWFold s2;
-    s1.build(*dev, E.s1);
-    s2.build(*dev, E.s2);
-    s3.build(*dev, E.s3);
+    const size_t n1 = (size_t)E.s1.out.total, n2 = (size_t)E.s2.out.total;
+    const int64_t n3 = E.s3.out.total;
     auto out = Tensor::create(dev, E.s3.out, false);
+    s1.stage(*dev, std::move(E.s1), L);
+    s2.stage(std::move(E.s2), L);
+    s3.stage(*dev, std::move(E.s3), L);
+    L.commit(*dev);
+    s1.bind(L);
+    s2.bind(L);
+    s3.bind(L);
+    if (kt)
+        launch_perm<double2>(dev->stream, ket.d(), kt->d(), L.at<PermTask>(pk_off), (int)pk.tasks.size(), pk.maxsize);
+    if (bt)
+        launch_perm<double2>(dev->stream, bra->d(), bt->d(), L.at<PermTask>(pb_off), (int)pb.tasks.size(),
+                             pb.maxsize);
     if (prec == PREC_F64) {
-        DevBuf t1(dev->pool.get(), (size_t)E.s1.out.total * sizeof(double2));
-        DevBuf t2(dev->pool.get(), (size_t)E.s2.out.total * sizeof(double2));
+        DevBuf t1(dev->pool.get(), n1 * sizeof(double2));
+        DevBuf t2(dev->pool.get(), n2 * sizeof(double2));
         s1.run<double2>(*dev, env.d(), k->d(), t1.as<double2>(), 1.0, 0.0, log);
         s2.run<double2>(*dev, t1.as<double2>(), t2.as<double2>(), log);
         s3.run<double2>(*dev, b->d(), t2.as<double2>(), out->d(), 1.0, 0.0, log);
-        dev->sync();
     } else {
         DevBuf e32(dev->pool.get(), (size_t)env.lay.total * sizeof(float2));
         DevBuf k32(dev->pool.get(), (size_t)k->lay.total * sizeof(float2));
         DevBuf b32(dev->pool.get(), (size_t)b->lay.total * sizeof(float2));
-        DevBuf o32(dev->pool.get(), (size_t)E.s3.out.total * sizeof(float2));
-        DevBuf t1(dev->pool.get(), (size_t)E.s1.out.total * sizeof(float2));
-        DevBuf t2(dev->pool.get(), (size_t)E.s2.out.total * sizeof(float2));
+        DevBuf o32(dev->pool.get(), (size_t)n3 * sizeof(float2));
+        DevBuf t1(dev->pool.get(), n1 * sizeof(float2));
+        DevBuf t2(dev->pool.get(), n2 * sizeof(float2));
         launch_f64_to_f32(dev->stream, env.d(), e32.as<float2>(), env.lay.total);
         launch_f64_to_f32(dev->stream, k->d(), k32.as<float2>(), k->lay.total);
         launch_f64_to_f32(dev->stream, b->d(), b32.as<float2>(), b->lay.total);
         s1.run<float2>(*dev, e32.as<float2>(), k32.as<float2>(), t1.as<float2>(), 1.0, 0.0, log);
         s2.run<float2>(*dev, t1.as<float2>(), t2.as<float2>(), log);
         s3.run<float2>(*dev, b32.as<float2>(), t2.as<float2>(), o32.as<float2>(), 1.0, 0.0, log);
-        launch_f32_to_f64(dev->stream, o32.as<float2>(), out->d(), 1.0, E.s3.out.total);
-        dev->sync();
+        launch_f32_to_f64(dev->stream, o32.as<float2>(), out->d(), 1.0, n3);
     }
+    Mark* done = log ? log->end() : nullptr;
+    if (done) launch_mark(dev->stream, done);
+    if (wait) dev->sync();
     return out;
 }
 

@@ -239,10 +239,15 @@ class TDVP {
     const TdvpTimers& timers() const { return tm_; }
     const LanczosStats& lanczos_stats() const { return ls_; }
     const KernelStats& heff_kernels() const { return heff_k_; }
-    const KernelStats& env_kernels() const { return env_k_; }
+    const KernelStats& env_kernels() {
+        dev_->sync();
+        env_log_.resolve(env_k_);
+        return env_k_;
+    }
     double env_flop() const { return env_flop_; }
     Device& device() { return *dev_; }
     void reset_stats() {
+        (void)env_kernels();
         tm_ = TdvpTimers();
         ls_ = LanczosStats();
         env_flop_ = 0;
@@ -278,15 +283,14 @@ class TDVP {
     // their rounding error would bias the effective Hamiltonian itself (they cost ~5% of
     // the H_eff work).
     std::unique_ptr<Tensor> update(const Tensor& env, const Tensor& A, Tensor& W, bool l2r) {
-        auto out = env_update(dev_, env, nullptr, W, A, l2r, PREC_F64, timing ? &log_ : nullptr,
-                              &env_flop_);
-        if (timing) log_.resolve(env_k_);
-        return out;
+        return env_update(dev_, env, nullptr, W, A, l2r, PREC_F64, timing ? &env_log_ : nullptr, &env_flop_,
+                          false);
     }
     void krylov(int nsite, std::unique_ptr<Tensor>& x, Tensor* W1, Tensor* W2, bool reverse) {
         KrylovExit ex = local_krylov(dev_, nsite, *envL_.back(), W1, W2, *envR_.back(), x, cfg_.dt,
                                      cfg_.krylov_tol, cfg_.krylov_maxiter, reverse, cfg_.prec,
                                      timing ? &log_ : nullptr, &ls_, &heff_k_);
+        env_log_.resolve(env_k_);  // the step has waited for the stream
         last_iters_ = ex.iterations;
     }
 
@@ -297,7 +301,7 @@ class TDVP {
     TdvpConfig cfg_;
     TdvpTimers tm_;
     LanczosStats ls_;
-    EventLog log_;
+    MarkLog log_{*dev_}, env_log_{*dev_};
     KernelStats heff_k_, env_k_;
     double env_flop_ = 0;
     bool verbose_ = false;
@@ -324,7 +328,7 @@ inline std::complex<double> join(const std::shared_ptr<Device>& dev, std::vector
                                  const std::vector<const Tensor*>& ket) {
     auto env = left_boundary(dev);
     for (size_t i = 0; i < mpo.size(); ++i)
-        env = env_update(dev, *env, bra[i], *mpo[i], *ket[i], true, PREC_F64);
+        env = env_update(dev, *env, bra[i], *mpo[i], *ket[i], true, PREC_F64, nullptr, nullptr, false);
     return closing_value(*env);
 }
 

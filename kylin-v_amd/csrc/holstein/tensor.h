@@ -80,6 +80,32 @@ inline DevBuf upload_vec(Device& dev, const std::vector<T>& v) {
     return b;
 }
 
+// Work lists of several launches gathered for one upload: stage() every array, commit() once,
+// then at() gives the device address of each.
+class StagedLists {
+  public:
+    template <class T>
+    size_t stage(const std::vector<T>& v) {
+        const size_t o = (host_.size() + 255) / 256 * 256;
+        host_.resize(o + v.size() * sizeof(T));
+        if (!v.empty()) std::memcpy(host_.data() + o, v.data(), v.size() * sizeof(T));
+        return o;
+    }
+    void commit(Device& dev) {
+        buf_ = DevBuf(dev.pool.get(), host_.size());
+        dev.upload(buf_.get(), host_.data(), host_.size());
+        std::vector<char>().swap(host_);
+    }
+    template <class T>
+    const T* at(size_t off) const {
+        return reinterpret_cast<const T*>(static_cast<const char*>(buf_.get()) + off);
+    }
+
+  private:
+    std::vector<char> host_;
+    DevBuf buf_;
+};
+
 // Several host arrays in one device buffer by one upload (each array 256-byte aligned),
 // so a launch's descriptor lists cost one copy instead of one each.
 struct PackedUpload {

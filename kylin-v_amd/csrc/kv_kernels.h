@@ -9,6 +9,10 @@
 
 namespace kv {
 
+// `mark` on a launch: where its first workgroup writes the device's wall clock as it starts (null:
+// nowhere).  Successive launches of a stream time each other this way with no packets of their own.
+typedef unsigned long long Mark;
+
 // `stop` on the launches of an H_eff matvec: a device word; the kernel does nothing when it is
 // set (the Lanczos iteration it belongs to comes after the one that converged).
 
@@ -17,7 +21,7 @@ template <class T2>
 void launch_gemm(hipStream_t st, int opA, int opB, const T2* A, const T2* B, T2* C,
                  const GemmTile* tiles, int ntiles, const GemmGroup* groups,
                  const GemmSeg* segs, double alpha_re, double alpha_im, int cfg = 0,
-                 const int* stop = nullptr);
+                 const int* stop = nullptr, Mark* mark = nullptr);
 // Tile configs built per op pair and precision (every config is free of register spills).
 bool gemm_config_supports(int cfg, int opA, int opB, bool fp64);
 // Split-BF16 variant on the tile list of config 0 (64x64) or 4 (128x128): FP32 complex
@@ -25,12 +29,12 @@ bool gemm_config_supports(int cfg, int opA, int opB, bool fp64);
 void launch_gemm_bf16x3(hipStream_t st, int opA, int opB, const float2* A, const float2* B,
                         float2* C, const GemmTile* tiles, int ntiles, const GemmGroup* groups,
                         const GemmSeg* segs, double alpha_re, double alpha_im, int cfg,
-                        const int* stop = nullptr);
+                        const int* stop = nullptr, Mark* mark = nullptr);
 
 // MPO fold; maxPQ = the largest task's P x Q (sets the workgroups per task).
 template <class T2>
 void launch_wfold(hipStream_t st, const T2* in, T2* out, const WTask* tasks, int ntasks,
-                  const WTerm* terms, int64_t maxPQ, const int* stop = nullptr);
+                  const WTerm* terms, int64_t maxPQ, const int* stop = nullptr, Mark* mark = nullptr);
 
 // Expands the composite of two folds (wcompose_expand for every task and s1').
 void launch_wcompose(hipStream_t st, const WComposeTask* tasks2, int n2, const WComposeTerm* terms2,
@@ -81,14 +85,16 @@ void launch_lanczos_begin(hipStream_t st, const double2* x, double2* v0, int64_t
 // h = H v_k -> beta (k > 0), alpha, |h|, v_{k+1} and the stop word of iteration k + 1: set when the
 // product of the residual norms is no longer above tol.  Does nothing when iteration k is stopped.
 void launch_lanczos_step(hipStream_t st, double2* h, const double2* vkm, const double2* vk, double2* vn, int64_t n,
-                         double* part, LanczosDev* dev, int k, double tol, LanczosHost* rec, uint64_t tag);
+                         double* part, LanczosDev* dev, int k, double tol, LanczosHost* rec, uint64_t tag,
+                         Mark* mark = nullptr);
 // out = sum_i c_i V_i (c on the host, nv <= kLanczosMax); |out|^2 to rec->nsq.
 void launch_lanczos_end(hipStream_t st, double2* out, const double2* V, const double2* c, int nv, int64_t n,
                         double* part, LanczosHost* rec, uint64_t tag);
 void launch_f64_to_f32(hipStream_t st, const double2* src, float2* dst, int64_t n, const int* stop = nullptr);
 // dst = s * src
 void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n,
-                       const int* stop = nullptr);
+                       const int* stop = nullptr, Mark* mark = nullptr);
+void launch_mark(hipStream_t st, Mark* mark);
 
 // ---- SVD of small sectors ----------------------------------------------------------------
 constexpr int kJacobiMax = 64;  // largest smaller side

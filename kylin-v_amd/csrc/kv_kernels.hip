@@ -21,6 +21,16 @@ namespace kv {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// The device's wall clock (100 MHz) at the start of a launch's first workgroup.
+__device__ inline void write_mark(Mark* mark) {
+    if (mark && (blockIdx.x | blockIdx.y | threadIdx.x) == 0) *mark = wall_clock64();
+}
+__global__ void mark_kernel(Mark* mark) { write_mark(mark); }
+void launch_mark(hipStream_t st, Mark* mark) {
+    hipLaunchKernelGGL(mark_kernel, dim3(1), dim3(1), 0, st, mark);
+    KV_HIP(hipGetLastError());
+}
+
 template <class T> struct Cx;
 template <> struct Cx<double> {
     using T2 = double2;
@@ -60,8 +70,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM * BN <= 
     const typename Cx<T>::T2* __restrict__ A, const typename Cx<T>::T2* __restrict__ B,
     typename Cx<T>::T2* __restrict__ C, const GemmTile* __restrict__ tiles,
     const GemmGroup* __restrict__ groups, const GemmSeg* __restrict__ segs, T alpha_re,
-    T alpha_im, const int* __restrict__ stop) {
+    T alpha_im, const int* __restrict__ stop, Mark* mark) {
     if (stop && *stop) return;
+    write_mark(mark);
     using T2 = typename Cx<T>::T2;
     using acc_t = typename Cx<T>::acc;
     constexpr int SI = BM / 32, SJ = BN / 32;  // 16x16 sub-tiles per wave
@@ -367,7 +378,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM * BN <= 
 template <class T2>
 void launch_gemm(hipStream_t st, int opA, int opB, const T2* A, const T2* B, T2* C,
                  const GemmTile* tiles, int ntiles, const GemmGroup* groups,
-                 const GemmSeg* segs, double alpha_re, double alpha_im, int cfg, const int* stop) {
+                 const GemmSeg* segs, double alpha_re, double alpha_im, int cfg, const int* stop,
+                 Mark* mark) {
     using T = typename ScalarOf<T2>::T;
     if (ntiles <= 0) return;
     const dim3 grid(ntiles), block(256);
@@ -375,7 +387,7 @@ void launch_gemm(hipStream_t st, int opA, int opB, const T2* A, const T2* B, T2*
 #define KV_GEMM_CASE(C_, OA, OB, BM_, BN_, BK_)                                                  \
     if (cfg == C_ && opA == OA && opB == OB) {                                                 \
         hipLaunchKernelGGL((zgemm_grouped_kernel<T, OA, OB, BM_, BN_, BK_>), grid, block, 0, st, \
-                           A, B, C, tiles, groups, segs, ar, ai, stop);                        \
+                           A, B, C, tiles, groups, segs, ar, ai, stop, mark);                  \
         KV_HIP(hipGetLastError());                                                             \
         return;                                                                                \
     }
@@ -421,10 +433,10 @@ bool gemm_config_supports(int cfg, int opA, int opB, bool fp64) {
 
 template void launch_gemm<double2>(hipStream_t, int, int, const double2*, const double2*,
                                    double2*, const GemmTile*, int, const GemmGroup*,
-                                   const GemmSeg*, double, double, int, const int*);
+                                   const GemmSeg*, double, double, int, const int*, Mark*);
 template void launch_gemm<float2>(hipStream_t, int, int, const float2*, const float2*,
                                   float2*, const GemmTile*, int, const GemmGroup*,
-                                  const GemmSeg*, double, double, int, const int*);
+                                  const GemmSeg*, double, double, int, const int*, Mark*);
 
 // ------------------------------------------------------------------------------------
 // grouped complex GEMM, split-BF16 (FP32 operands and accumulation)
@@ -460,8 +472,10 @@ template <int OPA, int OPB, int BM, int BN, int SI, int SJ>
 __global__ __launch_bounds__(64 * (BM / (16 * SI)) * (BN / (16 * SJ))) void zgemm_bf16x3_kernel(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C,
     const GemmTile* __restrict__ tiles, const GemmGroup* __restrict__ groups,
-    const GemmSeg* __restrict__ segs, float alpha_re, float alpha_im, const int* __restrict__ stop) {
+    const GemmSeg* __restrict__ segs, float alpha_re, float alpha_im, const int* __restrict__ stop,
+    Mark* mark) {
     if (stop && *stop) return;
+    write_mark(mark);
     constexpr int BK = 32, LDK = BK + 8;  // row pitch stays a multiple of 16 bytes
     constexpr int WN = BN / (16 * SJ), NT = 64 * (BM / (16 * SI)) * WN;
     __shared__ __attribute__((aligned(16))) __bf16 As[4][BM][LDK];
@@ -664,17 +678,18 @@ __global__ __launch_bounds__(64 * (BM / (16 * SI)) * (BN / (16 * SJ))) void zgem
 // the FP32 kernel's configs 0 and 4.
 void launch_gemm_bf16x3(hipStream_t st, int opA, int opB, const float2* A, const float2* B,
                         float2* C, const GemmTile* tiles, int ntiles, const GemmGroup* groups,
-                        const GemmSeg* segs, double alpha_re, double alpha_im, int cfg, const int* stop) {
+                        const GemmSeg* segs, double alpha_re, double alpha_im, int cfg, const int* stop,
+                 Mark* mark) {
     if (ntiles <= 0) return;
     const float ar = (float)alpha_re, ai = (float)alpha_im;
 #define KV_BF_CASE(OA, OB)                                                                     \
     if (opA == OA && opB == OB) {                                                              \
         if (cfg == 4)                                                                          \
             hipLaunchKernelGGL((zgemm_bf16x3_kernel<OA, OB, 128, 128, 4, 2>), dim3(ntiles),     \
-                               dim3(512), 0, st, A, B, C, tiles, groups, segs, ar, ai, stop);  \
+                               dim3(512), 0, st, A, B, C, tiles, groups, segs, ar, ai, stop, mark); \
         else                                                                                   \
             hipLaunchKernelGGL((zgemm_bf16x3_kernel<OA, OB, 64, 64, 2, 2>), dim3(ntiles),       \
-                               dim3(256), 0, st, A, B, C, tiles, groups, segs, ar, ai, stop);  \
+                               dim3(256), 0, st, A, B, C, tiles, groups, segs, ar, ai, stop, mark); \
         KV_HIP(hipGetLastError());                                                             \
         return;                                                                                \
     }
@@ -704,8 +719,9 @@ __global__ __launch_bounds__(256) void wfold_kernel(const T2* __restrict__ in,
                                                     T2* __restrict__ out,
                                                     const WTask* __restrict__ tasks,
                                                     const WTerm* __restrict__ terms,
-                                                    const int* __restrict__ stop) {
+                                                    const int* __restrict__ stop, Mark* mark) {
     if (stop && *stop) return;
+    write_mark(mark);
     using T = typename ScalarOf<T2>::T;
     const WTask tk = tasks[blockIdx.x];
     const WTerm* __restrict__ tt = terms + tk.term_begin;
@@ -768,19 +784,19 @@ __global__ __launch_bounds__(256) void wfold_kernel(const T2* __restrict__ in,
 
 template <class T2>
 void launch_wfold(hipStream_t st, const T2* in, T2* out, const WTask* tasks, int ntasks,
-                  const WTerm* terms, int64_t maxPQ, const int* stop) {
+                  const WTerm* terms, int64_t maxPQ, const int* stop, Mark* mark) {
     if (ntasks <= 0) return;
     int64_t gy = (maxPQ + 255) / 256;
     if (gy > 64) gy = 64;
     if (gy < 1) gy = 1;
-    hipLaunchKernelGGL((wfold_kernel<T2>), dim3(ntasks, (unsigned)gy), dim3(256), 0, st, in, out, tasks,
-                       terms, stop);
+    hipLaunchKernelGGL((wfold_kernel<T2>), dim3(ntasks, (unsigned)gy), dim3(256), 0, st, in, out, tasks, terms, stop,
+                       mark);
     KV_HIP(hipGetLastError());
 }
 template void launch_wfold<double2>(hipStream_t, const double2*, double2*, const WTask*, int,
-                                    const WTerm*, int64_t, const int*);
+                                    const WTerm*, int64_t, const int*, Mark*);
 template void launch_wfold<float2>(hipStream_t, const float2*, float2*, const WTask*, int,
-                                   const WTerm*, int64_t, const int*);
+                                   const WTerm*, int64_t, const int*, Mark*);
 
 __global__ __launch_bounds__(64) void wcompose_kernel(const WComposeTask* __restrict__ tasks2,
                                                       const WComposeTerm* __restrict__ terms2,
@@ -1137,8 +1153,9 @@ __global__ __launch_bounds__(256) void lanczos_phase_kernel(double2* __restrict_
                                                             const double2* __restrict__ z, int64_t n,
                                                             const double* __restrict__ in, int nb,
                                                             double* __restrict__ out, double2* __restrict__ c_out,
-                                                            const int* __restrict__ stop) {
+                                                            const int* __restrict__ stop, Mark* mark) {
     if (*stop) return;
+    write_mark(mark);
     __shared__ double sh[2][256];
     double2 c = make_double2(0, 0);
     if constexpr (PHASE != LZ_DOT) {
@@ -1238,8 +1255,9 @@ __global__ __launch_bounds__(1024) void lanczos_small_kernel(const double2* __re
                                                              const double2* __restrict__ vk,
                                                              double2* __restrict__ vn, int n,
                                                              LanczosDev* __restrict__ st, int k, double tol,
-                                                             LanczosHost* rec, unsigned long long tag) {
+                                                             LanczosHost* rec, unsigned long long tag, Mark* mark) {
     if (st->stop[k]) return;
+    write_mark(mark);
     __shared__ double sr[64], si[64];
     const int wave = threadIdx.x >> 6, t = threadIdx.x & 63;
     const int nb = (n + 255) / 256;
@@ -1375,14 +1393,14 @@ void launch_lanczos_begin(hipStream_t st, const double2* x, double2* v0, int64_t
 }
 
 void launch_lanczos_step(hipStream_t st, double2* h, const double2* vkm, const double2* vk, double2* vn, int64_t n,
-                         double* part, LanczosDev* dev, int k, double tol, LanczosHost* rec, uint64_t tag) {
+                         double* part, LanczosDev* dev, int k, double tol, LanczosHost* rec, uint64_t tag, Mark* mark) {
     if (n <= kLanczosSmall) {
         static_assert(kLanczosSmall == 3 * 16 * 256, "the chunks of the largest variant");
         const auto f = n <= kLanczosSmall / 3       ? lanczos_small_kernel<1>
                        : n <= 2 * kLanczosSmall / 3 ? lanczos_small_kernel<2>
                                                     : lanczos_small_kernel<3>;
         hipLaunchKernelGGL(f, dim3(1), dim3(1024), 0, st, h, vkm, vk, vn, (int)n, dev, k, tol, rec,
-                           (unsigned long long)tag);
+                           (unsigned long long)tag, mark);
         KV_HIP(hipGetLastError());
         return;
     }
@@ -1392,17 +1410,17 @@ void launch_lanczos_step(hipStream_t st, double2* h, const double2* vkm, const d
     const int* stop = &dev->stop[k];
     if (k > 0) {
         hipLaunchKernelGGL(lanczos_phase_kernel<LZ_DOT>, grid, block, 0, st, h, nullptr, vkm, n, nullptr, 0, pa,
-                           nullptr, stop);
+                           nullptr, stop, mark);
         KV_HIP(hipGetLastError());
         hipLaunchKernelGGL(lanczos_phase_kernel<LZ_SUBDOT>, grid, block, 0, st, h, vkm, vk, n, pa, nb, pb, &dev->beta,
-                           stop);
+                           stop, nullptr);
     } else {
         hipLaunchKernelGGL(lanczos_phase_kernel<LZ_DOT>, grid, block, 0, st, h, nullptr, vk, n, nullptr, 0, pb,
-                           nullptr, stop);
+                           nullptr, stop, mark);
     }
     KV_HIP(hipGetLastError());
     hipLaunchKernelGGL(lanczos_phase_kernel<LZ_SUBNRM>, grid, block, 0, st, h, vk, nullptr, n, pb, nb, pc, &dev->alpha,
-                       stop);
+                       stop, nullptr);
     KV_HIP(hipGetLastError());
     hipLaunchKernelGGL(lanczos_next_kernel, grid, block, 0, st, h, vn, n, pc, nb, dev, k, tol, rec,
                        (unsigned long long)tag);
@@ -1483,17 +1501,19 @@ void launch_f64_to_f32(hipStream_t st, const double2* src, float2* dst, int64_t 
 
 __global__ __launch_bounds__(256) void f32_to_f64_kernel(const float2* __restrict__ s,
                                                          double2* __restrict__ d, double f,
-                                                         int64_t n, const int* __restrict__ stop) {
+                                                         int64_t n, const int* __restrict__ stop, Mark* mark) {
     if (stop && *stop) return;
+    write_mark(mark);
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
         const float2 v = s[e];
         d[e] = make_double2(f * (double)v.x, f * (double)v.y);
     }
 }
 
-void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n, const int* stop) {
+void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s, int64_t n, const int* stop,
+                       Mark* mark) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(f32_to_f64_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, src, dst, s, n, stop);
+    hipLaunchKernelGGL(f32_to_f64_kernel, dim3(ew_blocks(n)), dim3(256), 0, st, src, dst, s, n, stop, mark);
     KV_HIP(hipGetLastError());
 }
 

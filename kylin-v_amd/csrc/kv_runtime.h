@@ -245,6 +245,20 @@ struct Device {
     LanczosDev* lanczos_dev = nullptr;
     LanczosHost* lanczos_host = nullptr;
     uint64_t lanczos_calls = 0;
+    // Pinned chunks of clock marks that no log holds at the moment.  A log is destroyed on the
+    // thread of its context, after the launches that mark into it (its owner waits for them).
+    static constexpr size_t kMarkChunk = 4096;
+    std::vector<Mark*> mark_chunks;
+    Mark* mark_chunk() {
+        Mark* c = nullptr;
+        if (!mark_chunks.empty()) {
+            c = mark_chunks.back();
+            mark_chunks.pop_back();
+        } else {
+            KV_HIP(hipHostMalloc((void**)&c, kMarkChunk * sizeof(Mark), hipHostMallocMapped | hipHostMallocCoherent));
+        }
+        return c;
+    }
     explicit Device(int dev) : id(dev) {
         KV_HIP(hipSetDevice(dev));
         KV_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
@@ -263,6 +277,7 @@ struct Device {
             (void)hipStreamDestroy(stream);
         }
         if (ring_) (void)hipHostFree(ring_);
+        for (Mark* c : mark_chunks) (void)hipHostFree(c);
         if (lanczos_host) (void)hipHostFree(lanczos_host);
         if (lanczos_dev) (void)hipFree(lanczos_dev);
     }
