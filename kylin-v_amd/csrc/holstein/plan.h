@@ -31,7 +31,7 @@ inline std::vector<GemmTile> cut_tiles(const std::vector<GemmGroup>& groups, int
     for (int gi = 0; gi < (int)groups.size(); ++gi) {
         const int tm = (groups[gi].m + bm - 1) / bm, tn = (groups[gi].n + bn - 1) / bn;
         for (int a = 0; a < tm; ++a)
-            for (int b = 0; b < tn; ++b) t.push_back(GemmTile{gi, a, b, 0});
+            for (int b = 0; b < tn; ++b) t.push_back(GemmTile{gi, a, b, groups[gi].seg_begin});
     }
     return t;
 }

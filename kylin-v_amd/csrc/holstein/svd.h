@@ -288,7 +288,8 @@ inline void jacobi_sectors(Device& D, Solver& sol, const std::vector<SectorSvd*>
     size_t work = 0, ns = 0;
     int nmax = 0, mmax = 0;
     for (auto* x : xs) {
-        work += (size_t)(x->nr * x->nc) * (x->nr >= x->nc ? 2 : 1);
+        const size_t k = (size_t)std::min(x->nr, x->nc);
+        work += (size_t)(x->nr * x->nc) * (x->nr >= x->nc ? 2 : 1) + k * k + k;
         soff.push_back(ns);
         ns += (size_t)std::min(x->nr, x->nc);
     }
@@ -311,6 +312,9 @@ inline void jacobi_sectors(Device& D, Solver& sol, const std::vector<SectorSvd*>
             j.T = W.as<double2>() + at;
             at += (size_t)(X.nr * X.nc);
         }
+        j.W = W.as<double2>() + at;
+        j.tau = j.W + (size_t)k * k;
+        at += (size_t)k * k + k;
         j.S = S.as<double>() + soff[i];
         j.nr = (int)X.nr;
         j.nc = (int)X.nc;
@@ -747,7 +751,7 @@ inline void gram_eigvecs(Device& D, Solver& sol, SectorSvd& X, int lo, hipStream
             const int gi = (int)gs.size();
             gs.push_back(g);
             for (int a = 0; a < (m + GEMM_BM - 1) / GEMM_BM; ++a)
-                for (int b = 0; b < (bw + GEMM_BN - 1) / GEMM_BN; ++b) ts.push_back(GemmTile{gi, a, b, 0});
+                for (int b = 0; b < (bw + GEMM_BN - 1) / GEMM_BN; ++b) ts.push_back(GemmTile{gi, a, b, gs[gi].seg_begin});
         };
         std::vector<int> nch(nblk);
         for (int b = 0; b < nblk; ++b) {
@@ -1086,10 +1090,10 @@ inline void gemm_jobs(Device& D, char opA, char opB, const std::vector<GemmJob>&
             if (tune.xcd) {  // rows of tiles in groups of 8, each row's tiles 8 apart
                 for (int a0 = 0; a0 < MT; a0 += 8)
                     for (int b = 0; b < NT; ++b)
-                        for (int a = a0; a < std::min(a0 + 8, MT); ++a) ts.push_back(GemmTile{gi, a, b, 0});
+                        for (int a = a0; a < std::min(a0 + 8, MT); ++a) ts.push_back(GemmTile{gi, a, b, gs[gi].seg_begin});
             } else {
                 for (int a = 0; a < MT; ++a)
-                    for (int b = 0; b < NT; ++b) ts.push_back(GemmTile{gi, a, b, 0});
+                    for (int b = 0; b < NT; ++b) ts.push_back(GemmTile{gi, a, b, gs[gi].seg_begin});
             }
         }
         if (nch > 1) pos += (int64_t)nch * j.m * j.n;

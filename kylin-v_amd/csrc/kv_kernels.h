@@ -99,12 +99,12 @@ void launch_mark(hipStream_t st, Mark* mark);
 // ---- SVD of small sectors ----------------------------------------------------------------
 constexpr int kJacobiMax = 64;  // largest smaller side
 // M (nr x nc, row-major) = U S Vh: U nr x k, Vh k x nc (row-major), S descending, k = min(nr, nc).
-// A and T: workspaces of nr x nc (T only where nr >= nc).  S is NaN where M holds a NaN or an
+// Workspaces: A and T of nr x nc (T only where nr >= nc), W of k x k, tau of k.  S is NaN where M holds a NaN or an
 // infinity and -1 where the rotations did not converge.  Vectors of zero singular values are
 // zero on the shorter side, except those of a zero matrix.
 struct SvdJob {
     const double2* M;
-    double2 *U, *Vh, *A, *T;
+    double2 *U, *Vh, *A, *T, *W, *tau;
     double* S;
     int nr, nc;
 };

@@ -21,6 +21,54 @@ namespace kv {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// ---- sums over a wave's lanes by DPP moves and lane swaps (a few cycles a step; a permute through
+// LDS takes about a hundred) ---------------------------------------------------------------
+// v[t + 32], v[t + 16]: valid in lanes 0..31 / in the lanes of each even row of 16
+__device__ inline double lane_up32(double v) {
+    const long long b = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane32_swap((int)b, (int)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((int)(b >> 32), (int)(b >> 32), false, false);
+    return __longlong_as_double(((long long)hi[1] << 32) | (unsigned)lo[1]);
+}
+__device__ inline double lane_up16(double v) {
+    const long long b = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane16_swap((int)b, (int)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((int)(b >> 32), (int)(b >> 32), false, false);
+    return __longlong_as_double(((long long)hi[1] << 32) | (unsigned)lo[1]);
+}
+// a DPP move of both halves: CTRL 0x100 + s shifts a row of 16 so that lane t reads lane t + s,
+// 0xB1 / 0x4E swap neighbours / pairs, 0x141 mirrors rows of 8, 0x140 rows of 16
+template <int CTRL>
+__device__ inline double lane_dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ inline double lane_first(double v) {  // lane 0's value in every lane
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// The pairwise tree v[t] += v[t + s], s = 32, 16, ..., 1: lane 0 holds the total.
+__device__ inline double tree64(double v) {
+    v += lane_up32(v);
+    v += lane_up16(v);
+    v += lane_dpp<0x108>(v);
+    v += lane_dpp<0x104>(v);
+    v += lane_dpp<0x102>(v);
+    v += lane_dpp<0x101>(v);
+    return v;
+}
+// The sum over each row of 16 in all of its lanes.
+__device__ inline double row_all(double v) {
+    v += lane_dpp<0xB1>(v);
+    v += lane_dpp<0x4E>(v);
+    v += lane_dpp<0x141>(v);
+    v += lane_dpp<0x140>(v);
+    return v;
+}
+
 // The device's wall clock (100 MHz) at the start of a launch's first workgroup.
 __device__ inline void write_mark(Mark* mark) {
     if (mark && (blockIdx.x | blockIdx.y | threadIdx.x) == 0) *mark = wall_clock64();
@@ -110,7 +158,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM * BN <= 
     // thread (one 16-byte access when the segment's offset and leading dimension are even).
     constexpr bool kPair = sizeof(T2) == 8;
     auto load = [&](int s, int k0) {
-        const GemmSeg sg = segs[g.seg_begin + s];
+        const GemmSeg sg = segs[tile.seg + s];
         const T2* __restrict__ a = A + sg.a_off;
         const T2* __restrict__ b = B + sg.b_off;
         const int K = sg.k;
@@ -296,7 +344,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM * BN <= 
         }
     };
     int s = 0, k0 = 0, buf = 0;
-    while (s < g.seg_count && segs[g.seg_begin + s].k <= 0) ++s;
+    while (s < g.seg_count && segs[tile.seg + s].k <= 0) ++s;
     if (s < g.seg_count) {
         load(s, 0);
         store(0);
@@ -306,10 +354,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM * BN <= 
     // other one; the single barrier ends both (the other buffer was last read in t-1)
     while (s < g.seg_count) {
         int s2 = s, k2 = k0 + BK;
-        if (k2 >= segs[g.seg_begin + s].k) {
+        if (k2 >= segs[tile.seg + s].k) {
             k2 = 0;
             ++s2;
-            while (s2 < g.seg_count && segs[g.seg_begin + s2].k <= 0) ++s2;
+            while (s2 < g.seg_count && segs[tile.seg + s2].k <= 0) ++s2;
         }
         if (s2 < g.seg_count) load(s2, k2);
 #pragma unroll
@@ -504,7 +552,7 @@ __global__ __launch_bounds__(64 * (BM / (16 * SI)) * (BN / (16 * SJ))) void zgem
     constexpr int RA = (BM * BK / 2) / NT, RB = (BN * BK / 2) / NT;
     float2 ra[RA][2], rb[RB][2];
     auto load = [&](int s, int k0) {
-        const GemmSeg sg = segs[g.seg_begin + s];
+        const GemmSeg sg = segs[tile.seg + s];
         const float2* __restrict__ a = A + sg.a_off;
         const float2* __restrict__ b = B + sg.b_off;
         const int K = sg.k;
@@ -598,7 +646,7 @@ __global__ __launch_bounds__(64 * (BM / (16 * SI)) * (BN / (16 * SJ))) void zgem
         }
     };
     int s = 0, k0 = 0;
-    while (s < g.seg_count && segs[g.seg_begin + s].k <= 0) ++s;
+    while (s < g.seg_count && segs[tile.seg + s].k <= 0) ++s;
     if (s < g.seg_count) {
         load(s, 0);
         store();
@@ -606,10 +654,10 @@ __global__ __launch_bounds__(64 * (BM / (16 * SI)) * (BN / (16 * SJ))) void zgem
     __syncthreads();
     while (s < g.seg_count) {
         int s2 = s, k2 = k0 + BK;
-        if (k2 >= segs[g.seg_begin + s].k) {
+        if (k2 >= segs[tile.seg + s].k) {
             k2 = 0;
             ++s2;
-            while (s2 < g.seg_count && segs[g.seg_begin + s2].k <= 0) ++s2;
+            while (s2 < g.seg_count && segs[tile.seg + s2].k <= 0) ++s2;
         }
         if (s2 < g.seg_count) load(s2, k2);
         {
@@ -1055,14 +1103,7 @@ static unsigned ew_blocks(int64_t n) {
 // of an iteration read its stop word first, so the host may queue the next iteration before
 // it has seen the scalars of this one.
 // One site at D = 16, 4 levels (nine iterations of 11 launches, a copy and a wait each): 796 us a
-// call before, 368 now; the middle bond at D = 256, 16 levels with its SVD 32.0 -> 29.3 ms.
-
-// The total over a wave of values already summed to one per lane, in the tree's order.
-__device__ inline double tree64(double v) {
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) v += __shfl_down(v, s);
-    return v;
-}
+// call before, 337 now; the middle bond at D = 256, 16 levels with its SVD 32.0 -> 29.3 ms.
 
 // Total of nb partials (NC interleaved components), formed by every wave of a 256-thread
 // workgroup; sh holds 256 values per component.
@@ -1079,8 +1120,8 @@ __device__ inline double2 partials_total(const double* __restrict__ part, int nb
     __syncthreads();
     const int t = threadIdx.x & 63;
     double2 r = make_double2(0, 0);
-    r.x = __shfl(tree64((sh[0][t] + sh[0][t + 128]) + (sh[0][t + 64] + sh[0][t + 192])), 0);
-    if (NC == 2) r.y = __shfl(tree64((sh[1][t] + sh[1][t + 128]) + (sh[1][t + 64] + sh[1][t + 192])), 0);
+    r.x = lane_first(tree64((sh[0][t] + sh[0][t + 128]) + (sh[0][t + 64] + sh[0][t + 192])));
+    if (NC == 2) r.y = lane_first(tree64((sh[1][t] + sh[1][t + 128]) + (sh[1][t + 64] + sh[1][t + 192])));
     return r;
 }
 
@@ -1105,14 +1146,17 @@ __device__ inline void partial_store(double a, double b, double* __restrict__ pa
 // What the host reads of iteration k; `seen` is written last.
 __device__ inline void lanczos_publish(LanczosHost* rec, double2 beta, double2 alpha, double nsq, double err,
                                        unsigned long long tag) {
-    rec->beta_re = beta.x;
-    rec->beta_im = beta.y;
-    rec->alpha_re = alpha.x;
-    rec->alpha_im = alpha.y;
-    rec->nsq = nsq;
-    rec->err = err;
-    __threadfence_system();
-    __hip_atomic_store(&rec->seen, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    // stores past the caches, and a wait for them in place of a system-scope fence, which would
+    // write back the whole L2
+    auto put = [](double* p, double v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+    put(&rec->beta_re, beta.x);
+    put(&rec->beta_im, beta.y);
+    put(&rec->alpha_re, alpha.x);
+    put(&rec->alpha_im, alpha.y);
+    put(&rec->nsq, nsq);
+    put(&rec->err, err);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&rec->seen, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // partial sums of |x|^2; clears the call's stop words and sets err[0] = 1.
@@ -1212,7 +1256,7 @@ __device__ inline double chunk_sum(const double (&p)[4]) { return tree64((p[0] +
 // Total of nb <= 64 chunk partials, in every lane.
 __device__ inline double chunks_total(const double* sh, int nb) {
     const int t = threadIdx.x & 63;
-    return __shfl(tree64(t < nb ? sh[t] : 0.0), 0);
+    return lane_first(tree64(t < nb ? sh[t] : 0.0));
 }
 
 // v_0 = x / |x| and the call's state, in one workgroup (n <= kLanczosSmall).
@@ -1529,7 +1573,7 @@ void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s
 // rows strided over the lanes so that a lane rereads only what it wrote; the wave that updates
 // the next pivot column forms its reflector in the same step.  A half wave takes a pair of
 // columns (n / 2 disjoint pairs a round).
-// A bond of two 768 x 32 sectors: 1.13 ms, 3.7 through zgesvdj.
+// A bond of two 768 x 32 sectors: 0.52 ms (reduction 0.33, rotations 0.16), 3.7 through zgesvdj.
 constexpr double kJacobiTol = 4e-16;  // x sqrt(n): |x_i^H x_j| against |x_i| |x_j|
 constexpr int kJacobiSweeps = 40;
 // Squared norm, next to a largest entry of about one, below which a column counts as zero.  The
@@ -1537,10 +1581,11 @@ constexpr int kJacobiSweeps = 40;
 // length with every sweep and would be rotated until they underflow.
 constexpr double kJacobiZero = 1e-60;
 
-__device__ inline double wave_all(double v) {
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) v += __shfl_xor(v, s);
-    return v;
+__device__ inline double wave_all(double v) { return lane_first(tree64(v)); }
+// the sum over each half wave in all of its lanes
+__device__ inline double half_all(double v) {
+    v = row_all(v);
+    return v + __shfl_xor(v, 16);
 }
 
 // a column's rows lane, lane + 64, ...: in registers (NT > 0, m <= 64 NT) or in memory
@@ -1582,10 +1627,11 @@ struct ColView {
     }
 };
 
-template <int NT>
-__global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restrict__ jobs) {
+template <int NT, int THREADS>
+__global__ __launch_bounds__(THREADS) void jacobi_svd_kernel(const SvdJob* __restrict__ jobs) {
+    constexpr int NW = THREADS / 64;
     extern __shared__ double2 lds[];  // X (n x n), W (n x n)
-    __shared__ double red[16];
+    __shared__ double red[NW];
     __shared__ double2 tau[kJacobiMax];
     __shared__ double rdiag[kJacobiMax], nrm[kJacobiMax];
     __shared__ int ord[kJacobiMax], rotated;
@@ -1599,7 +1645,7 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
     // vanish next to the largest value
     double amax = 0;
     bool bad = false;
-    for (int e = tid; e < m * n; e += 1024) {
+    for (int e = tid; e < m * n; e += THREADS) {
         const double2 v = J.M[e];
         const double a = fmax(fabs(v.x), fabs(v.y));
         bad = bad || !(fabs(v.x) <= 1.7976931348623157e308 && fabs(v.y) <= 1.7976931348623157e308);
@@ -1613,10 +1659,10 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
         return;
     }
     amax = 0;
-    for (int w = 0; w < 16; ++w) amax = fmax(amax, red[w]);
+    for (int w = 0; w < NW; ++w) amax = fmax(amax, red[w]);
     int ex = 0;
     if (amax > 0) (void)frexp(amax, &ex);
-    for (int e = tid; e < m * n; e += 1024) {
+    for (int e = tid; e < m * n; e += THREADS) {
         const double2 v = J.M[e];
         if (tall)
             A[(int64_t)(e % n) * m + e / n] = make_double2(ldexp(v.x, -ex), ldexp(v.y, -ex));
@@ -1656,8 +1702,8 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
             rdiag[j] = beta;
         }
     };
-    // column -= f v (v^H column) over rows j.., f = conj(tau_j) (QR) or tau_j (Q applied)
-    auto reflect = [&](ColView<NT>& c, int j, double2 f, bool store) {
+    // column -= f v (v^H column) over rows j.., f = conj(tau_j)
+    auto reflect = [&](ColView<NT>& c, int j, double2 f) {
         const double2* v = A + (int64_t)j * m;
         double wr = 0, wi = 0;
         c.each(j, false, [&](int i, double2& a) {
@@ -1668,7 +1714,7 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
         wr = wave_all(wr);
         wi = wave_all(wi);
         const double gr = f.x * wr - f.y * wi, gi = f.x * wi + f.y * wr;
-        c.each(j, store, [&](int i, double2& a) {
+        c.each(j, true, [&](int i, double2& a) {
             const double2 u = v[i];
             a.x -= u.x * gr - u.y * gi;
             a.y -= u.x * gi + u.y * gr;
@@ -1682,10 +1728,10 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
     __syncthreads();
     for (int j = 0; j + 1 < n; ++j) {
         const double2 f = make_double2(tau[j].x, -tau[j].y);
-        for (int k = j + 1 + wave; k < n; k += 16) {
+        for (int k = j + 1 + wave; k < n; k += NW) {
             ColView<NT> c(A + (int64_t)k * m, m, lane);
             c.load();
-            reflect(c, j, f, true);
+            reflect(c, j, f);
             if (k == j + 1) reflector(c, j + 1);
         }
         __syncthreads();
@@ -1693,7 +1739,7 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
 
     // X = R^H column by column, W = 1
     double2 *X = lds, *W = lds + n * n;
-    for (int e = tid; e < n * n; e += 1024) {
+    for (int e = tid; e < n * n; e += THREADS) {
         const int i = e / n, r = e % n;
         double2 v = make_double2(0, 0);
         if (r > i) {
@@ -1714,56 +1760,54 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
     int sweep = 0;
     for (; sweep < kJacobiSweeps && n > 1; ++sweep) {
         for (int round = 0; round < N - 1; ++round) {
-            int a = pair == 0 ? N - 1 : (round + pair) % (N - 1);
-            int b = pair == 0 ? round : (round + N - 1 - pair) % (N - 1);
-            if (a > b) {
-                const int q = a;
-                a = b;
-                b = q;
-            }
-            if (pair < N / 2 && b < n) {
-                double2* xa = X + a * n;
-                double2* xb = X + b * n;
+            for (int pr = pair; pr < N / 2; pr += THREADS / 32) {
+                int a = round + pr, b = round + N - 1 - pr;  // mod N - 1; pair 0 holds column N - 1
+                a = pr == 0 ? N - 1 : a >= N - 1 ? a - (N - 1) : a;
+                b = pr == 0 ? round : b >= N - 1 ? b - (N - 1) : b;
+                if (a > b) {
+                    const int q = a;
+                    a = b;
+                    b = q;
+                }
+                if (b >= n) continue;  // odd n: no partner this round
+                double2 *xa = X + a * n, *xb = X + b * n, *wa = W + a * n, *wb = W + b * n;
                 const bool in0 = half < n, in1 = half + 32 < n;
                 const double2 z = make_double2(0, 0);
-                const double2 a0 = in0 ? xa[half] : z, b0 = in0 ? xb[half] : z;
-                const double2 a1 = in1 ? xa[half + 32] : z, b1 = in1 ? xb[half + 32] : z;
-                double na = a0.x * a0.x + a0.y * a0.y + a1.x * a1.x + a1.y * a1.y;
-                double nb = b0.x * b0.x + b0.y * b0.y + b1.x * b1.x + b1.y * b1.y;
-                double cr = a0.x * b0.x + a0.y * b0.y + a1.x * b1.x + a1.y * b1.y;
-                double ci = a0.x * b0.y - a0.y * b0.x + a1.x * b1.y - a1.y * b1.x;
-#pragma unroll
-                for (int s = 16; s > 0; s >>= 1) {
-                    na += __shfl_xor(na, s);
-                    nb += __shfl_xor(nb, s);
-                    cr += __shfl_xor(cr, s);
-                    ci += __shfl_xor(ci, s);
-                }
+                double2 a0 = in0 ? xa[half] : z, b0 = in0 ? xb[half] : z;
+                double2 a1 = in1 ? xa[half + 32] : z, b1 = in1 ? xb[half + 32] : z;
+                double2 p0 = in0 ? wa[half] : z, q0 = in0 ? wb[half] : z;
+                double2 p1 = in1 ? wa[half + 32] : z, q1 = in1 ? wb[half + 32] : z;
+                const double na = half_all(a0.x * a0.x + a0.y * a0.y + a1.x * a1.x + a1.y * a1.y);
+                const double nb = half_all(b0.x * b0.x + b0.y * b0.y + b1.x * b1.x + b1.y * b1.y);
+                const double cr = half_all(a0.x * b0.x + a0.y * b0.y + a1.x * b1.x + a1.y * b1.y);
+                const double ci = half_all(a0.x * b0.y - a0.y * b0.x + a1.x * b1.y - a1.y * b1.x);
                 const double c2 = cr * cr + ci * ci;
                 if (c2 > tol2 * na * nb && fmin(na, nb) > kJacobiZero) {
-                    const double cm = sqrt(c2), zeta = (nb - na) / (2.0 * cm);
-                    const double t = copysign(1.0 / (fabs(zeta) + sqrt(1.0 + zeta * zeta)), zeta);
-                    const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
-                    // the second column's phase that makes <a|b> real
-                    const double er = cr / cm, ei = -ci / cm;
-                    auto turn = [&](double2& u, double2& v) {
-                        const double vr = v.x * er - v.y * ei, vi = v.x * ei + v.y * er;
+                    // d = |b|^2 - |a|^2, r = sqrt(d^2 + 4 |c|^2): cos^2 = (1 + |d| / r) / 2 and
+                    // sin cos = |c| / r; the phase of c goes with the sine
+                    const double d = nb - na, ir = rsqrt(d * d + 4.0 * c2);
+                    const double cs2 = 0.5 + 0.5 * fabs(d) * ir, ic = rsqrt(cs2), cs = cs2 * ic;
+                    const double f = copysign(ir * ic, d), sr = f * cr, si = -f * ci;
+                    auto turn = [&](double2& u, double2& v) {  // (u, v) <- (cs u - s v, conj(s) u + cs v)
                         const double2 o = u;
-                        u = make_double2(cs * o.x - sn * vr, cs * o.y - sn * vi);
-                        v = make_double2(sn * o.x + cs * vr, sn * o.y + cs * vi);
+                        u = make_double2(cs * o.x - (sr * v.x - si * v.y), cs * o.y - (sr * v.y + si * v.x));
+                        v = make_double2(cs * v.x + (sr * o.x + si * o.y), cs * v.y + (sr * o.y - si * o.x));
                     };
-                    double2* wa = W + a * n;
-                    double2* wb = W + b * n;
-                    for (int i = half; i < n; i += 32) {
-                        double2 u = i < 32 ? a0 : a1, v = i < 32 ? b0 : b1;
-                        turn(u, v);
-                        xa[i] = u;
-                        xb[i] = v;
-                        u = wa[i];
-                        v = wb[i];
-                        turn(u, v);
-                        wa[i] = u;
-                        wb[i] = v;
+                    turn(a0, b0);
+                    turn(p0, q0);
+                    if (in0) {
+                        xa[half] = a0;
+                        xb[half] = b0;
+                        wa[half] = p0;
+                        wb[half] = q0;
+                    }
+                    if (in1) {
+                        turn(a1, b1);
+                        turn(p1, q1);
+                        xa[half + 32] = a1;
+                        xb[half + 32] = b1;
+                        wa[half + 32] = p1;
+                        wb[half + 32] = q1;
                     }
                     if (half == 0) rotated = 1;
                 }
@@ -1780,14 +1824,13 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
     const bool failed = sweep == kJacobiSweeps;
 
     // singular values in descending order
-    for (int i = pair; i < n; i += 32) {
+    for (int i = pair; i < n; i += THREADS / 32) {
         double s = 0;
         for (int r = half; r < n; r += 32) {
             const double2 v = X[i * n + r];
             s += v.x * v.x + v.y * v.y;
         }
-#pragma unroll
-        for (int d = 16; d > 0; d >>= 1) s += __shfl_xor(s, d);
+        s = half_all(s);
         if (half == 0) nrm[i] = s > kJacobiZero ? sqrt(s) : 0.0;
     }
     __syncthreads();
@@ -1799,7 +1842,7 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
     }
     __syncthreads();
     // the short side's vectors x = Y / s
-    for (int e = tid; e < n * n; e += 1024) {
+    for (int e = tid; e < n * n; e += THREADS) {
         const int k = e / n, r = e % n, o = ord[k];
         const double f = nrm[o] > 0 ? 1.0 / nrm[o] : amax > 0 ? 0.0 : 1.0;
         // (the value 0 is kept of a zero matrix only: any orthonormal vectors)
@@ -1809,39 +1852,113 @@ __global__ __launch_bounds__(1024) void jacobi_svd_kernel(const SvdJob* __restri
         else
             J.U[r * n + k] = make_double2(f * v.x, f * v.y);
     }
-    // the long side's: Q W
-    for (int k = wave; k < n; k += 16) {
-        ColView<NT> c((tall ? J.T : J.Vh) + (int64_t)k * m, m, lane);
-        const double2* w = W + ord[k] * n;
-        if constexpr (NT > 0) {
+    // the rotations in that order and the reflectors' scalars, for jacobi_apply_kernel
+    for (int e = tid; e < n * n; e += THREADS) J.W[e] = W[ord[e / n] * n + e % n];
+    if (tid < n) J.tau[tid] = tau[tid];
+}
+
+// The long side's vectors: column k of Q [W; 0] in one wave, the next reflector's entries loaded
+// while this one's inner product is reduced.  The columns are spread over the CUs: in the
+// decomposition's own workgroup they took as long as its reduction and rotations together.
+template <int NT>
+__global__ __launch_bounds__(64) void jacobi_apply_kernel(const SvdJob* __restrict__ jobs) {
+    const SvdJob J = jobs[blockIdx.y];
+    const bool tall = J.nr >= J.nc;
+    const int n = tall ? J.nc : J.nr, m = tall ? J.nr : J.nc, k = blockIdx.x, lane = threadIdx.x;
+    if (k >= n) return;
+    const double2* w = J.W + k * n;
+    const double2* A = J.A;
+    ColView<NT> c((tall ? J.T : J.Vh) + (int64_t)k * m, m, lane);
+    auto out = [&](int i, double2& v) {
+        if (tall)
+            J.U[(int64_t)i * n + k] = v;
+        else
+            J.Vh[(int64_t)k * m + i] = make_double2(v.x, -v.y);
+    };
+    if constexpr (NT > 0) {
+        double2 v[NT];
+        auto load = [&](int j) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 const int i = lane + 64 * t;
-                c.r[t] = i < n ? w[i] : make_double2(0, 0);
+                v[t] = make_double2(0, 0);
+                if (i >= j && i < m) v[t] = A[(int64_t)j * m + i];
             }
-        } else {
-            for (int i = lane; i < m; i += 64) c.p[i] = i < n ? w[i] : make_double2(0, 0);
+        };
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int i = lane + 64 * t;
+            c.r[t] = i < n ? w[i] : make_double2(0, 0);
         }
-        for (int j = n - 1; j >= 0; --j) reflect(c, j, tau[j], NT == 0);
-        c.each(0, false, [&](int i, double2& v) {
-            if (tall)
-                J.U[(int64_t)i * n + k] = v;
-            else
-                J.Vh[(int64_t)k * m + i] = make_double2(v.x, -v.y);
-        });
+        load(n - 1);
+        for (int j = n - 1; j >= 0; --j) {
+            const double2 tj = J.tau[j];
+            double2 u[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) u[t] = v[t];
+            if (j > 0) load(j - 1);
+            double wr = 0, wi = 0;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                wr += u[t].x * c.r[t].x + u[t].y * c.r[t].y;
+                wi += u[t].x * c.r[t].y - u[t].y * c.r[t].x;
+            }
+            wr = wave_all(wr);
+            wi = wave_all(wi);
+            const double gr = tj.x * wr - tj.y * wi, gi = tj.x * wi + tj.y * wr;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                c.r[t].x -= u[t].x * gr - u[t].y * gi;
+                c.r[t].y -= u[t].x * gi + u[t].y * gr;
+            }
+        }
+        c.each(0, false, out);
+    } else {
+        for (int i = lane; i < m; i += 64) c.p[i] = i < n ? w[i] : make_double2(0, 0);
+        for (int j = n - 1; j >= 0; --j) {
+            const double2 tj = J.tau[j];
+            const double2* v = A + (int64_t)j * m;
+            double wr = 0, wi = 0;
+            c.each(j, false, [&](int i, double2& a) {
+                const double2 u = v[i];
+                wr += u.x * a.x + u.y * a.y;
+                wi += u.x * a.y - u.y * a.x;
+            });
+            wr = wave_all(wr);
+            wi = wave_all(wi);
+            const double gr = tj.x * wr - tj.y * wi, gi = tj.x * wi + tj.y * wr;
+            c.each(j, true, [&](int i, double2& a) {
+                const double2 u = v[i];
+                a.x -= u.x * gr - u.y * gi;
+                a.y -= u.x * gi + u.y * gr;
+            });
+        }
+        c.each(0, false, out);
     }
 }
 
 void launch_jacobi_svd(hipStream_t st, const SvdJob* jobs, int njobs, int nmax, int mmax) {
     if (njobs <= 0) return;
     const size_t lds = (size_t)2 * nmax * nmax * sizeof(double2);
-    const auto f = mmax <= 64     ? jacobi_svd_kernel<1>
-                   : mmax <= 256  ? jacobi_svd_kernel<4>
-                   : mmax <= 512  ? jacobi_svd_kernel<8>
-                                  : jacobi_svd_kernel<0>;
+    // a column's rows per lane; from nine up half the waves, for the registers
+    const auto f = mmax <= 64     ? jacobi_svd_kernel<1, 1024>
+                   : mmax <= 256  ? jacobi_svd_kernel<4, 1024>
+                   : mmax <= 512  ? jacobi_svd_kernel<8, 1024>
+                   : mmax <= 768  ? jacobi_svd_kernel<12, 512>
+                   : mmax <= 1536 ? jacobi_svd_kernel<24, 512>
+                                  : jacobi_svd_kernel<0, 1024>;
+    const int threads = mmax > 512 && mmax <= 1536 ? 512 : 1024;
     KV_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)((size_t)2 * kJacobiMax * kJacobiMax * sizeof(double2))));
-    hipLaunchKernelGGL(f, dim3(njobs), dim3(1024), lds, st, jobs);
+    hipLaunchKernelGGL(f, dim3(njobs), dim3(threads), lds, st, jobs);
+    KV_HIP(hipGetLastError());
+    const auto g = mmax <= 64     ? jacobi_apply_kernel<1>
+                   : mmax <= 256  ? jacobi_apply_kernel<4>
+                   : mmax <= 512  ? jacobi_apply_kernel<8>
+                   : mmax <= 768  ? jacobi_apply_kernel<12>
+                   : mmax <= 1536 ? jacobi_apply_kernel<24>
+                                  : jacobi_apply_kernel<0>;
+    hipLaunchKernelGGL(g, dim3(nmax, njobs), dim3(64), 0, st, jobs);
     KV_HIP(hipGetLastError());
 }
 
@@ -1960,12 +2077,10 @@ __global__ __launch_bounds__(64) void hh_apply_kernel(const double2* __restrict_
             }
         }
 #pragma unroll
-        for (int s = 32; s > 0; s >>= 1)
-#pragma unroll
-            for (int c = 0; c < HHC; ++c) {
-                dr[c] += __shfl_xor(dr[c], s);
-                di[c] += __shfl_xor(di[c], s);
-            }
+        for (int c = 0; c < HHC; ++c) {
+            dr[c] = lane_first(tree64(dr[c]));
+            di[c] = lane_first(tree64(di[c]));
+        }
 #pragma unroll
         for (int c = 0; c < HHC; ++c) {
             const double gr = ti.x * dr[c] - ti.y * di[c], gi = ti.x * di[c] + ti.y * dr[c];

@@ -20,7 +20,8 @@ struct GemmGroup {
     int m, n, ldc, seg_begin, seg_count, pad;
 };
 struct GemmTile {
-    int group, tm, tn, pad;
+    int group, tm, tn;
+    int seg;  // the group's seg_begin: group and first segment load side by side
 };
 
 constexpr int GEMM_BM = 64, GEMM_BN = 64, GEMM_BK = 8;
