@@ -8,8 +8,8 @@
 //    bond in one launch), else rocSOLVER's (zgesvdj, or zgesvd when cutoff < 0 keeps zero
 //    singular values, whose vectors must still be an orthonormal completion);
 //  * smaller-side Gram (when the isometry is the larger side): G on the smaller side by
-//    the MFMA GEMM, Hermitian eigen-decomposition (batched zhetrd, dstedc per sector,
-//    eigenvectors back-transformed only for the kept values), the isometry as M V / s by
+//    the MFMA GEMM, Hermitian eigen-decomposition (batched zhetrd, divide and
+//    conquer, eigenvectors back-transformed only for the kept values), the isometry as M V / s by
 //    one more GEMM.  The eigenproblem of the two 2048-side Gram matrices of a 32-site,
 //    D=256 bond takes ~0.07 s on MI355X against ~2 s per sector for the Jacobi SVD.
 //    M V / s loses orthonormality like eps (s_max / s)^2, so a sector that keeps values
@@ -491,9 +491,9 @@ inline void hetrd_lower(Device& D, Solver& sol, double2* A, int N, int batch, do
 // batched zhetrd for all sectors (its cost is per column, not per matrix, so the sectors of
 // a bond cost about as much as the largest), every sector padded to the largest side N as
 // diag(G, -I) (G is positive semidefinite, so the padding stays exactly decoupled and each
-// sector's reflectors and tridiagonal are those of G); then dstedc per sector at its own
-// side, and the vectors formed later, only for the rows the truncation needs
-// (gram_eigvecs).  zheevd (all vectors at once, batched) for equal sides below
+// sector's reflectors and tridiagonal are those of G); then the tridiagonals' divide and conquer,
+// all sectors together up to kStedcMax (launch_stedc) and dstedc per sector above, and the
+// vectors formed later, only for the rows the truncation needs (gram_eigvecs).  zheevd (all vectors at once, batched) for equal sides below
 // kSplitEigMin.  (zheevd cannot take the padded matrices: on the split tridiagonal its
 // divide and conquer returns NaN eigenvectors.  dstedc of a pair on two streams measured
 // slower in the sweep than one after the other.)
@@ -586,29 +586,57 @@ inline void gram_solve(Device& D, Solver& sol, std::vector<SectorSvd*> xs, int m
             }
             D.spans.close(trd_t0, D.stream, &D.trd.ms);
         }
-        // the tridiagonal forms, kept for a redo (dstedc overwrites both arrays)
-        DevBuf W0(D.pool.get(), W.bytes()), E0(D.pool.get(), E.bytes());
-        KV_HIP(hipMemcpyAsync(W0.get(), W.get(), W.bytes(), hipMemcpyDeviceToDevice, D.stream));
-        KV_HIP(hipMemcpyAsync(E0.get(), E.get(), E.bytes(), hipMemcpyDeviceToDevice, D.stream));
-        // with `overlap`, a pair of sectors is solved on two streams (the second handle's
-        // stream forks after everything queued so far and the context stream joins it)
-        const bool two = overlap && nb == 2;
-        if (two) {
-            sol.second();
-            KV_HIP(hipEventRecord(sol.fork, D.stream));
-            KV_HIP(hipStreamWaitEvent(sol.s2, sol.fork, 0));
-        }
         for (int b = 0; b < nb; ++b) xs[b]->Zt = DevBuf(D.pool.get(), (size_t)xs[b]->k * xs[b]->k * sizeof(double));
-        for (int b = 0; b < nb; ++b) {
-            const int n = xs[b]->k;
-            const rocblas_status s2 = rocsolver_dstedc(
-                two && b == 1 ? sol.h2 : sol.h, rocblas_evect_tridiagonal, n, W.as<double>() + (size_t)b * N,
-                E.as<double>() + (size_t)b * N, xs[b]->Zt.as<double>(), n, info.as<rocblas_int>() + b);
-            KV_REQUIRE(s2 == rocblas_status_success, ERR_SOLVER, "rocsolver_dstedc failed");
-        }
-        if (two) {
-            KV_HIP(hipEventRecord(sol.join, sol.s2));
-            KV_HIP(hipStreamWaitEvent(D.stream, sol.join, 0));
+        // the tridiagonal forms, kept for a redo (dstedc overwrites both arrays)
+        DevBuf W0(D.pool.get(), W.bytes()), E0(D.pool.get(), E.bytes()), work, jobs;
+        const bool own = N <= kStedcMax;
+        if (own) {
+            std::vector<StedcJob> js(nb);
+            work = DevBuf(D.pool.get(), nb * (3 * NN + 4 * (size_t)N + 4) * sizeof(double));
+            double* at = work.as<double>();
+            for (int b = 0; b < nb; ++b) {
+                StedcJob& j = js[b];
+                j.n = xs[b]->k;
+                j.d = W.as<double>() + (size_t)b * N;
+                j.e = E.as<double>() + (size_t)b * N;
+                j.w = W0.as<double>() + (size_t)b * N;
+                j.Z = xs[b]->Zt.as<double>();
+                j.Q1 = at;
+                j.Q2 = at + NN;
+                j.U = at + 2 * NN;
+                j.d1 = at + 3 * NN;
+                j.d2 = j.d1 + N;
+                j.scale = j.d2 + N;
+                j.src = reinterpret_cast<int*>(j.scale + 1);
+                j.pos = j.src + N;
+                j.kcount = j.pos + N;
+                at += 3 * NN + 4 * (size_t)N + 4;
+            }
+            jobs = upload_vec(D, js);
+            launch_stedc(D.stream, jobs.as<StedcJob>(), nb, N);
+            std::swap(W, W0);
+        } else {
+            KV_HIP(hipMemcpyAsync(W0.get(), W.get(), W.bytes(), hipMemcpyDeviceToDevice, D.stream));
+            KV_HIP(hipMemcpyAsync(E0.get(), E.get(), E.bytes(), hipMemcpyDeviceToDevice, D.stream));
+            // with `overlap`, a pair of sectors is solved on two streams (the second handle's
+            // stream forks after everything queued so far and the context stream joins it)
+            const bool two = overlap && nb == 2;
+            if (two) {
+                sol.second();
+                KV_HIP(hipEventRecord(sol.fork, D.stream));
+                KV_HIP(hipStreamWaitEvent(sol.s2, sol.fork, 0));
+            }
+            for (int b = 0; b < nb; ++b) {
+                const int n = xs[b]->k;
+                const rocblas_status s2 = rocsolver_dstedc(
+                    two && b == 1 ? sol.h2 : sol.h, rocblas_evect_tridiagonal, n, W.as<double>() + (size_t)b * N, E.as<double>() + (size_t)b * N,
+                    xs[b]->Zt.as<double>(), n, info.as<rocblas_int>() + b);
+                KV_REQUIRE(s2 == rocblas_status_success, ERR_SOLVER, "rocsolver_dstedc failed");
+            }
+            if (two) {
+                KV_HIP(hipEventRecord(sol.join, sol.s2));
+                KV_HIP(hipStreamWaitEvent(D.stream, sol.join, 0));
+            }
         }
         // info and the sum of squares of every sector's eigenvectors (NaN check), one wait
         std::vector<double> zsq(nb, 0.0);
@@ -624,8 +652,9 @@ inline void gram_solve(Device& D, Solver& sol, std::vector<SectorSvd*> xs, int m
                     KV_HIP(hipMemcpyAsync(&tails[b], z + cnt - 1, sizeof(double), hipMemcpyDeviceToHost, D.stream));
             }
             KV_HIP(hipMemcpyAsync(zsq.data(), zs.get(), nb * sizeof(double), hipMemcpyDeviceToHost, D.stream));
-            KV_HIP(hipMemcpyAsync(hinfo.data(), info.get(), nb * sizeof(rocblas_int), hipMemcpyDeviceToHost,
-                                  D.stream));
+            if (!own)
+                KV_HIP(hipMemcpyAsync(hinfo.data(), info.get(), nb * sizeof(rocblas_int), hipMemcpyDeviceToHost,
+                                      D.stream));
             D.sync();
             for (int b = 0; b < nb; ++b) zsq[b] += tails[b] * tails[b];
         }
@@ -640,8 +669,9 @@ inline void gram_solve(Device& D, Solver& sol, std::vector<SectorSvd*> xs, int m
             if (ok) continue;
             KV_HIP(hipMemcpyAsync(W.as<double>() + (size_t)b * N, W0.as<double>() + (size_t)b * N, n * sizeof(double),
                                   hipMemcpyDeviceToDevice, D.stream));
-            KV_HIP(hipMemcpyAsync(E.as<double>() + (size_t)b * N, E0.as<double>() + (size_t)b * N, n * sizeof(double),
-                                  hipMemcpyDeviceToDevice, D.stream));
+            if (!own)
+                KV_HIP(hipMemcpyAsync(E.as<double>() + (size_t)b * N, E0.as<double>() + (size_t)b * N,
+                                      n * sizeof(double), hipMemcpyDeviceToDevice, D.stream));
             const rocblas_status s2 = rocsolver_dsteqr(
                 sol.h, rocblas_evect_tridiagonal, n, W.as<double>() + (size_t)b * N,
                 E.as<double>() + (size_t)b * N, xs[b]->Zt.as<double>(), n, info.as<rocblas_int>() + b);
@@ -1282,7 +1312,7 @@ inline void block_ritz(Device& D, Solver& sol, std::vector<BlockJob*>& J, bool i
                       make_double2(1.0 / J[q]->f2, 0.0), make_double2(0.0, 0.0), (int64_t)b * b);
     {
         hipEvent_t t0 = D.spans.mark(D.stream);
-        // the split route (one-workgroup tridiagonalisation, dstedc, back-transformation):
+        // the split route (one-workgroup tridiagonalisation, divide and conquer, back-transformation):
         // rocSOLVER's zheevd spends most of its time reducing a 256-wide matrix column by column
         gram_solve(D, sol, hp, mode == EIG_HEEVD ? EIG_HEEVD : EIG_SPLIT, roc_trd, true);
         if (hp.size() == 2 && mode != EIG_HEEVD) {

@@ -116,6 +116,19 @@ void launch_set_diag(hipStream_t st, double2* A, int64_t ld, int from, int to, d
 // dst (n x n, ld n) = the lower (j <= i) or upper (j >= i) triangle of src (ld lds), the rest zero.
 void launch_tri_copy(hipStream_t st, const double2* src, int64_t lds, double2* dst, int n, bool lower);
 
+// ---- symmetric tridiagonal eigenproblem ------------------------------------------------------
+constexpr int kStedcMax = 512;
+// diag d (n), subdiagonal e (n - 1): eigenvalues ascending into w, vectors into Z (n x n, column-major).
+// Workspaces: Q1, Q2, U of n x n, d1, d2 of n, scale of one; src, pos of n ints, kcount of
+// n / 16 + 1.
+struct StedcJob {
+    const double *d, *e;
+    double *w, *Z, *Q1, *Q2, *U, *d1, *d2, *scale;
+    int *src, *pos, *kcount;
+    int n;
+};
+void launch_stedc(hipStream_t st, const StedcJob* jobs, int njobs, int nmax);
+
 // Back-transformation of a lower-triangle Householder tridiagonalisation (LAPACK layout:
 // reflector i stored below the subdiagonal of column i, tau_i separately).
 // Sides up to kHhApplyMax in one launch: Z = Q C(:, c0 : c0 + k), C real (ld n), Z complex (ld n).

@@ -2023,6 +2023,453 @@ void launch_hh_explicit(hipStream_t st, const double2* A, double2* V, int n, int
     KV_HIP(hipGetLastError());
 }
 
+// ---- symmetric tridiagonal eigenproblem: divide and conquer --------------------------------
+// All matrices of a bond together (sides up to kStedcMax): diagonal blocks of 8 by cyclic Jacobi
+// in a wave each, then levels of merges, each one launch that deflates and solves the secular equations
+// (one workgroup per merge) and one that multiplies the eigenvectors (32 x 32 tiles over all
+// CUs).  Cuppen's splitting with the deflation of LAPACK's dlaed2, roots by Li's two-pole
+// interpolation inside a bracket (LAPACK Working Note 89), vectors from the recomputed z of Gu and
+// Eisenstat (SIAM J. Matrix Anal. Appl. 16 (1995)), which are orthonormal to rounding.
+// Bound by latency: a root's iterations, and the deflation scan.  rocSOLVER's dstedc takes some
+// twenty launches a level and one matrix at a time: 0.45 ms for a side of 128, 0.95 for 256; here a
+// bond's matrices take 0.17 ms together at 128, of which the four merges' secular equations 0.11.
+constexpr int kLeaf = 8;  // (blocks of 32 in 256 threads: 0.34 ms, longer than all merges)
+constexpr double kEps = 1.1102230246251565e-16;
+
+// Total order on (value, index), NaN included, so that a rank by counting is a permutation.
+__device__ inline bool before(double a, int i, double b, int k) {
+    const int64_t u = __double_as_longlong(a), v = __double_as_longlong(b);
+    const int64_t x = u ^ (int64_t)((uint64_t)(u >> 63) >> 1), y = v ^ (int64_t)((uint64_t)(v >> 63) >> 1);
+    return x < y || (x == y && i < k);
+}
+
+__device__ inline double rcp64(double x) {  // 1 / x to an ulp, no special cases
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// Leaves: block b of matrix blockIdx.y, after the split subtracted |e| on both sides of every
+// block boundary; values ascending into d1, vectors into the block of Q.
+__global__ __launch_bounds__(64) void stedc_leaf_kernel(const StedcJob* __restrict__ jobs) {
+    __shared__ double A[kLeaf][kLeaf + 1], V[kLeaf][kLeaf + 1], cs[kLeaf / 2], sn[kLeaf / 2];
+    __shared__ double val[kLeaf];
+    __shared__ int pp[kLeaf / 2], qq[kLeaf / 2], live;
+    const StedcJob J = jobs[blockIdx.y];
+    const int lo = blockIdx.x * kLeaf, n = J.n, tid = threadIdx.x;
+    if (lo >= n) return;
+    const int m = min(kLeaf, n - lo);
+    double big = 0;
+    for (int i = tid; i < n; i += 64) big = fmax(big, fmax(fabs(J.d[i]), i + 1 < n ? fabs(J.e[i]) : 0.0));
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) big = fmax(big, __shfl_xor(big, s));
+    big = fmax(big, 1e-300);
+    const double sc = 1.0 / big;
+    if (blockIdx.x == 0 && tid == 0) J.scale[0] = sc;
+    for (int64_t e = (int64_t)lo * n + tid; e < (int64_t)(lo + m) * n; e += 64) J.Q1[e] = J.Q2[e] = 0.0;
+    for (int e = tid; e < kLeaf * kLeaf; e += 64) {
+        const int i = e / kLeaf, j = e % kLeaf;
+        double v = 0;
+        if (i < m && j < m) {
+            if (i == j) {
+                v = J.d[lo + i] * sc;
+                if (i == 0 && lo > 0) v -= fabs(J.e[lo - 1] * sc);
+                if (i == m - 1 && lo + m < n) v -= fabs(J.e[lo + m - 1] * sc);
+            } else if (i == j + 1 || j == i + 1) {
+                v = J.e[lo + min(i, j)] * sc;
+            }
+        }
+        A[i][j] = v;
+        V[i][j] = i == j ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    for (int sweep = 0; sweep < 20; ++sweep) {
+        if (tid == 0) live = 0;
+        __syncthreads();
+        for (int round = 0; round < kLeaf - 1; ++round) {
+            if (tid < kLeaf / 2) {
+                int a = round + tid, b = round + kLeaf - 1 - tid;
+                a = tid == 0 ? kLeaf - 1 : a >= kLeaf - 1 ? a - (kLeaf - 1) : a;
+                b = tid == 0 ? round : b >= kLeaf - 1 ? b - (kLeaf - 1) : b;
+                const int p = min(a, b), q = max(a, b);
+                const double apq = A[p][q], app = A[p][p], aqq = A[q][q];
+                double c = 1, s = 0;
+                if (fabs(apq) > 0.5 * kEps * (fabs(app) + fabs(aqq)) && fabs(apq) > 1e-300) {
+                    const double th = (aqq - app) / (2.0 * apq);
+                    const double t = copysign(1.0 / (fabs(th) + sqrt(1.0 + th * th)), th);
+                    c = 1.0 / sqrt(1.0 + t * t);
+                    s = t * c;
+                    // a rotation below the absolute accuracy of the block does not hold up the end
+                    if (fabs(apq) > 1e-18) live = 1;
+                }
+                pp[tid] = p;
+                qq[tid] = q;
+                cs[tid] = c;
+                sn[tid] = s;
+            }
+            __syncthreads();
+            {  // columns p, q of A by one half of the wave, of V by the other
+                const int k = (tid & 31) / kLeaf, r = tid % kLeaf, p = pp[k], q = qq[k];
+                const double c = cs[k], s = sn[k];
+                double(*M)[kLeaf + 1] = tid < 32 ? A : V;
+                const double x = M[r][p], y = M[r][q];
+                M[r][p] = c * x - s * y;
+                M[r][q] = s * x + c * y;
+            }
+            __syncthreads();
+            if (tid < 32) {  // rows
+                const int k = tid / kLeaf, r = tid % kLeaf, p = pp[k], q = qq[k];
+                const double c = cs[k], s = sn[k];
+                const double x = A[p][r], y = A[q][r];
+                A[p][r] = c * x - s * y;
+                A[q][r] = s * x + c * y;
+            }
+            __syncthreads();
+        }
+        const int again = live;
+        __syncthreads();
+        if (!again) break;
+    }
+    if (tid < m) val[tid] = A[tid][tid];
+    __syncthreads();
+    if (tid < m) {
+        int rank = 0;
+        for (int i = 0; i < m; ++i) rank += before(val[i], i, val[tid], tid);
+        J.d1[lo + rank] = val[tid];
+        for (int i = 0; i < m; ++i) J.Q1[(int64_t)(lo + rank) * n + lo + i] = V[i][tid];
+    }
+}
+
+// One merge of blocks [lo, mid) and [mid, hi) of width h: what becomes of every column.
+__global__ __launch_bounds__(512) void stedc_merge_kernel(const StedcJob* __restrict__ jobs, int h, int flip) {
+    __shared__ double d[kStedcMax], z[kStedcMax], dk[kStedcMax], zk[kStedcMax], tau[kStedcMax], zh[kStedcMax];
+    __shared__ double rc[kStedcMax], rs[kStedcMax], red[16];
+    __shared__ int ord[kStedcMax], col[kStedcMax], org[kStedcMax], rp[kStedcMax], rq[kStedcMax];
+    __shared__ int K_s, nrot_s;
+    const StedcJob J = jobs[blockIdx.y];
+    const int n = J.n, lo = blockIdx.x * 2 * h, mid = min(lo + h, n), hi = min(lo + 2 * h, n), tid = threadIdx.x;
+    if (lo >= n) return;
+    const int N = hi - lo;
+    const double* din = flip ? J.d2 : J.d1;
+    double* dout = flip ? J.d1 : J.d2;
+    double* Q = flip ? J.Q2 : J.Q1;
+    if (mid >= hi) {  // no partner: every column stays
+        if (tid == 0) J.kcount[lo / (2 * h)] = 0;
+        for (int i = tid; i < N; i += 512) {
+            dout[lo + i] = din[lo + i];
+            J.src[lo + i] = lo + i;
+            J.pos[lo + i] = lo + i;
+        }
+        return;
+    }
+    const double e = J.e[mid - 1] * J.scale[0], rho = 2.0 * fabs(e), inv2 = 0.70710678118654752440;
+    double dm = 0, zm = 0;
+    for (int i = tid; i < N; i += 512) {
+        d[i] = din[lo + i];
+        const double q = i < mid - lo ? Q[(int64_t)(lo + i) * n + mid - 1] : copysign(1.0, e) * Q[(int64_t)(lo + i) * n + mid];
+        z[i] = q * inv2;
+        dm = fmax(dm, fabs(d[i]));
+        zm = fmax(zm, fabs(z[i]));
+    }
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+        dm = fmax(dm, __shfl_xor(dm, s));
+        zm = fmax(zm, __shfl_xor(zm, s));
+    }
+    if ((tid & 63) == 0) {
+        red[tid >> 6] = dm;
+        red[8 + (tid >> 6)] = zm;
+    }
+    __syncthreads();
+    for (int w = 0; w < 8; ++w) {
+        dm = fmax(dm, red[w]);
+        zm = fmax(zm, red[8 + w]);
+    }
+    const double tol = 8.0 * kEps * fmax(dm, zm);
+    for (int i = tid; i < N; i += 512) {
+        int rank = 0;
+        for (int k = 0; k < N; ++k) rank += before(d[k], k, d[i], i);
+        ord[rank] = i;
+    }
+    __syncthreads();
+    for (int k = tid; k < N; k += 512) {
+        tau[k] = d[ord[k]];
+        zh[k] = z[ord[k]];
+    }
+    __syncthreads();
+    // deflation along the ascending values (one thread: each decision depends on the one before)
+    if (tid == 0) {
+        int K = 0, nd = N, nrot = 0, pj = -1, no = ord[0];
+        double dp = 0, zp = 0, dn = tau[0], zn = zh[0];
+        for (int k = 0; k < N; ++k) {
+            const int nj = no, k1 = min(k + 1, N - 1);
+            double dj = dn, zj = zn;
+            no = ord[k1];
+            dn = tau[k1];
+            zn = zh[k1];
+            if (rho * fabs(zj) <= tol) {
+                col[--nd] = nj;
+                continue;
+            }
+            if (pj >= 0) {
+                const double t2 = zp * zp + zj * zj;
+                if (fabs((dj - dp) * zj * zp) <= tol * t2) {  // rotate zp away: its column is an eigenvector
+                    const double ir = 1.0 / sqrt(t2), c = zj * ir, s = -zp * ir;
+                    rp[nrot] = pj;
+                    rq[nrot] = nj;
+                    rc[nrot] = c;
+                    rs[nrot++] = s;
+                    d[pj] = dp * c * c + dj * s * s;
+                    dj = dp * s * s + dj * c * c;
+                    zj = t2 * ir;
+                    col[--nd] = pj;
+                } else {
+                    dk[K] = dp;
+                    zk[K] = zp;
+                    col[K++] = pj;
+                }
+            }
+            pj = nj;
+            dp = dj;
+            zp = zj;
+        }
+        if (pj >= 0) {
+            dk[K] = dp;
+            zk[K] = zp;
+            col[K++] = pj;
+        }
+        K_s = K;
+        nrot_s = nrot;
+    }
+    __syncthreads();
+    const int K = K_s, nrot = nrot_s;
+    // rotations, a row a thread; where one starts at the column that the last one ended at, its
+    // value is carried over, and the loads of eight run together
+    for (int r = lo + tid; nrot > 0 && r < hi; r += 512) {
+        double carry = 0;
+        for (int k0 = 0; k0 < nrot; k0 += 8) {
+            double y[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) y[u] = Q[(int64_t)(lo + rq[min(k0 + u, nrot - 1)]) * n + r];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int k = k0 + u;
+                if (k >= nrot) break;
+                double* x = Q + (int64_t)(lo + rp[k]) * n + r;
+                const double a = k > 0 && rp[k] == rq[k - 1] ? carry : *x;
+                *x = rc[k] * a + rs[k] * y[u];
+                carry = rc[k] * y[u] - rs[k] * a;
+                if (k + 1 == nrot || rp[k + 1] != rq[k]) Q[(int64_t)(lo + rq[k]) * n + r] = carry;
+            }
+        }
+    }
+    // secular equation 1 / rho + sum_j z_j^2 / (d_j - x) = 0: root k between poles k and k + 1 (the
+    // last one above the last pole), as an offset t from the nearer pole in a bracket (a, b) there;
+    // first the root of the two nearest terms with the others as they are in the middle, then
+    // steps of the same form fitted to the value and slopes of the two sides.  TPR lanes a root.
+    constexpr int TPR = 2;
+    const int sub = tid % TPR;
+    const double irho = 1.0 / rho;
+    for (int k = tid / TPR; k < K; k += 512 / TPR) {
+        const bool last = k == K - 1;
+        double zz = 0;
+        if (last) {
+            for (int j = sub; j < K; j += TPR) zz += zk[j] * zk[j];
+            zz += __shfl_xor(zz, 1);
+        }
+        const double gap = last ? rho * zz : dk[k + 1] - dk[k];
+        if (K == 1) {
+            if (sub == 0) {
+                tau[0] = gap;
+                org[0] = 0;
+            }
+            continue;
+        }
+        const int sp = last ? k - 1 : k;  // the two poles of the interpolation: sp and sp + 1
+        double psi, dpsi, phi, dphi;
+        auto eval = [&](int s, double t) {  // the sums over poles <= sp and > sp at d_s + t
+            psi = dpsi = phi = dphi = 0;
+            const double o = dk[s];
+            for (int j = sub; j < K; j += TPR) {
+                const double r = rcp64((dk[j] - o) - t), w = zk[j] * zk[j] * r;
+                if (j <= sp) {
+                    psi += w;
+                    dpsi += w * r;
+                } else {
+                    phi += w;
+                    dphi += w * r;
+                }
+            }
+            psi += __shfl_xor(psi, 1);
+            dpsi += __shfl_xor(dpsi, 1);
+            phi += __shfl_xor(phi, 1);
+            dphi += __shfl_xor(dphi, 1);
+        };
+        int s = k;
+        double t = 0.5 * gap, a = 0.0, b = gap;
+        eval(s, t);
+        double f = irho + psi + phi;
+        const double z1 = zk[sp] * zk[sp], z2 = zk[sp + 1] * zk[sp + 1], del = dk[sp + 1] - dk[sp];
+        const double c = f - z1 / ((dk[sp] - dk[s]) - t) - z2 / ((dk[sp + 1] - dk[s]) - t);
+        if (!last && f < 0) {  // nearer to the upper pole
+            s = k + 1;
+            t = -0.5 * gap;
+            a = t;
+            b = 0.0;
+        } else if (f < 0) {
+            a = t;
+        } else {
+            b = t;
+        }
+        const double p1 = dk[sp] - dk[s], p2 = dk[sp + 1] - dk[s];
+        double x;
+        if (s == sp) {
+            const double A = c * del + z1 + z2, B = z1 * del, D = sqrt(fabs(A * A - 4.0 * B * c));
+            x = A > 0 ? 2.0 * B / (A + D) : (A - D) / (2.0 * c);
+        } else {
+            const double A = z1 + z2 - c * del, B = z2 * del, D = sqrt(fabs(A * A + 4.0 * B * c));
+            x = last ? (A < 0 ? 2.0 * B / (D - A) : (A + D) / (2.0 * c))
+                     : (A > 0 ? -2.0 * B / (A + D) : (A - D) / (2.0 * c));
+        }
+        if (x > a && x < b && x != t) t = x;
+        eval(s, t);
+        f = irho + psi + phi;
+        for (int it = 0; it < 60; ++it) {
+            const double df = dpsi + dphi;
+            if (fabs(f) <= kEps * (8.0 * (fabs(psi) + fabs(phi) + irho) + fabs(t) * df)) break;
+            if (f < 0)
+                a = t;
+            else
+                b = t;
+            const double d1 = p1 - t, d2 = p2 - t;
+            double cc = f - d1 * dpsi - d2 * dphi;
+            const double aa = (d1 + d2) * f - d1 * d2 * df, bb = d1 * d2 * f;
+            const double disc = sqrt(fabs(aa * aa - 4.0 * bb * cc));
+            double eta;
+            if (last) {
+                cc = fabs(cc);
+                eta = aa >= 0 ? (aa + disc) / (2.0 * cc) : 2.0 * bb / (aa - disc);
+            } else {
+                eta = cc == 0 ? bb / aa : aa <= 0 ? (aa - disc) / (2.0 * cc) : 2.0 * bb / (aa + disc);
+            }
+            if (!(f * eta < 0)) eta = -f / df;
+            double tn = t + eta;
+            if (!(tn > a && tn < b)) tn = (f > 0 && a == 0) || (f < 0 && b == 0) ? t / 32 : 0.5 * (a + b);
+            if (tn == t || !(tn > a && tn < b)) break;  // the bracket has closed
+            t = tn;
+            eval(s, t);
+            f = irho + psi + phi;
+        }
+        if (sub == 0) {
+            tau[k] = t;
+            org[k] = s;
+        }
+    }
+    __syncthreads();
+    // z recomputed from the roots, so that they are exact eigenvalues of the modified matrix
+    for (int j = tid / TPR; j < K; j += 512 / TPR) {
+        double p = 1.0;
+        for (int k = sub; k < K; k += TPR) {
+            const double lam = (dk[org[k]] - dk[j]) + tau[k];  // lambda_k - d_j
+            const double den = k < j ? dk[k] - dk[j] : k + 1 < K ? dk[k + 1] - dk[j] : 1.0;
+            p *= lam / den;
+        }
+        p *= __shfl_xor(p, 1);
+        if (sub == 0) zh[j] = copysign(sqrt(fabs(p)), zk[j]);
+    }
+    __syncthreads();
+    for (int k = tid / TPR; k < K; k += 512 / TPR) {
+        const double o = dk[org[k]], t = tau[k];
+        double q = 0;
+        for (int j = sub; j < K; j += TPR) {
+            const double u = zh[j] / ((dk[j] - o) - t);
+            q += u * u;
+        }
+        q += __shfl_xor(q, 1);
+        const double f = 1.0 / sqrt(q);
+        for (int j = sub; j < K; j += TPR) J.U[(int64_t)(lo + j) * n + lo + k] = f * (zh[j] / ((dk[j] - o) - t));
+    }
+    __syncthreads();
+    // ascending order over roots and deflated values
+    for (int i = tid; i < N; i += 512) z[i] = i < K ? dk[org[i]] + tau[i] : d[col[i]];
+    __syncthreads();
+    for (int i = tid; i < N; i += 512) {
+        int rank = 0;
+        for (int k = 0; k < N; ++k) rank += before(z[k], k, z[i], i);
+        dout[lo + rank] = z[i];
+        J.src[lo + i] = lo + col[i];
+        J.pos[lo + i] = lo + rank;
+    }
+    if (tid == 0) J.kcount[lo / (2 * h)] = K;
+}
+
+// Eigenvectors of the merged blocks: column pos[k] = sum_j Q(:, src[j]) U(j, k) over the K roots, the
+// deflated columns copied.  Workgroup (x, y, z): 32 rows x 32 columns of a block pair.
+__global__ __launch_bounds__(256) void stedc_vectors_kernel(const StedcJob* __restrict__ jobs, int h, int flip) {
+    __shared__ double As[32][33], Bs[32][33];
+    const StedcJob J = jobs[blockIdx.z];
+    const int n = J.n, tiles = (2 * h + 31) / 32;
+    const int lo = blockIdx.y * 2 * h, hi = min(lo + 2 * h, n), N = hi - lo;
+    const int r0 = (blockIdx.x / tiles) * 32, c0 = (blockIdx.x % tiles) * 32, tid = threadIdx.x;
+    if (lo >= n || r0 >= N || c0 >= N) return;
+    const double* Q = flip ? J.Q2 : J.Q1;
+    double* out = flip ? J.Q1 : J.Q2;
+    const int K = J.kcount[blockIdx.y];
+    const int tx = tid & 31, ty = tid >> 5;
+    double acc[4] = {0, 0, 0, 0};
+    if (c0 < K) {
+        for (int j0 = 0; j0 < K; j0 += 32) {
+            for (int q = 0; q < 4; ++q) {
+                const int i = ty + 8 * q, j = j0 + i;
+                As[i][tx] = j < K && r0 + tx < N ? Q[(int64_t)J.src[lo + j] * n + lo + r0 + tx] : 0.0;
+                Bs[i][tx] = j < K && c0 + tx < K ? J.U[(int64_t)(lo + j) * n + lo + c0 + tx] : 0.0;
+            }
+            __syncthreads();
+            for (int j = 0; j < 32; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[q] += As[j][tx] * Bs[j][ty + 8 * q];
+            __syncthreads();
+        }
+    }
+    for (int q = 0; q < 4; ++q) {
+        const int c = c0 + ty + 8 * q, r = r0 + tx;
+        if (c < N && r < N) {
+            const double v = c < K ? acc[q] : Q[(int64_t)J.src[lo + c] * n + lo + r];
+            out[(int64_t)J.pos[lo + c] * n + lo + r] = v;
+        }
+    }
+}
+
+// Values scaled back, vectors to their place.
+__global__ __launch_bounds__(256) void stedc_end_kernel(const StedcJob* __restrict__ jobs, int flip) {
+    const StedcJob J = jobs[blockIdx.y];
+    const int64_t nn = (int64_t)J.n * J.n;
+    const double* Q = flip ? J.Q2 : J.Q1;
+    const double* d = flip ? J.d2 : J.d1;
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < nn; e += (int64_t)gridDim.x * 256) J.Z[e] = Q[e];
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < J.n; i += 256) J.w[i] = d[i] / J.scale[0];
+}
+
+static_assert(kLeaf == 8, "the leaf kernel's lanes");
+
+void launch_stedc(hipStream_t st, const StedcJob* jobs, int njobs, int nmax) {
+    KV_REQUIRE(nmax >= 1 && nmax <= kStedcMax, ERR_INTERNAL, "stedc: side above kStedcMax");
+    if (njobs <= 0) return;
+    hipLaunchKernelGGL(stedc_leaf_kernel, dim3((nmax + kLeaf - 1) / kLeaf, njobs), dim3(64), 0, st, jobs);
+    KV_HIP(hipGetLastError());
+    int flip = 0;
+    for (int h = kLeaf; h < nmax; h *= 2, flip ^= 1) {
+        const int nm = (nmax + 2 * h - 1) / (2 * h), tiles = (2 * h + 31) / 32;
+        hipLaunchKernelGGL(stedc_merge_kernel, dim3(nm, njobs), dim3(512), 0, st, jobs, h, flip);
+        KV_HIP(hipGetLastError());
+        hipLaunchKernelGGL(stedc_vectors_kernel, dim3(tiles * tiles, nm, njobs), dim3(256), 0, st, jobs, h, flip);
+        KV_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(stedc_end_kernel, dim3((nmax * nmax + 1023) / 1024, njobs), dim3(256), 0, st, jobs, flip);
+    KV_HIP(hipGetLastError());
+}
+
 // Columns [c0, c0 + k) of C (real, column-major, ld n) carried through the reflectors of A
 // (LAPACK zhetrd('L') storage): Z = H_0 H_1 ... H_{n-2} C(:, c0:c0+k), column-major complex.
 // A wave keeps HHC columns in registers (rows lane + 64 u) and applies the reflectors from the

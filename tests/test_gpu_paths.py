@@ -180,3 +180,30 @@ def test_gram_sectors_svd(sides, keep, l2r, monkeypatch):
         assert np.abs(iso - np.eye(k)).max() < 16 * n * EPS
         gap = s[k - 1] ** 2 - (s[k] ** 2 if k < n else 0.0)
         assert np.linalg.norm(u @ v - (U[:, :k] * s[:k]) @ V[:k]) < 64 * n * EPS / gap
+
+
+# sides around the leaves (32) and merges of the tridiagonal divide and conquer and its largest;
+# spectra whose values deflate in part, all at once and not at all
+@pytest.mark.parametrize("sides", [[128], [130, 66], [97, 160, 95], [193], [384, 64], [512, 65]])
+@pytest.mark.parametrize("spectrum", ["equal", "steps", "deficient", "graded"])
+def test_gram_sectors_of_clustered_values(sides, spectrum, monkeypatch):
+    monkeypatch.setenv("KV_SVD", "full")
+    kv = GE.load_package()
+    rng = np.random.default_rng([*sides, len(spectrum)])
+    print(f"case clustered gram {sides} {spectrum}", flush=True)
+    blocks, rank = {}, 0
+    for q, n in enumerate(sides):
+        u, v = np.linalg.qr(cplx(rng, n, n))[0], np.linalg.qr(cplx(rng, n + 3, n))[0]
+        x = np.arange(n) / n
+        s = {"equal": 0 * x + 1, "steps": 0.5 ** np.floor(4 * x), "deficient": np.where(x < 0.5, 1 - x, 0.0),
+             "graded": 10.0 ** (-3.0 * x)}[spectrum]
+        rank += np.count_nonzero(s)
+        blocks[(q, q)] = (u * s) @ v.conj().T
+    left, right = kv.svd_impl(kv.Tensor.from_blocks((1, -1), blocks), 1, 1e-6, rank, True)
+    L, R = left.to_blocks()[1], right.to_blocks()[1]
+    assert sum(b.shape[1] for b in L.values()) == rank
+    for (q, _), m in blocks.items():
+        n, u = m.shape[0], L[(q, q)]
+        # as in test_gram_sectors_svd; nothing is cut off but zeros, so all of m comes back
+        assert np.abs(u.conj().T @ u - np.eye(u.shape[1])).max() < 16 * n * EPS
+        assert np.linalg.norm(u @ R[(q, q)] - m) < 64 * n * EPS
