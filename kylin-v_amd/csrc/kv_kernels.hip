@@ -3029,8 +3029,8 @@ __global__ __launch_bounds__(256) void trd_matvec_kernel(const double2* __restri
     }
 }
 
-// Householder tridiagonalisation in zhetrd('L')'s form of Hermitian matrices up to
-// kTrdSmallMax wide, one 768-thread workgroup per matrix (column-major, both triangles
+// The columns before the last kTrdRegMax of a Householder tridiagonalisation in zhetrd('L')'s
+// form, Hermitian matrices up to kTrdSmallMax wide, one 768-thread workgroup per matrix (column-major, both triangles
 // valid, as herm_fill leaves them).  Unblocked, with each step's rank-2 update fused into the
 // next step's matrix-vector product: after column j's reflector v_j and y_j = A v_j,
 //   w_j = tau_j y_j - (tau_j / 2) (tau_j y_j)^H v_j v_j,
@@ -3039,9 +3039,10 @@ __global__ __launch_bounds__(256) void trd_matvec_kernel(const double2* __restri
 //   the subdiagonal of column j + 1 and beta on it),
 //   one pass over A(j+2:, j+2:) applying the same update and forming y_{j+1} = A v_{j+1}
 //   (as a combination of columns, exact for the Hermitian A the updates keep).
+// Ends at column `end` (0 < end < n).
 // D, E, tau and the stored reflectors are hetrd_lower's (the back-transformation reads them).
 constexpr int kTrdSmallThreads = 768;
-__global__ __launch_bounds__(kTrdSmallThreads) void trd_small_kernel(double2* __restrict__ A, int n,
+__global__ __launch_bounds__(kTrdSmallThreads) void trd_small_kernel(double2* __restrict__ A, int n, int end,
                                                                      double* __restrict__ Dg, double* __restrict__ Eg,
                                                                      double2* __restrict__ tau) {
     constexpr int NW = kTrdSmallThreads / 64, RU = kTrdSmallMax / 64;
@@ -3196,6 +3197,14 @@ __global__ __launch_bounds__(kTrdSmallThreads) void trd_small_kernel(double2* __
         __syncthreads();
         // column j + 1, up to date, and the norm of its tail
         const int c1 = j + 1;
+        if (c1 == end) {  // the rest is trd_reg_kernel's: brought up to date
+            for (int c = c1 + wv; c < n; c += NW)
+                for (int r = c1 + lane; r < n; r += 64) {
+                    const double2 a = A[(int64_t)c * n + r], p = cmulc(v0[r], w0[c]), q = cmulc(w0[r], v0[c]);
+                    A[(int64_t)c * n + r] = make_double2(a.x - p.x - q.x, a.y - p.y - q.y);
+                }
+            break;
+        }
         const double2 wc = w0[c1], vc = v0[c1];
         s2 = 0.0;
         for (int r = c1 + tid; r < n; r += kTrdSmallThreads) {
@@ -3213,9 +3222,174 @@ __global__ __launch_bounds__(kTrdSmallThreads) void trd_small_kernel(double2* __
     }
 }
 
+// The same for a matrix of up to kTrdRegMax (its corner, when trd_small_kernel has done the columns
+// before it), held in the registers of one 512-thread workgroup: waves 1 to 7 have columns
+// w - 1 + 7 t, lane l rows l and l + 64.  The first wave alone does what is serial, its
+// reductions by DPP: from the waves' parts of y it forms w, and while the others apply the update
+// it brings the next column up to date and reflects it; then the others form y.  Column scalars
+// come by readlane (LDS broadcasts would take as long as the arithmetic).
+// Bound by that chain, 2.5 us a column: a side of 128 takes 0.32 ms (0.78 by trd_small_kernel, which
+// reads and writes the matrix through L2 in every column; 0.43 with all eight waves in turn doing the
+// chain, update and product behind two barriers), a side of 132 0.38 with its first columns (0.80).
+constexpr int kTrdRegMax = 128;
+__device__ inline double lane_get(double v, int l) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, l), hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), l);
+    return __longlong_as_double((int64_t)(((uint64_t)hi << 32) | lo));
+}
+__device__ inline double2 lane_get2(double2 v, int l) { return make_double2(lane_get(v.x, l), lane_get(v.y, l)); }
+
+__global__ __launch_bounds__(512) void trd_reg_kernel(double2* __restrict__ A, int ld, int j0, double* __restrict__ Dg,
+                                                      double* __restrict__ Eg, double2* __restrict__ tau) {
+    constexpr int NW = 7, CT = (kTrdRegMax + NW - 1) / NW;
+    const int n = ld - j0;
+    A += (int64_t)blockIdx.x * ld * ld + (int64_t)j0 * (ld + 1);
+    Dg += (int64_t)blockIdx.x * ld + j0;
+    Eg += (int64_t)blockIdx.x * ld + j0;
+    tau += (int64_t)blockIdx.x * ld + j0;
+    __shared__ double2 vs[2][kTrdRegMax], ws[kTrdRegMax], cs[kTrdRegMax], part[NW][kTrdRegMax];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6) - 1;
+    const double2 zero2 = make_double2(0.0, 0.0);
+    // z - v conj(w)
+    auto sub_mulc = [](double2 z, double2 v, double2 w) {
+        return make_double2(fma(-v.y, w.y, fma(-v.x, w.x, z.x)), fma(v.x, w.y, fma(-v.y, w.x, z.y)));
+    };
+    if (wv >= 0) {
+        double2 a[CT][2];
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int r = lane + 64 * u, c = wv + NW * t;
+                a[t][u] = zero2;
+                if (r < n && c < n && c > 0) a[t][u] = A[(int64_t)c * ld + r];
+            }
+        const int cl = min(wv + NW * (lane % CT), kTrdRegMax - 1);
+        for (int j = 0; j + 1 < n; ++j) {
+            __syncthreads();  // v of column j is there
+            const double2* vj = vs[j & 1];
+            const double2 xs = vj[cl];
+            double2 acc[2] = {zero2, zero2};
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                const int c = wv + NW * t;
+                if (c <= j || c >= n) continue;
+                const double2 xc = lane_get2(xs, t);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    acc[u].x = fma(-a[t][u].y, xc.y, fma(a[t][u].x, xc.x, acc[u].x));
+                    acc[u].y = fma(a[t][u].y, xc.x, fma(a[t][u].x, xc.y, acc[u].y));
+                }
+                if (c == j + 1) {
+                    cs[lane] = a[t][0];
+                    cs[lane + 64] = a[t][1];
+                }
+            }
+            part[wv][lane] = acc[0];
+            part[wv][lane + 64] = acc[1];
+            __syncthreads();
+            double2 vr[2], wr[2];
+            for (int u = 0; u < 2; ++u) vr[u] = vj[lane + 64 * u];
+            __syncthreads();  // w of column j is there
+            const double2 pw = ws[cl];
+            for (int u = 0; u < 2; ++u) wr[u] = ws[lane + 64 * u];
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                const int c = wv + NW * t;
+                if (c <= j + 1 || c >= n) continue;
+                const double2 vc = lane_get2(xs, t), wc = lane_get2(pw, t);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) a[t][u] = sub_mulc(sub_mulc(a[t][u], vr[u], wc), wr[u], vc);
+            }
+        }
+        return;
+    }
+    // larfg on the column x (rows lane, lane + 64) below row j, as trd_small_kernel's reflect
+    double2 v[2] = {zero2, zero2}, x[2], tj = zero2;
+    auto reflect = [&](int j) {
+        double s2 = 0.0;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if (lane + 64 * u >= j + 2) s2 += x[u].x * x[u].x + x[u].y * x[u].y;
+        const double xn2 = wave_all(s2);
+        const int l1 = (j + 1) & 63;
+        const double2 al = lane_get2(j + 1 < 64 ? x[0] : x[1], l1);
+        double beta, tr = 0.0, ti = 0.0;
+        double2 z = make_double2(1.0, 0.0);
+        if (xn2 == 0.0 && al.y == 0.0) {
+            beta = al.x;
+        } else {
+            beta = -copysign(sqrt(al.x * al.x + al.y * al.y + xn2), al.x);
+            tr = (beta - al.x) / beta;
+            ti = -al.y / beta;
+            const double zr = al.x - beta, zi = al.y, z2 = zr * zr + zi * zi;
+            z = make_double2(zr / z2, -zi / z2);
+        }
+        tj = make_double2(tr, ti);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int r = lane + 64 * u;
+            v[u] = r == j + 1 ? make_double2(1.0, 0.0) : r > j + 1 ? cmul(x[u], z) : zero2;
+            vs[j & 1][r] = v[u];
+            if (r > j && r < n) A[(int64_t)j * ld + r] = r == j + 1 ? make_double2(beta, 0.0) : v[u];
+        }
+        if (lane == 0) {
+            Eg[j] = beta;
+            tau[j] = tj;
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < 2; ++u) x[u] = lane + 64 * u < n ? A[lane + 64 * u] : zero2;
+    if (lane == 0) Dg[0] = x[0].x;
+    if (n > 1) reflect(0);
+    for (int j = 0; j + 1 < n; ++j) {
+        __syncthreads();
+        __syncthreads();  // y's parts and column j + 1 are there
+        double2 y[2], d = zero2;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int r = lane + 64 * u;
+            double2 t = part[0][r];
+#pragma unroll
+            for (int q = 1; q < NW; ++q) {
+                t.x += part[q][r].x;
+                t.y += part[q][r].y;
+            }
+            y[u] = r > j ? cmul(tj, t) : zero2;
+            x[u] = cs[r];
+            const double2 e = cmulc(v[u], y[u]);  // conj(tau y) v
+            d.x += e.x;
+            d.y += e.y;
+        }
+        d = make_double2(wave_all(d.x), wave_all(d.y));
+        const double2 al = cmul(make_double2(-0.5 * tj.x, -0.5 * tj.y), d);
+        double2 w[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const double2 av = cmul(al, v[u]);
+            w[u] = make_double2(y[u].x + av.x, y[u].y + av.y);
+            ws[lane + 64 * u] = w[u];
+        }
+        __syncthreads();
+        const int c1 = j + 1, l1 = c1 & 63;
+        const double2 wc = lane_get2(c1 < 64 ? w[0] : w[1], l1), vc = lane_get2(c1 < 64 ? v[0] : v[1], l1);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            x[u] = sub_mulc(sub_mulc(x[u], v[u], wc), w[u], vc);
+            if (lane + 64 * u == c1) Dg[c1] = x[u].x;
+        }
+        if (c1 + 1 < n) reflect(c1);
+    }
+}
+
 void launch_trd_small(hipStream_t st, double2* A, int n, double* D, double* E, double2* tau, int batch) {
     KV_REQUIRE(n >= 1 && n <= kTrdSmallMax && batch >= 1, ERR_INTERNAL, "trd_small: side above kTrdSmallMax");
-    hipLaunchKernelGGL(trd_small_kernel, dim3(batch), dim3(kTrdSmallThreads), 0, st, A, n, D, E, tau);
+    const int j0 = std::max(n - kTrdRegMax, 0);
+    if (j0 > 0) {
+        hipLaunchKernelGGL(trd_small_kernel, dim3(batch), dim3(kTrdSmallThreads), 0, st, A, n, j0, D, E, tau);
+        KV_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(trd_reg_kernel, dim3(batch), dim3(512), 0, st, A, n, j0, D, E, tau);
     KV_HIP(hipGetLastError());
 }
 

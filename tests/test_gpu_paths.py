@@ -182,9 +182,10 @@ def test_gram_sectors_svd(sides, keep, l2r, monkeypatch):
         assert np.linalg.norm(u @ v - (U[:, :k] * s[:k]) @ V[:k]) < 64 * n * EPS / gap
 
 
-# sides around the leaves (32) and merges of the tridiagonal divide and conquer and its largest;
+# sides around the merges (8, 16, ... 256) of the tridiagonal divide and conquer and its largest, and
+# around the side (128) whose reduction stays in registers;
 # spectra whose values deflate in part, all at once and not at all
-@pytest.mark.parametrize("sides", [[128], [130, 66], [97, 160, 95], [193], [384, 64], [512, 65]])
+@pytest.mark.parametrize("sides", [[128], [65, 64], [127, 66], [129], [130, 66], [97, 160, 95], [193], [256], [384, 64], [512, 65]])
 @pytest.mark.parametrize("spectrum", ["equal", "steps", "deficient", "graded"])
 def test_gram_sectors_of_clustered_values(sides, spectrum, monkeypatch):
     monkeypatch.setenv("KV_SVD", "full")
