@@ -3517,7 +3517,8 @@ __device__ __forceinline__ void chol_tile_sum(CholTiles& L, double2 (&acc)[4][4]
             if (cc < bw) pb[q] = S[(int64_t)(i0 + ii) * ld + b_col + cc];
         }
     };
-    if (i_begin < i_end) fetch(i_begin);
+    if (i_begin >= i_end) return;  // uniform over the workgroup
+    fetch(i_begin);
     for (int i0 = i_begin; i0 < i_end; i0 += NB) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
@@ -3604,42 +3605,47 @@ __global__ __launch_bounds__(256) void chol_diag_kernel(const double2* __restric
                 Rf[r][c] = zero2;
             }
     __syncthreads();
-    // factor in LDS, right-looking, all threads, one phase per pivot: every thread reads the
-    // pivot; row kk of R (Dg's row over sqrt(piv)) goes to Rf and the trailing triangle takes
-    // the update with Dg's unscaled row over piv.  Dg's row kk is only read in the phase, and
-    // each thread loads all its operands before it stores.
+    // factor, right-looking, all threads, one phase per pivot: a thread keeps column tid % 32 of
+    // rows tid / 32 + 8 q in registers and updates them with row kk unscaled over the pivot; row
+    // kk + 1, then final, goes to LDS for the next phase.  R's rows (Dg's over sqrt(piv)) are
+    // formed after the last one, so that a phase waits for a reciprocal and not for a root and a
+    // division (with both in each phase, all rows read back from LDS, and both kinds of tile in one
+    // workgroup of the panel's second launch: 31 and 19 us for the two launches of a panel in
+    // blocks 132 wide, 37 and 25 us 256 wide; now 24 and 15, 29 and 18).
     constexpr int NQ = NB * NB / 256;
+    static_assert(NB == 32, "the factor's rows and columns per thread");
+    const int c = tid % NB, i0 = tid / NB;
+    double2 z[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) z[q] = Dg[i0 + 8 * q][c];
+    __syncthreads();
     unsigned lv = 0u;
     for (int kk = 0; kk < w; ++kk) {
         const double piv = Dg[kk][kk].x;
+        const double2 y = Dg[kk][c];
         const bool lk = piv > thr && piv > 0.0;  // NaN is not live
-        const double sp = lk ? sqrt(piv) : 0.0;
-        const double ri = lk ? 1.0 / sp : 0.0, rp = ri * ri;
+        const double rp = lk ? rcp64(piv) : 0.0;
         lv |= lk ? 1u << kk : 0u;
-        double2 xa[NQ], ya[NQ], za[NQ];
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-            const int e = tid + 256 * q, i = e / NB, c = e % NB;
-            xa[q] = zero2;
-            za[q] = zero2;
-            ya[q] = Dg[kk][c];
+            const int i = i0 + 8 * q;
+            if (8 * q + 7 <= kk) continue;  // uniform
             if (i > kk && c >= i && c < w) {
-                xa[q] = Dg[kk][i];
-                za[q] = Dg[i][c];
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int e = tid + 256 * q, i = e / NB, c = e % NB;
-            if (i == kk && c >= kk && c < w)
-                Rf[kk][c] = c == kk ? make_double2(sp, 0.0) : make_double2(ya[q].x * ri, ya[q].y * ri);
-            if (lk && i > kk && c >= i && c < w) {
-                const double2 x = xa[q], y = ya[q];
-                Dg[i][c] = make_double2(za[q].x - (x.x * y.x + x.y * y.y) * rp, za[q].y - (x.x * y.y - x.y * y.x) * rp);
+                const double2 x = Dg[kk][i];
+                if (lk) z[q] = make_double2(z[q].x - (x.x * y.x + x.y * y.y) * rp, z[q].y - (x.x * y.y - x.y * y.x) * rp);
+                if (i == kk + 1) Dg[i][c] = z[q];
             }
         }
         __syncthreads();
     }
+    for (int e = tid; e < NB * NB; e += 256) {
+        const int i = e / NB, c = e % NB;
+        if (i < w && c >= i && c < w) {  // R
+            const double sp = (lv >> i) & 1u ? sqrt(Dg[i][i].x) : 0.0, ri = sp > 0.0 ? 1.0 / sp : 0.0;
+            Rf[i][c] = c == i ? make_double2(sp, 0.0) : make_double2(Dg[i][c].x * ri, Dg[i][c].y * ri);
+        }
+    }
+    __syncthreads();
     // Ti = diag(1 / R_ii) over live indices
     for (int e = tid; e < NB * NB; e += 256) {
         const int i = e / NB, c = e % NB;
@@ -3648,19 +3654,24 @@ __global__ __launch_bounds__(256) void chol_diag_kernel(const double2* __restric
     __syncthreads();
     // recursive doubling: for pairs (A = [p, p+s), C = [p+s, p+2s)): M = R_AC T_C, T_AC = -T_A M
     // (M in Dg, free after the factor)
+#pragma unroll
     for (int s = 1; s < NB; s *= 2) {
         const int per = s * s, tot = (NB / (2 * s)) * per;  // outputs per pair, all pairs
         for (int e = tid; e < tot; e += 256) {
             const int pr = e / per, rr = (e % per) / s, cc = e % s, p = pr * 2 * s;
             double2 m = zero2;
-            for (int t = 0; t <= cc; ++t) m = cfma(m, Rf[p + rr][p + s + t], Ti[p + s + t][p + s + cc]);
+#pragma unroll
+            for (int t = 0; t < s; ++t)
+                if (t <= cc) m = cfma(m, Rf[p + rr][p + s + t], Ti[p + s + t][p + s + cc]);
             Dg[p + rr][p + s + cc] = m;
         }
         __syncthreads();
         for (int e = tid; e < tot; e += 256) {
             const int pr = e / per, rr = (e % per) / s, cc = e % s, p = pr * 2 * s;
             double2 m = zero2;
-            for (int t = rr; t < s; ++t) m = cfma(m, Ti[p + rr][p + t], Dg[p + t][p + s + cc]);
+#pragma unroll
+            for (int t = 0; t < s; ++t)
+                if (t >= rr) m = cfma(m, Ti[p + rr][p + t], Dg[p + t][p + s + cc]);
             Ti[p + rr][p + s + cc] = make_double2(-m.x, -m.y);
         }
         __syncthreads();
@@ -3673,9 +3684,9 @@ __global__ __launch_bounds__(256) void chol_diag_kernel(const double2* __restric
     if (tid < w) live[p0 + tid] = (lv >> tid) & 1u;
 }
 
-// Launch B of panel k, grid (ceil(nmax / 32), batch): workgroup j with 0 < j < (panels from k
-// on) writes R's tile (k, k + j) = Di^H (S_kc - R_{<k,k}^H R_{<k,c}) into S and a zero tile
-// (k + j, k) into T; workgroup j < k writes T's tile (j, k) = -(T_{j, j..k-1} R_{j..k-1, k}) Di.
+// Launch B of panel k, grid (ceil(nmax / 32), batch), one of np - 1 tiles a workgroup: for 0 < j <
+// npk (panels from k on) R's tile (k, k + j) = Di^H (S_kc - R_{<k,k}^H R_{<k,c}) into S and a zero
+// tile (k + j, k) into T; for j < k T's tile (j, k) = -(T_{j, j..k-1} R_{j..k-1, k}) Di.
 // Tiles of S and T written here are read by no other workgroup of the launch.
 __global__ __launch_bounds__(256) void chol_panel_kernel(double2* __restrict__ S, const int* __restrict__ sizes,
                                                          int ld, int64_t stride, double2* __restrict__ T,
@@ -3685,10 +3696,9 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(double2* __restrict__ S
     const int p0 = k * NB;
     if (p0 >= n) return;  // uniform over the workgroup
     const int w = min(NB, n - p0);
-    const int j = blockIdx.x;
     const int npk = (n - p0 + NB - 1) / NB;
-    const bool off = j > 0 && j < npk;
-    const bool inv = j < k;
+    const bool off = (int)blockIdx.x < npk - 1, inv = !off && (int)blockIdx.x < npk - 1 + k;
+    const int j = off ? blockIdx.x + 1 : blockIdx.x - (npk - 1);
     if (!off && !inv) return;  // uniform over the workgroup
     S += (int64_t)b * stride;
     T += (int64_t)b * stride;
@@ -3718,15 +3728,19 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(double2* __restrict__ S
                     Ct[rr][c] = v;
                 }
         __syncthreads();
+        double2 yv[4] = {zero2, zero2, zero2, zero2};
+#pragma unroll 4
+        for (int m = 0; m <= r; ++m) {
+            const double2 d = Di[m][r];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) yv[q] = cfma_conj(yv[q], d, Ct[m][cq + q]);
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int c = cq + q;
-            double2 yv = zero2;
-            for (int m = 0; m <= r; ++m) yv = cfma_conj(yv, Di[m][r], Ct[m][c]);
-            if (r < w && c < wc) S[(int64_t)(p0 + r) * ld + c0 + c] = yv;
+            if (r < w && c < wc) S[(int64_t)(p0 + r) * ld + c0 + c] = yv[q];
             if (c < w && r < wc) T[(int64_t)(c0 + r) * ld + p0 + c] = zero2;
         }
-        __syncthreads();  // Ct is reused
     }
     if (inv) {
         const int R0 = j * NB;
@@ -3738,13 +3752,17 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(double2* __restrict__ S
 #pragma unroll
                 for (int y = 0; y < 4; ++y) Ct[r4 + x][c4 + y] = xa[x][y];
         __syncthreads();
+        double2 yv[4] = {zero2, zero2, zero2, zero2};
+#pragma unroll 4
+        for (int m = 0; m < cq + 4; ++m) {
+            const double2 d = Ct[r][m];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int c = cq + q;
-            double2 yv = zero2;
-            for (int m = 0; m <= c; ++m) yv = cfma(yv, Ct[r][m], Di[m][c]);
-            if (c < w) T[(int64_t)(R0 + r) * ld + p0 + c] = make_double2(-yv.x, -yv.y);
+            for (int q = 0; q < 4; ++q)
+                if (m <= cq + q) yv[q] = cfma(yv[q], d, Di[m][cq + q]);
         }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (cq + q < w) T[(int64_t)(R0 + r) * ld + p0 + cq + q] = make_double2(-yv[q].x, -yv[q].y);
     }
 }
 
