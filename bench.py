@@ -163,7 +163,7 @@ def traffic_from_profiles(kernel_key):
 
 
 def kernel_table(st, steps):
-    """GPU seconds per step of each kernel class, from the engine's HIP-event counters."""
+    """GPU seconds per step of each kernel class, from the engine's counters of device time."""
     g64 = st["heff_gemm_gpu_s"] - st["heff_gemm32_gpu_s"]
     return {
         "heff_gemm_fp32_operands": st["heff_gemm32_gpu_s"] / steps,
@@ -179,7 +179,7 @@ def kernel_table(st, steps):
 
 def rooflines(st, precision):
     """Roofline entries for the kernels that have one, each from algorithmic work per launch
-    over the HIP-event time per launch."""
+    over the device time per launch."""
     out = {}
     n32 = st["heff_gemm32_launches"]
     if n32 > 0 and st["heff_gemm32_gpu_s"] > 0:

@@ -179,11 +179,12 @@ int kv_krylov_step(kv_ctx* ctx, int nsite, const kv_tensor* L, const kv_tensor* 
  * Rayleigh-Ritz, each Ritz pair's residual checked against 1e-13 of the largest value;
  * a cut the certified values cannot settle sends the sector to the full route.  Otherwise
  * sectors whose smaller side is at least 64 are solved through their Gram matrix on the
- * isometric side (Hermitian eigen-decomposition: from side 512, or for sectors of
- * different sides, the engine's batched Householder tridiagonalisation, rocSOLVER's dstedc
- * and the kept vectors carried back through the reflectors; below that rocSOLVER's zheevd;
- * a second pass over the tail below 1e-5 of the largest value); smaller ones by rocSOLVER's
- * Jacobi SVD.  KV_SVD=full in the environment turns the block route off. */
+ * isometric side (Hermitian eigen-decomposition: from side 128, or for sectors of
+ * different sides, the engine's batched Householder tridiagonalisation, its tridiagonal
+ * divide and conquer (rocSOLVER's dstedc above side 512) and the kept vectors carried back
+ * through the reflectors; below that rocSOLVER's zheevd; a second pass over the tail below
+ * 1e-5 of the largest value); smaller ones by a one-workgroup Jacobi SVD where cutoff < 0 or
+ * the longer side is at least 128, else by rocSOLVER's.  KV_SVD=full in the environment turns the block route off. */
 int kv_svd_truncate(kv_ctx* ctx, const kv_tensor* A, int r1, double cutoff, int maxdim,
                     int left_to_right, kv_tensor** left, kv_tensor** right, int* nkept);
 

@@ -1,7 +1,7 @@
 // The enrichment SVD of SA-1TDVP on the device.
 //
 // Replaces sa_svd_impl<R1,R2> (holstein/svd.h:443-614) with gs_ortho (util/allocation.h:
-// 260-327): every sector is decomposed in full (rocSOLVER's one-sided SVD, nothing
+// 260-327): every sector is decomposed in full (the exact route of svd.h, nothing
 // truncated, S absorbed as svd_impl does), sa_extension_count decides how many states to
 // add, and the sectors with room on the isometric side (rows when sweeping right, columns
 // when sweeping left), in ascending row charge, receive seeded random vectors made

@@ -233,7 +233,7 @@ struct Device {
     hipStream_t stream = nullptr;
     std::unique_ptr<Pool> pool;
     SpanLog spans;
-    bool timing = false;  // record HIP events around contraction kernels
+    bool timing = false;  // take the device's clock around contraction kernels
     KernelStats stats;
     TrdStats trd;
     BlockStats blk;
