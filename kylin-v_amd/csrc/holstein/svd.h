@@ -662,11 +662,10 @@ inline void gram_solve(Device& D, Solver& sol, std::vector<SectorSvd*> xs, int m
             for (int64_t m = 1; m < N; ++m) D.trd.bytes += 16.0 * (double)(m * (m + 1) / 2) * nb;
             D.trd.columns += (long)N * nb;
         }
-        for (int b = 0; b < nb; ++b) {
+        // the own divide and conquer writes no status
+        for (int b : eig_redos(own ? std::vector<int>() : hinfo, zsq)) {
             const int n = xs[b]->k;
             const int64_t nn = (int64_t)n * n;
-            const bool ok = hinfo[b] == 0 && std::isfinite(zsq[b]);
-            if (ok) continue;
             KV_HIP(hipMemcpyAsync(W.as<double>() + (size_t)b * N, W0.as<double>() + (size_t)b * N, n * sizeof(double),
                                   hipMemcpyDeviceToDevice, D.stream));
             if (!own)
@@ -676,8 +675,10 @@ inline void gram_solve(Device& D, Solver& sol, std::vector<SectorSvd*> xs, int m
                 sol.h, rocblas_evect_tridiagonal, n, W.as<double>() + (size_t)b * N,
                 E.as<double>() + (size_t)b * N, xs[b]->Zt.as<double>(), n, info.as<rocblas_int>() + b);
             KV_REQUIRE(s2 == rocblas_status_success, ERR_SOLVER, "rocsolver_dsteqr failed");
-            read_info();
-            KV_REQUIRE(hinfo[b] == 0 && std::isfinite(dev_sumsq(D, xs[b]->Zt.as<double>(), nn)), ERR_SOLVER,
+            rocblas_int st = 0;
+            KV_HIP(hipMemcpyAsync(&st, info.as<rocblas_int>() + b, sizeof st, hipMemcpyDeviceToHost, D.stream));
+            D.sync();
+            KV_REQUIRE(st == 0 && std::isfinite(dev_sumsq(D, xs[b]->Zt.as<double>(), nn)), ERR_SOLVER,
                        "Hermitian eigensolver did not converge");
         }
         for (int b = 0; b < nb; ++b) {

@@ -10,6 +10,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <tuple>
 #include <vector>
@@ -104,6 +105,15 @@ inline std::vector<int> truncation_counts(const std::vector<std::vector<double>>
             break;
     }
     return kept;
+}
+
+// Matrices of a batched eigensolve that have to be redone: those whose status is not 0 (`info`, empty
+// for a solver that reports none) or whose eigenvectors' sum of squares is not finite.
+inline std::vector<int> eig_redos(const std::vector<int>& info, const std::vector<double>& sumsq) {
+    std::vector<int> redo;
+    for (int b = 0; b < (int)sumsq.size(); ++b)
+        if ((!info.empty() && info[b] != 0) || !std::isfinite(sumsq[b])) redo.push_back(b);
+    return redo;
 }
 
 }  // namespace kv
