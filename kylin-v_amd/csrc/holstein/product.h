@@ -157,7 +157,7 @@ struct DevProduct {
     }
     void ensure_tiles(Device& dev, int cfg) {
         if (cut[cfg]) return;
-        std::vector<GemmTile> t = cut_tiles(p.groups, cfg);
+        std::vector<GemmTile> t = cut_tiles(nch > 1 ? split_k(p, nch).groups : p.groups, cfg);
         tiles[cfg] = upload_vec(dev, t);
         tp[cfg] = tiles[cfg].as<GemmTile>();
         ntiles[cfg] = (int)t.size();
@@ -215,11 +215,11 @@ struct DevProduct {
                            groups, segs, ar, ai, cfg, stop, mark);
         if (nch > 1) launch_sum_parts<float2>(dev.stream, part.as<float2>(), nch, p.out.total, C, stop);
     }
-    // Split-BF16 tile (64x64 or 128x128), timed once per shape class like choose().
+    // Split-BF16 tile (64x64 or 128x128): KV_SPLIT_TILE's, also for a plan cut into K chunks, else
+    // timed once per shape class like choose().
     int choose_split(Device& dev, const float2* A, const float2* B, float2* C, double ar, double ai) {
-        if (nch > 1) return 0;
         if (const char* t = std::getenv("KV_SPLIT_TILE")) return std::atoi(t) == 128 ? 4 : 0;
-        if (!dev.autotune || p.flop < 1e8) return 0;
+        if (!dev.autotune || p.flop < 1e8 || nch > 1) return 0;
         const uint64_t key = gemm_shape_key(p, 2);
         auto it = dev.gemm_tuned.find(key);
         if (it != dev.gemm_tuned.end()) return it->second;
