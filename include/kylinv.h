@@ -238,7 +238,9 @@ int kv_tdvp_bond_dims(kv_tdvp* s, int* dims);
  * (holstein/tdvp.h:85-214): "Evl-2","Evl-1","Evl-0","SVD","Update","Sweep", plus
  * GPU time (the device clock at the start of successive launches) and algorithmic flops of the H_eff matvec
  * kernels and of the environment-update kernels.  Writes up to n values in this order:
- *   0 Evl-2  1 Evl-1  2 Evl-0  3 SVD  4 Update  5 Sweep  (wall seconds)
+ *   0 Evl-2  1 Evl-1  2 Evl-0  3 SVD  4 Update  5 Sweep  (wall seconds; an environment
+ *      update is only queued where it is called: the device time that the next module then
+ *      waits for counts as Update and not as that module)
  *   6 heff_gpu_s  7 heff_flop  8 env_gpu_s  9 env_flop  10 matvecs
  *   11 heff_gemm_gpu_s  12 heff_gemm_flop  13 heff_gemm_launches
  *   14 heff_wfold_gpu_s 15 heff_wfold_flop 16 heff_wfold_launches

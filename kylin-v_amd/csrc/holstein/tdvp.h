@@ -5,6 +5,7 @@
 // and overlap(State, State) (holstein/state.h:206-227).
 #pragma once
 
+#include <algorithm>
 #include <chrono>
 #include <complex>
 #include <cstdio>
@@ -27,7 +28,9 @@ struct TdvpConfig {
     Prec prec = PREC_F64;
 };
 
-// Wall-clock module timers with the reference's Timer names (holstein/tdvp.h:85-214).
+// Wall-clock module timers with the reference's Timer names (holstein/tdvp.h:85-214).  A sweep does
+// not wait for an environment update: its device time is taken from the module that does, and added
+// to update.
 struct TdvpTimers {
     double evl2 = 0, evl1 = 0, evl0 = 0, svd = 0, update = 0, sweep = 0;
     double global = 0;  // global Krylov steps ("Krylov-Iter" + "Krylov-Diag")
@@ -100,6 +103,7 @@ class TDVP {
         envR_.push_back(right_boundary(dev_, last.blocks[0].qn[2]));
         for (int i = (int)mps_.size() - 1; i > 0; --i)
             envR_.push_back(update(*envR_.back(), *mps_[i], *mpo_[i], false));
+        settle();
     }
 
     // One global Krylov step (defined in krylov.h).
@@ -114,7 +118,7 @@ class TDVP {
             auto mm = product(dev_, *mps_[i], *mps_[i + 1], 1, 'N', 'N');
             krylov(2, mm, mpo_[i].get(), mpo_[i + 1].get(), false);
             const double te = c.s();
-            tm_.evl2 += te;
+            book(tm_.evl2, te);
             Clock c2;
             SvdResult r = bond_svd(*mm, i, true);
             log_svs(r);
@@ -130,7 +134,7 @@ class TDVP {
                 tm_.update += c3.s();
                 Clock c4;
                 krylov(1, r.right, mpo_[i + 1].get(), nullptr, true);
-                tm_.evl1 += c4.s();
+                book(tm_.evl1, c4.s());
                 mps_[i + 1] = std::move(r.right);
                 envR_.pop_back();
             } else {
@@ -142,7 +146,7 @@ class TDVP {
             auto mm = product(dev_, *mps_[i - 1], *mps_[i], 1, 'N', 'N');
             krylov(2, mm, mpo_[i - 1].get(), mpo_[i].get(), false);
             const double te = c.s();
-            tm_.evl2 += te;
+            book(tm_.evl2, te);
             Clock c2;
             SvdResult r = bond_svd(*mm, i - 1, false);
             log_svs(r);
@@ -158,7 +162,7 @@ class TDVP {
                 tm_.update += c3.s();
                 Clock c4;
                 krylov(1, r.left, mpo_[i - 1].get(), nullptr, true);
-                tm_.evl1 += c4.s();
+                book(tm_.evl1, c4.s());
                 mps_[i - 1] = std::move(r.left);
                 envL_.pop_back();
             } else {
@@ -167,6 +171,7 @@ class TDVP {
         }
         Clock c5;
         envR_.push_back(update(*envR_.back(), *mps_[1], *mpo_[1], false));
+        settle();
         tm_.update += c5.s();
     }
 
@@ -188,7 +193,7 @@ class TDVP {
         for (int i = 0; i < ns; ++i) {
             Clock c;
             krylov(1, mps_[i], mpo_[i].get(), nullptr, false);
-            tm_.evl1 += c.s();
+            book(tm_.evl1, c.s());
             if (i < ns - 1) {
                 Clock c2;
                 SvdResult r = split(*mps_[i], 2, true, i);
@@ -199,7 +204,7 @@ class TDVP {
                 tm_.update += c3.s();
                 Clock c4;
                 krylov(0, r.right, nullptr, nullptr, true);
-                tm_.evl0 += c4.s();
+                book(tm_.evl0, c4.s());
                 Clock c5;
                 mps_[i + 1] = product(dev_, *r.right, *mps_[i + 1], 1, 'N', 'N');
                 tm_.sweep += c5.s();
@@ -209,7 +214,7 @@ class TDVP {
         for (int i = ns - 1; i >= 0; --i) {
             Clock c;
             krylov(1, mps_[i], mpo_[i].get(), nullptr, false);
-            tm_.evl1 += c.s();
+            book(tm_.evl1, c.s());
             if (i > 0) {
                 Clock c2;
                 SvdResult r = split(*mps_[i], 1, false, i - 1);
@@ -220,7 +225,7 @@ class TDVP {
                 tm_.update += c3.s();
                 Clock c4;
                 krylov(0, r.left, nullptr, nullptr, true);
-                tm_.evl0 += c4.s();
+                book(tm_.evl0, c4.s());
                 Clock c5;
                 mps_[i - 1] = product(dev_, *mps_[i - 1], *r.left, 1, 'N', 'N');
                 tm_.sweep += c5.s();
@@ -239,15 +244,10 @@ class TDVP {
     const TdvpTimers& timers() const { return tm_; }
     const LanczosStats& lanczos_stats() const { return ls_; }
     const KernelStats& heff_kernels() const { return heff_k_; }
-    const KernelStats& env_kernels() {
-        dev_->sync();
-        env_log_.resolve(env_k_);
-        return env_k_;
-    }
+    const KernelStats& env_kernels() const { return env_k_; }
     double env_flop() const { return env_flop_; }
     Device& device() { return *dev_; }
     void reset_stats() {
-        (void)env_kernels();
         tm_ = TdvpTimers();
         ls_ = LanczosStats();
         env_flop_ = 0;
@@ -290,8 +290,23 @@ class TDVP {
         KrylovExit ex = local_krylov(dev_, nsite, *envL_.back(), W1, W2, *envR_.back(), x, cfg_.dt,
                                      cfg_.krylov_tol, cfg_.krylov_maxiter, reverse, cfg_.prec,
                                      timing ? &log_ : nullptr, &ls_, &heff_k_);
+        const double before = env_k_.gemm_ms + env_k_.wfold_ms;
         env_log_.resolve(env_k_);  // the step has waited for the stream
+        env_late_ = 1e-3 * (env_k_.gemm_ms + env_k_.wfold_ms - before);
         last_iters_ = ex.iterations;
+    }
+    // Books the wall time of a module whose krylov() has just returned: what of it the environment
+    // updates queued before it ran on for is theirs.
+    void book(double& module, double wall) {
+        const double late = std::min(wall, env_late_);
+        env_late_ = 0;
+        module += wall - late;
+        tm_.update += late;
+    }
+    // Waits for the updates that no later module waits for.
+    void settle() {
+        dev_->sync();
+        env_log_.resolve(env_k_);
     }
 
     std::shared_ptr<Device> dev_;
@@ -303,7 +318,7 @@ class TDVP {
     LanczosStats ls_;
     MarkLog log_{*dev_}, env_log_{*dev_};
     KernelStats heff_k_, env_k_;
-    double env_flop_ = 0;
+    double env_flop_ = 0, env_late_ = 0;
     bool verbose_ = false;
     int last_iters_ = 0;
     long long sa_added_ = 0;
