@@ -236,7 +236,8 @@ int kv_tdvp_get_site(kv_tdvp* s, int i, kv_tensor** out);
 int kv_tdvp_bond_dims(kv_tdvp* s, int* dims);
 /* Per-module timing in seconds, names of the reference's Timer modules
  * (holstein/tdvp.h:85-214): "Evl-2","Evl-1","Evl-0","SVD","Update","Sweep", plus
- * GPU time (the device clock at the start of successive launches) and algorithmic flops of the H_eff matvec
+ * GPU time (the device clock at the start of successive launches, so with the gaps between
+ * them) and algorithmic flops of the H_eff matvec
  * kernels and of the environment-update kernels.  Writes up to n values in this order:
  *   0 Evl-2  1 Evl-1  2 Evl-0  3 SVD  4 Update  5 Sweep  (wall seconds; an environment
  *      update is only queued where it is called: the device time that the next module then

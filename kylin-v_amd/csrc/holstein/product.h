@@ -171,14 +171,19 @@ struct DevProduct {
                         groups, segs, ar, ai, cfg, stop, mark);
         if (nch > 1) launch_sum_parts<T2>(dev.stream, part.as<T2>(), nch, p.out.total, C, stop);
     }
+    // Ends the log's open record: the launches that time the tiles are no part of it.
+    static void close(Device& dev, MarkLog* log) {
+        if (Mark* done = log ? log->end() : nullptr) launch_mark(dev.stream, done);
+    }
     // Tile config for this plan: cached per shape class; on a first encounter every config
     // built for the op pair runs twice on the real operands and the fastest is kept.
     template <class T2>
-    int choose(Device& dev, const T2* A, const T2* B, T2* C, double ar, double ai) {
+    int choose(Device& dev, const T2* A, const T2* B, T2* C, double ar, double ai, MarkLog* log) {
         if (!dev.autotune || p.flop < 1e8 || nch > 1) return 0;
         const uint64_t key = gemm_shape_key(p, sizeof(T2) == sizeof(double2) ? 0 : 1);
         auto it = dev.gemm_tuned.find(key);
         if (it != dev.gemm_tuned.end()) return it->second;
+        close(dev, log);
         EventTimer ev;
         int best = 0;
         float best_ms = 1e30f;
@@ -217,12 +222,13 @@ struct DevProduct {
     }
     // Split-BF16 tile (64x64 or 128x128): KV_SPLIT_TILE's, also for a plan cut into K chunks, else
     // timed once per shape class like choose().
-    int choose_split(Device& dev, const float2* A, const float2* B, float2* C, double ar, double ai) {
+    int choose_split(Device& dev, const float2* A, const float2* B, float2* C, double ar, double ai, MarkLog* log) {
         if (const char* t = std::getenv("KV_SPLIT_TILE")) return std::atoi(t) == 128 ? 4 : 0;
         if (!dev.autotune || p.flop < 1e8 || nch > 1) return 0;
         const uint64_t key = gemm_shape_key(p, 2);
         auto it = dev.gemm_tuned.find(key);
         if (it != dev.gemm_tuned.end()) return it->second;
+        close(dev, log);
         EventTimer ev;
         int best = 0;
         float best_ms = 1e30f;
@@ -245,10 +251,10 @@ struct DevProduct {
              double alpha_im = 0.0, MarkLog* log = nullptr, bool split = false, const int* stop = nullptr) {
         int cfg = 0;
         if constexpr (std::is_same<T2, float2>::value) {
-            cfg = split ? choose_split(dev, A, B, C, alpha_re, alpha_im)
-                        : choose<T2>(dev, A, B, C, alpha_re, alpha_im);
+            cfg = split ? choose_split(dev, A, B, C, alpha_re, alpha_im, log)
+                        : choose<T2>(dev, A, B, C, alpha_re, alpha_im, log);
         } else {
-            cfg = choose<T2>(dev, A, B, C, alpha_re, alpha_im);
+            cfg = choose<T2>(dev, A, B, C, alpha_re, alpha_im, log);
         }
         Mark* mark = nullptr;
         if (log && !p.tiles.empty())

@@ -57,3 +57,27 @@ def test_update_time_holds_the_environments_device_time(step):
     assert st["Update"] >= st["env_gpu_s"]
     assert all(st[m] >= 0 for m in MODULES)
     assert sum(st[m] for m in MODULES) <= wall
+
+def test_tile_tuning_is_not_booked_on_the_launch_before():
+    """A context's first step times the tiles of a product between two launches of a matvec; the
+    fold before it must not be charged for that."""
+    kv = GE.load_package()
+    print("case tuning", flush=True)
+
+    def fold_times():
+        ctx = kv.Context(0)  # the tuned tiles are the context's
+        # site 2's last product: 900 x 120, K = 120: tuned, and too shallow to be cut into K chunks
+        eng = kv.TDVP(*chain(kv, 30, (30, 120, 30), False, ctx), cutoff=1e-12, maxdim=120, dt=0.05, max_iter=2)
+        t = []
+        for _ in range(2):
+            eng.reset_stats()
+            eng.one_site()
+            t.append(eng.stats()["heff_wfold_gpu_s"])
+        del eng
+        ctx.close()
+        return t
+
+    fold_times()  # loads the kernels
+    pairs = [fold_times() for _ in range(3)]
+    first, second = (min(p[k] for p in pairs) for k in (0, 1))
+    assert 0 < first < 3 * second, pairs
