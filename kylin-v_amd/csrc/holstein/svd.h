@@ -265,19 +265,6 @@ inline void exact_sector(Device& D, Solver& sol, SectorSvd& X, bool keep_zero) {
     KV_REQUIRE(hinfo == 0, ERR_SOLVER, "Problems in SVD (did not converge)");
 }
 
-// Sectors the one-workgroup SVD takes.  Above kJacobiElems its reflectors would walk the long side
-// through one CU for longer than zgeqrf's launches take.  Under a truncating cutoff it starts at a
-// larger side of kJacobiLong: chains whose sectors are all smaller than that (the
-// projected-purification layout) truncate at values below what zgesvdj resolves, so what they
-// keep, and with it their results at the 1e-10 level, follows zgesvdj's rounding (an 8-site step:
-// energy 4e-10 where it is 0, and 2e-12 with this kernel, in 59 instead of 114 ms), and runs of
-// such chains go on as they began.
-constexpr int64_t kJacobiElems = (int64_t)1 << 18, kJacobiLong = 128;
-inline bool jacobi_takes(int64_t nr, int64_t nc, double cutoff) {
-    return std::min(nr, nc) <= kJacobiMax && nr * nc <= kJacobiElems &&
-           (cutoff < 0.0 || std::max(nr, nc) >= kJacobiLong);
-}
-
 // The exact route for sectors that jacobi_takes: all of them in one launch and one wait.  With
 // keep_zero a sector whose smallest values vanish next to its largest goes to zgesvd, whose
 // vectors for them are an orthonormal completion.
@@ -1458,6 +1445,12 @@ inline SvdResult svd_truncate(const std::shared_ptr<Device>& dev, Solver& sol, c
             exact_sector(D, sol, X[p], cutoff < 0.0);
     };
     auto small_sectors = [&] {  // those full_route has left to the batched exact route
+        auto slow = [&](const SectorSvd* x) { return jacobi_slower_alone(x->nr, x->nc, cutoff); };
+        if (std::count_if(small.begin(), small.end(), slow) == 1) {
+            const auto it = std::find_if(small.begin(), small.end(), slow);
+            exact_sector(D, sol, **it, cutoff < 0.0);
+            small.erase(it);
+        }
         jacobi_sectors(D, sol, small, cutoff < 0.0);
         small.clear();
     };

@@ -15,6 +15,7 @@
 #include <tuple>
 #include <vector>
 
+#include "../kv_types.h"
 #include "layout.h"
 
 namespace kv {
@@ -105,6 +106,34 @@ inline std::vector<int> truncation_counts(const std::vector<std::vector<double>>
             break;
     }
     return kept;
+}
+
+// Sectors the one-workgroup SVD takes (rocSOLVER's: zgesvdj under a truncating cutoff, else zgesvd).
+// Its reflectors walk the long side through one CU.  Under a truncating cutoff it takes all up to
+// kJacobiElems: ahead of zgesvdj (ms for one sector, 512 x 63 1.8 / 8.0, 65536 x 4 5.5 / 14.7, 262144 x 1
+// 6.6 / 29.3) but for a long wide sector by itself (63 x 4096 9.4 / 8.0), where zgesvdj's factors of values
+// over fourteen decades miss the sector by 2.5e-8 of its norm.  With every value kept, zgesvd's
+// time hardly grows with the long side of a wide sector or a single column: two sectors of
+// 8 x 16384 take 2.6 / 2.9, of 8 x 32768 5.2 / 3.7.  Under a truncating cutoff it starts at a
+// larger side of kJacobiLong: chains whose sectors are all smaller than that (the
+// projected-purification layout) truncate at values below what zgesvdj resolves, so what they
+// keep, and with it their results at the 1e-10 level, follows zgesvdj's rounding (an 8-site step:
+// energy 4e-10 where it is 0, and 2e-12 with this kernel, in 59 instead of 114 ms), and runs of
+// such chains go on as they began.
+constexpr int64_t kJacobiElems = (int64_t)1 << 18, kJacobiLong = 128, kJacobiWide = 16384;
+inline bool jacobi_takes(int64_t nr, int64_t nc, double cutoff) {
+    const int64_t lo = std::min(nr, nc), hi = std::max(nr, nc);
+    return lo <= kJacobiMax && lo * hi <= kJacobiElems &&
+           (cutoff < 0.0 ? hi <= kJacobiWide || (nr > nc && lo > 1) : hi >= kJacobiLong);
+}
+
+// Sectors of those that zgesvd solves faster than the one-workgroup SVD does where there is one of
+// them; two or more are faster together, since a launch takes as long as its longest.  One sector, ms
+// against zgesvd's: 1 x 6144 0.16 / 0.17, 1 x 8192 0.20 / 0.17, 24 x 6144 3.5 / 4.2, 24 x 8192 4.6 / 4.2,
+// 8192 x 1 0.20 / 0.19, 8192 x 24 4.7 / 6.1, 13000 x 4 1.1 / 2.0 (10000 x 4 0.86 / 0.73, before zgesvd changes its
+// method).
+inline bool jacobi_slower_alone(int64_t nr, int64_t nc, double cutoff) {
+    return cutoff < 0.0 && std::max(nr, nc) > 6144 && (nr < nc || nc == 1);
 }
 
 // Matrices of a batched eigensolve that have to be redone: those whose status is not 0 (`info`, empty

@@ -97,7 +97,6 @@ void launch_f32_to_f64(hipStream_t st, const float2* src, double2* dst, double s
 void launch_mark(hipStream_t st, Mark* mark);
 
 // ---- SVD of small sectors ----------------------------------------------------------------
-constexpr int kJacobiMax = 64;  // largest smaller side
 // M (nr x nc, row-major) = U S Vh: U nr x k, Vh k x nc (row-major), S descending, k = min(nr, nc).
 // Workspaces: A and T of nr x nc (T only where nr >= nc), W of k x k, tau of k.  S is NaN where M holds a NaN or an
 // infinity and -1 where the rotations did not converge.  Vectors of zero singular values are

@@ -96,6 +96,9 @@ KV_HD inline void wcompose_expand(const WComposeTask& c, int s1, const WComposeT
     tasks[c.task0 + s1] = t;
 }
 
+// ---- SVD of small sectors (launch_jacobi_svd) --------------------------------------------
+constexpr int kJacobiMax = 64;  // largest smaller side
+
 // ---- block permutation (tensor transpose) ----------------------------------------------
 constexpr int PERM_MAXR = 6;
 struct PermTask {
