@@ -305,6 +305,7 @@ inline void jacobi_sectors(Device& D, Solver& sol, const std::vector<SectorSvd*>
         j.S = S.as<double>() + soff[i];
         j.nr = (int)X.nr;
         j.nc = (int)X.nc;
+        j.zero_ends = keep_zero;
         jobs.push_back(j);
         nmax = std::max(nmax, k);
         mmax = std::max(mmax, (int)std::max(X.nr, X.nc));

@@ -100,12 +100,13 @@ void launch_mark(hipStream_t st, Mark* mark);
 // M (nr x nc, row-major) = U S Vh: U nr x k, Vh k x nc (row-major), S descending, k = min(nr, nc).
 // Workspaces: A and T of nr x nc (T only where nr >= nc), W of k x k, tau of k.  S is NaN where M holds a NaN or an
 // infinity and -1 where the rotations did not converge.  Vectors of zero singular values are
-// zero on the shorter side, except those of a zero matrix.
+// zero on the shorter side, except those of a zero matrix.  With zero_ends set, a matrix whose
+// reduction meets a zero pivot is not decomposed: its last S is 0, no more.
 struct SvdJob {
     const double2* M;
     double2 *U, *Vh, *A, *T, *W, *tau;
     double* S;
-    int nr, nc;
+    int nr, nc, zero_ends;
 };
 // nmax / mmax: the largest smaller / larger side of the jobs.
 void launch_jacobi_svd(hipStream_t st, const SvdJob* jobs, int njobs, int nmax, int mmax);

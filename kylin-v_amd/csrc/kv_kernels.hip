@@ -1660,6 +1660,15 @@ __global__ __launch_bounds__(THREADS) void jacobi_svd_kernel(const SvdJob* __res
     }
     amax = 0;
     for (int w = 0; w < NW; ++w) amax = fmax(amax, red[w]);
+    // a sector that goes to zgesvd all the same (two of 1024 x 40, all zero: 9.8 ms with the
+    // decomposition before it, 8.9 without)
+    auto zero_end = [&] {
+        if (tid < n) J.S[tid] = tid + 1 < n ? 1.0 : 0.0;
+    };
+    if (J.zero_ends && amax == 0) {  // uniform
+        zero_end();
+        return;
+    }
     int ex = 0;
     if (amax > 0) (void)frexp(amax, &ex);
     for (int e = tid; e < m * n; e += THREADS) {
@@ -1737,6 +1746,14 @@ __global__ __launch_bounds__(THREADS) void jacobi_svd_kernel(const SvdJob* __res
         __syncthreads();
     }
 
+    if (J.zero_ends) {
+        bool zero = false;
+        for (int i = 0; i < n; ++i) zero = zero || rdiag[i] == 0;
+        if (zero) {  // uniform
+            zero_end();
+            return;
+        }
+    }
     // X = R^H column by column, W = 1
     double2 *X = lds, *W = lds + n * n;
     for (int e = tid; e < n * n; e += THREADS) {
@@ -1865,7 +1882,7 @@ __global__ __launch_bounds__(64) void jacobi_apply_kernel(const SvdJob* __restri
     const SvdJob J = jobs[blockIdx.y];
     const bool tall = J.nr >= J.nc;
     const int n = tall ? J.nc : J.nr, m = tall ? J.nr : J.nc, k = blockIdx.x, lane = threadIdx.x;
-    if (k >= n) return;
+    if (k >= n || (J.zero_ends && J.S[n - 1] == 0)) return;
     const double2* w = J.W + k * n;
     const double2* A = J.A;
     ColView<NT> c((tall ? J.T : J.Vh) + (int64_t)k * m, m, lane);
