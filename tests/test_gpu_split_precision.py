@@ -69,5 +69,28 @@ def test_pinned_tile_runs_in_plans_cut_into_chunks(tile, monkeypatch):
     assert abs(got - want).max() <= 2e-4 * mag.real.max()
 
 
+# (Dl, levels, Dr, W's channels): K of the two products 127 (uncut), 128 and 129 (two chunks), 255 and
+# 256 (two and four), 1047 and 2094 (16 and 32 chunks, of which the last two are empty), many tiles
+CHUNKS = [(127, 1, 127, 1), (128, 1, 128, 1), (129, 3, 65, 2), (255, 2, 256, 1), (1047, 1, 3, 1), (5, 1, 1047, 2),
+          (600, 1, 520, 1)]
+
+
+@pytest.mark.parametrize("dl,p,dr,w", CHUNKS)
+@pytest.mark.parametrize("precision", ["fp32", "bf16x3"])
+def test_heff_at_the_chunk_limits(dl, p, dr, w, precision):
+    kv = GE.load_package()
+    print(f"case chunks {dl}x{p}x{dr} w {w} {precision}", flush=True)
+    (L, x, W, R), ref = both(kv, operands(dl, p, dr, w))
+    (got,) = kv.apply_single(L, x, W, R, precision).to_blocks()[1].values()
+    (want,) = T.apply_single(*ref).blocks.values()
+    (mag,) = T.apply_single(*(OT(t.dirs, {q: abs(b).astype(complex) for q, b in t.blocks.items()})
+                              for t in ref)).blocks.values()
+    # two products in FP32: a rounding per term and a few for the operands, the fold and the complex
+    # products' three real ones, in units of the products of absolute values; split BF16 also drops
+    # 3 * 2^-18 of each of a complex product's four real ones, in either product
+    tol = 4 * (dl + w * dr + 16) * 2.0 ** -24 + (24 * 2.0 ** -18 if precision == "bf16x3" else 0)
+    assert np.all(abs(got - want) <= tol * mag.real)
+
+
 if __name__ == "__main__":
     launched()
