@@ -184,7 +184,9 @@ int kv_krylov_step(kv_ctx* ctx, int nsite, const kv_tensor* L, const kv_tensor* 
  * divide and conquer (rocSOLVER's dstedc above side 512) and the kept vectors carried back
  * through the reflectors; below that rocSOLVER's zheevd; a second pass over the tail below
  * 1e-5 of the largest value); smaller ones by a one-workgroup Jacobi SVD where cutoff < 0 or
- * the longer side is at least 128, else by rocSOLVER's.  KV_SVD=full in the environment turns the block route off. */
+ * the longer side is at least 128, else by rocSOLVER's, which also takes the largest sectors
+ * of few rows and, with cutoff < 0, those with singular values of 0.  KV_SVD=full in the
+ * environment turns the block route off. */
 int kv_svd_truncate(kv_ctx* ctx, const kv_tensor* A, int r1, double cutoff, int maxdim,
                     int left_to_right, kv_tensor** left, kv_tensor** right, int* nkept);
 

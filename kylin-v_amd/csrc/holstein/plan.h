@@ -212,6 +212,9 @@ struct SplitK {
 // workgroup walks its whole K range alone, 1.1 us per 8-deep stage (an environment update's
 // last product at D = 128, 16 levels: 6 tiles, K = 2048, 286 us whole, 17 + 4 us cut in 32).  Chunks
 // double while the workgroups stay under kSplitWgs and the deepest group keeps kSplitDepth per chunk.
+// Plans that are cut keep the 64x64 tile; the largest of them gain least over their tuned tile uncut (one-site
+// H_eff, us: 4 channels, D = 704, 121 tiles 689 -> 413, D = 1024, 256 tiles 1257 -> 1133, split BF16 396 -> 308; two
+// channels, D = 768, two levels 756 -> 735).
 constexpr int kSplitWgs = 512, kSplitDepth = 64, kSplitMax = 32;
 inline int split_chunks(const ProductPlan& P) {
     int64_t kmax = 0;
@@ -521,7 +524,8 @@ inline ComposePlan plan_compose(const WFoldPlan& F1, const WFoldPlan& F2, const 
     return C;
 }
 
-// The composite's lists, expanded on the host.
+// The composite's lists, expanded on the host: for plans checked without a GPU (the engine expands them on
+// the device).
 inline WFoldPlan compose_wfold(const WFoldPlan& F1, const WFoldPlan& F2, const Layout& Y) {
     const ComposePlan C = plan_compose(F1, F2, Y);
     WFoldPlan W;

@@ -103,10 +103,12 @@ struct SvdResult {
     std::string detail;  // per sector: rows x cols, route, s_max, last kept value
 };
 
-// Side from which the split eigensolver replaces zheevd by default.  With the reflectors
-// applied in one launch it is the faster one from 128 up, alone and with eight contexts at once
-// (a bond of two n x 2n sectors, ms, against zheevd: n = 80 1.82 / 1.85, 128 2.82 / 3.39,
-// 256 6.3 / 8.0, 500 11.9 / 14.7; eight at once, n = 128 10.1 / 10.8, 256 13.9 / 18.4).
+// Side from which the split eigensolver replaces zheevd by default (equal sides; sectors of
+// different sides always take it).  It is the faster one at every side (a bond of two n x 2n
+// sectors, ms, against zheevd: n = 64 0.71 / 2.6, 96 0.96 / 2.3, 112 1.06 / 2.8, 128 1.11 / 3.5, 256
+// 3.7 / 8.3, 448 7.9 / 13.8; eight contexts at once, n = 64 3.3 / 10.7, 96 3.4 / 4.6, 128 3.2 / 7.0, 256 7.5 / 17.8).
+// 128 and not 64 holds one truncation: the 32-site chain from its physical start has a value of bond 0 at
+// the cutoff in step 13, which LAPACK and zheevd keep and the split solver's rounding drops.
 constexpr int kSplitEigMin = 128;
 // The side from which the split route is taken (KV_SPLIT_MIN overrides kSplitEigMin).
 inline int split_eig_min() {
@@ -481,8 +483,8 @@ inline void hetrd_lower(Device& D, Solver& sol, double2* A, int N, int batch, do
 // diag(G, -I) (G is positive semidefinite, so the padding stays exactly decoupled and each
 // sector's reflectors and tridiagonal are those of G); then the tridiagonals' divide and conquer,
 // all sectors together up to kStedcMax (launch_stedc) and dstedc per sector above, and the
-// vectors formed later, only for the rows the truncation needs (gram_eigvecs).  zheevd (all vectors at once, batched) for equal sides below
-// kSplitEigMin.  (zheevd cannot take the padded matrices: on the split tridiagonal its
+// vectors formed later, only for the rows the truncation needs (gram_eigvecs).  zheevd (all
+// vectors at once, batched) for equal sides below kSplitEigMin.  (zheevd cannot take the padded matrices: on the split tridiagonal its
 // divide and conquer returns NaN eigenvectors.  dstedc of a pair on two streams measured
 // slower in the sweep than one after the other.)
 inline void gram_solve(Device& D, Solver& sol, std::vector<SectorSvd*> xs, int mode = EIG_AUTO,

@@ -117,6 +117,8 @@ void launch_set_diag(hipStream_t st, double2* A, int64_t ld, int from, int to, d
 void launch_tri_copy(hipStream_t st, const double2* src, int64_t lds, double2* dst, int n, bool lower);
 
 // ---- symmetric tridiagonal eigenproblem ------------------------------------------------------
+// The largest side: a merge keeps its values in LDS, one thread each.  Against dstedc beyond 256, a bond of two
+// n x 2n sectors takes, ms, n = 257 4.5 / 6.2, 384 6.8 / 9.0, 512 9.1 / 12.4; eight contexts at once, 512 22.8 / 29.9.
 constexpr int kStedcMax = 512;
 // diag d (n), subdiagonal e (n - 1): eigenvalues ascending into w, vectors into Z (n x n, column-major).
 // Workspaces: Q1, Q2, U of n x n, d1, d2 of n, scale of one; src, pos of n ints, kcount of
@@ -131,7 +133,9 @@ void launch_stedc(hipStream_t st, const StedcJob* jobs, int njobs, int nmax);
 
 // Back-transformation of a lower-triangle Householder tridiagonalisation (LAPACK layout:
 // reflector i stored below the subdiagonal of column i, tau_i separately).
-// Sides up to kHhApplyMax in one launch: Z = Q C(:, c0 : c0 + k), C real (ld n), Z complex (ld n).
+// Sides up to kHhApplyMax in one launch: Z = Q C(:, c0 : c0 + k), C real (ld n), Z complex (ld n).  Beyond
+// 256 it is even with the blocked form alone (a bond of two n x 2n sectors, ms, n = 257 4.5 / 4.7, 320 5.5 / 5.5,
+// 512 9.1 / 8.7), and with eight contexts at once its fewer launches count (400 16.8 / 22.6, 512 22.8 / 21.8).
 constexpr int kHhApplyMax = 512;
 void launch_hh_apply(hipStream_t st, const double2* A, const double2* tau, const double* C, int n, int c0, int k,
                      double2* Z);

@@ -1,6 +1,6 @@
 """Kernel-level H_eff measurement: one two-site effective Hamiltonian of a merged-layout
 Holstein chain at bond dimension D, applied `reps` times per precision (fp64, fp32,
-bf16x3 = split-BF16 products with FP32 accumulation), HIP-event timed, with the error of
+bf16x3 = split-BF16 products with FP32 accumulation), timed on the device, with the error of
 each precision against the FP64 result.
 
 The default is the scale + split-precision shape: each site an exciton times two phonon
